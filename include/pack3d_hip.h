@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define P3D_ABI_VERSION 19
+#define P3D_ABI_VERSION 20
 
 enum p3d_status { P3D_OK = 0, P3D_EINVAL = 1, P3D_EHIP = 2, P3D_EUNSUPPORTED = 3 };
 enum p3d_dtype { P3D_F32 = 0, P3D_F16 = 1, P3D_BF16 = 2 };
@@ -86,10 +86,36 @@ int p3d_geometry_check(const void* neighbors, int32_t nb_is64, int64_t n, int32_
 int p3d_reverse_adjacency(const int32_t* neighbors, int64_t n, int32_t width, int32_t* cursor,
                           int32_t* reverse, int32_t rwidth, void* stream);
 
+/* The same checks as p3d_geometry_check with the edges grouped by destination
+ * on the way, for p3d_reverse_bucketed: no per-row in-degree array and no global
+ * atomic per edge.  work: p3d_bucket_bytes(n, width) bytes of scratch (0 where
+ * this path does not take the table: more than 2^20 rows), kept by the caller
+ * until p3d_reverse_bucketed has run.  flags as p3d_geometry_check. */
+int64_t p3d_bucket_bytes(int64_t n, int32_t width);
+int p3d_geometry_check_bucketed(const void* neighbors, int32_t nb_is64, int64_t n, int32_t width,
+                                const void* blocks, int32_t blocks_is64, int64_t fine, int32_t slots,
+                                int32_t pool_size, int32_t* neighbors32, int32_t* blocks32, int32_t* cover,
+                                void* work, int32_t* flags, void* stream);
+
+/* reverse[j] = ascending sources whose row contains j, -1 padded to rwidth (at
+ * least the largest in-degree, flags[5]), from the edges that
+ * p3d_geometry_check_bucketed left in work. */
+int p3d_reverse_bucketed(void* work, int64_t n, int32_t width, int32_t* reverse, int32_t rwidth, void* stream);
+
+/* reverse[i] = the valid entries of rows[perm[i]] (perm NULL: row i), relabelled
+ * by inverse where it is given, ascending, -1 padded to rwidth: the reverse
+ * adjacency of a symmetric graph from its neighbour table, or of a relabelled
+ * graph from its reverse table.  width and rwidth are at most 128; valid
+ * entries past rwidth are dropped.  reverse may be rows itself when perm is
+ * NULL and width == rwidth. */
+int p3d_reverse_rows(const int32_t* rows, int64_t n, int32_t width, const int64_t* perm, const int64_t* inverse,
+                     int32_t* reverse, int32_t rwidth, void* stream);
+
 /* TokenLayout.repack (geometry.py:189-220): new row i = old row perm[i].
  * inverse[n] (int64 scratch) receives perm^-1.  flags[0] counts entries of perm
- * that are out of range or repeated (cleared by the call).  raster_map may be
- * NULL (identity); raster_map_out may be NULL (no grid tag). */
+ * that are out of range or repeated (cleared by the call); flags[1] is nonzero
+ * when raster_map_out is not the identity.  raster_map may be NULL (identity);
+ * raster_map_out may be NULL (no grid tag). */
 int p3d_repack(const int64_t* perm, int64_t n, const int32_t* neighbors, int32_t width,
                const int32_t* blocks, int64_t fine, int32_t slots, const int64_t* order,
                const int64_t* coords, const int32_t* raster_map, int64_t* inverse,

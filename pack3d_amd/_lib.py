@@ -25,7 +25,7 @@ class View(ctypes.Structure):
     _fields_ = [("data", c_void_p), ("sb", c_int64), ("sh", c_int64), ("sn", c_int64)]
 
 
-ABI_VERSION = 19  # P3D_ABI_VERSION in include/pack3d_hip.h
+ABI_VERSION = 20  # P3D_ABI_VERSION in include/pack3d_hip.h
 
 
 class Rope(ctypes.Structure):
@@ -85,6 +85,11 @@ SIGNATURES = {
     "p3d_geometry_check": ([_P, c_int32, c_int64, c_int32, _P, c_int32, c_int64, c_int32, c_int32,
                             _P, _P, _P, _P, _P, _P], c_int32),
     "p3d_reverse_adjacency": ([_P, c_int64, c_int32, _P, _P, c_int32, _P], c_int32),
+    "p3d_bucket_bytes": ([c_int64, c_int32], c_int64),
+    "p3d_geometry_check_bucketed": ([_P, c_int32, c_int64, c_int32, _P, c_int32, c_int64, c_int32, c_int32,
+                                     _P, _P, _P, _P, _P, _P], c_int32),
+    "p3d_reverse_bucketed": ([_P, c_int64, c_int32, _P, c_int32, _P], c_int32),
+    "p3d_reverse_rows": ([_P, c_int64, c_int32, _P, _P, _P, c_int32, _P], c_int32),
     "p3d_repack": ([_P, c_int64, _P, c_int32, _P, c_int64, c_int32, _P, _P, _P, _P, _P, _P, _P, _P, _P,
                     _P, _P], c_int32),
     "p3d_check_layout": ([_P, _P, _P, _P, _P, _P], c_int32),

@@ -4,11 +4,12 @@ Mirrors ``src/pack3d/geometry.py`` of amilworks/Pack3D -- same classes,
 arguments, error classes and messages -- but constructs the tables with the
 integer HIP kernels of ``libpack3d_hip.so``:
 
-* ``build_layout``      -> ``p3d_build_layout`` + ``p3d_reverse_adjacency``
+* ``build_layout``      -> ``p3d_build_layout`` + ``p3d_reverse_rows``
   (geometry.py:223-266)
-* ``prepare_geometry``  -> ``p3d_geometry_check`` + ``p3d_reverse_adjacency``
-  (geometry.py:53-101)
-* ``TokenLayout.repack`` -> ``p3d_repack`` + ``p3d_reverse_adjacency``
+* ``prepare_geometry``  -> ``p3d_geometry_check_bucketed`` +
+  ``p3d_reverse_bucketed``, or ``p3d_geometry_check`` +
+  ``p3d_reverse_adjacency`` past 2^20 rows (geometry.py:53-101)
+* ``TokenLayout.repack`` -> ``p3d_repack`` + ``p3d_reverse_rows``
   (geometry.py:189-220)
 
 All tables are bit-exact with the reference construction.  Geometry lives
@@ -112,6 +113,18 @@ def _reverse(nb32: Tensor, rwidth: int) -> Tensor:
 
 
 @torch.inference_mode(False)
+def _reverse_rows(rows: Tensor, rwidth: int, perm=None, inverse=None) -> Tensor:
+    """The reverse adjacency from a table that lists, per row, the rows that
+    reach it: the neighbour table of a symmetric graph, or (with a permutation
+    and its inverse) the reverse table of the graph before it is relabelled."""
+    n, width = rows.shape
+    reverse = torch.empty(n, rwidth, dtype=torch.int32, device=rows.device)
+    _lib.call("p3d_reverse_rows", rows.data_ptr(), n, width, _lib.ptr(perm), _lib.ptr(inverse), reverse.data_ptr(),
+              rwidth, _lib.stream_of(rows.device))
+    return reverse
+
+
+@torch.inference_mode(False)
 def prepare_geometry(neighbors: Tensor, blocks: Tensor, pool_size: int) -> Pack3DGeometry:
     """Validate a local graph and fine-block partition on the GPU (geometry.py:53-101).
 
@@ -137,13 +150,20 @@ def prepare_geometry(neighbors: Tensor, blocks: Tensor, pool_size: int) -> Pack3
     bl_in = blocks.detach().to(device).contiguous()
     nb32 = torch.empty(n, width, dtype=torch.int32, device=device)
     bl32 = torch.empty(fine, slots, dtype=torch.int32, device=device)
-    degree = torch.empty(n, dtype=torch.int32, device=device)
     cover = torch.empty(n, dtype=torch.int32, device=device)
     flags = torch.empty(8, dtype=torch.int32, device=device)
-    _lib.call("p3d_geometry_check", nb_in.data_ptr(), int(nb_in.dtype == torch.int64), n, width,
-              bl_in.data_ptr(), int(bl_in.dtype == torch.int64), fine, slots, pool_size,
-              nb32.data_ptr(), bl32.data_ptr(), degree.data_ptr(), cover.data_ptr(), flags.data_ptr(),
-              _lib.stream_of(device))
+    # Edges grouped by destination in scratch memory, or (past 2^20 rows) one
+    # atomic per edge on an in-degree array.
+    work_bytes = _lib.lib().p3d_bucket_bytes(n, width)
+    tables = (nb_in.data_ptr(), int(nb_in.dtype == torch.int64), n, width, bl_in.data_ptr(),
+              int(bl_in.dtype == torch.int64), fine, slots, pool_size, nb32.data_ptr(), bl32.data_ptr())
+    stream = _lib.stream_of(device)
+    if work_bytes:
+        work = torch.empty(work_bytes, dtype=torch.uint8, device=device)
+        _lib.call("p3d_geometry_check_bucketed", *tables, cover.data_ptr(), work.data_ptr(), flags.data_ptr(), stream)
+    else:
+        degree = torch.empty(n, dtype=torch.int32, device=device)
+        _lib.call("p3d_geometry_check", *tables, degree.data_ptr(), cover.data_ptr(), flags.data_ptr(), stream)
     f = _flags(flags)
     if f[0]:
         raise ValueError("neighbors contains an out-of-range token")
@@ -158,7 +178,13 @@ def prepare_geometry(neighbors: Tensor, blocks: Tensor, pool_size: int) -> Pack3
     rwidth = max(1, f[5])
     if rwidth > 128:
         raise ValueError("reverse local degree exceeds 128")
-    return Pack3DGeometry(nb32, _reverse(nb32, rwidth), bl32, pool_size, n, _SEAL)
+    if work_bytes:
+        reverse = torch.empty(n, rwidth, dtype=torch.int32, device=device)
+        _lib.call("p3d_reverse_bucketed", work.data_ptr(), n, width, reverse.data_ptr(), rwidth,
+                  _lib.stream_of(device))
+    else:
+        reverse = _reverse(nb32, rwidth)
+    return Pack3DGeometry(nb32, reverse, bl32, pool_size, n, _SEAL)
 
 
 def _triple(value, name, *, allow_zero=False):
@@ -283,13 +309,17 @@ class TokenLayout:
                   _lib.ptr(geom._raster_to_packed) if tagged else None, inverse.data_ptr(), nb.data_ptr(),
                   blocks.data_ptr(), order.data_ptr(), coords.data_ptr(), _lib.ptr(mapping), flags.data_ptr(),
                   _lib.stream_of(device))
-        if _flags(flags)[0]:
+        f = _flags(flags)
+        if f[0]:
             raise ValueError("permutation must contain every token exactly once")
         # Relabelling preserves every in-degree, so the reverse width is unchanged.
-        new = Pack3DGeometry(nb, _reverse(nb, geom.reverse_neighbors.shape[1]), blocks, geom.pool_size, n, _SEAL)
+        # A complete stencil is symmetric: its rows are their own sources.
+        rwidth = geom.reverse_neighbors.shape[1]
+        reverse = (_reverse_rows(nb, rwidth) if tagged
+                   else _reverse_rows(geom.reverse_neighbors, rwidth, p, inverse))
+        new = Pack3DGeometry(nb, reverse, blocks, geom.pool_size, n, _SEAL)
         if tagged:
-            identity = torch.equal(mapping, torch.arange(n, dtype=torch.int32, device=device))
-            new = replace(new, _seal=_SEAL, _grid=geom._grid, _raster_to_packed=None if identity else mapping)
+            new = replace(new, _seal=_SEAL, _grid=geom._grid, _raster_to_packed=mapping if f[1] else None)
         return TokenLayout(self.grid_shape, order, coords, new, _SEAL)
 
 
@@ -340,7 +370,8 @@ def build_layout(grid_shape, block_shape=(2, 2, 2), *, radius=1, pool_size=4,
               order.data_ptr(), coords.data_ptr(), _lib.ptr(mapping), nb.data_ptr(), blocks.data_ptr(),
               _lib.stream_of(dev))
     rwidth = max(1, _stencil_degree(shape, rad))
-    geom = Pack3DGeometry(nb, _reverse(nb, rwidth), blocks, pool_size, n, _SEAL,
+    # A complete stencil is symmetric: the rows that reach a token are its neighbours.
+    geom = Pack3DGeometry(nb, _reverse_rows(nb, rwidth), blocks, pool_size, n, _SEAL,
                           _grid=(shape, rad), _raster_to_packed=mapping)
     return TokenLayout(shape, order, coords, geom, _SEAL)
 

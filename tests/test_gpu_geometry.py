@@ -117,3 +117,66 @@ def test_layout_validation_and_mutation(gpu):
     lay.coords[0, 0] += 1
     with pytest.raises(RuntimeError, match="changed"):
         lay.pack(grid)
+
+
+def _random_graph(n, width, fill, gen):
+    """An asymmetric graph without duplicate edges: row i holds i and
+    pseudo-random distinct rows, `fill` of the entries present; in-degrees stay
+    below 128 (each column is a permutation of the rows)."""
+    columns = [(torch.arange(n) + int(s)) % n for s in torch.randperm(n, generator=gen)[:width]]
+    nb = torch.stack(columns, 1)
+    nb = torch.gather(nb, 1, torch.rand(n, width, generator=gen).argsort(1))
+    return torch.where(torch.rand(n, width, generator=gen) < fill, nb, -1)
+
+
+@pytest.mark.parametrize("n,width", [(127, 1), (128, 31), (129, 32), (200, 33), (257, 64), (300, 65), (1000, 127),
+                                     (4099, 128), (2 ** 20 + 1, 2)])
+def test_prepare_geometry_row_widths(gpu, n, width):
+    """Bucket edges (128 rows), the 32 / 64 / 128 column sorts, and the table
+    past 2^20 rows that takes the other route: integer work, bit-exact."""
+    print(f"prepare_geometry rows {n} width {width}", flush=True)
+    gen = torch.Generator().manual_seed(n)
+    nb = _random_graph(n, width, 0.8, gen)
+    blocks = torch.randperm(n, generator=gen)[:, None]
+    for dtype in (torch.int32, torch.int64):
+        got = p3d.prepare_geometry(nb.to(gpu, dtype), blocks.to(gpu, dtype), 1).to("cpu")
+        exp = ref.prepare_geometry(nb, blocks, 1)
+        for a, b in zip(got.tensors, exp.tensors):
+            assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("n", [40, 300])
+def test_prepare_geometry_in_degree_limit(gpu, n):
+    """Rows reached by every other row: in-degree n, past 128 an error, and a
+    duplicate edge into such a row is still reported first."""
+    print(f"in-degree {n}", flush=True)
+    nb = torch.stack((torch.zeros(n, dtype=torch.int64), torch.full((n,), -1)), 1)
+    blocks = torch.arange(n)[:, None]
+    if n <= 128:
+        got = p3d.prepare_geometry(nb, blocks, 1).to("cpu")
+        assert torch.equal(got.reverse_neighbors, ref.prepare_geometry(nb, blocks, 1).reverse_neighbors)
+    else:
+        with pytest.raises(ValueError, match="reverse local degree exceeds 128"):
+            p3d.prepare_geometry(nb, blocks, 1)
+    nb[n // 2, 1] = 0
+    with pytest.raises(ValueError, match="duplicate local edges"):
+        p3d.prepare_geometry(nb, blocks, 1)
+
+
+@pytest.mark.parametrize("tagged", [True, False])
+@pytest.mark.parametrize("shape,radius", [((3, 5, 70), (0, 0, 63)), ((4, 6, 10), (1, 1, 1)), ((5, 6, 8), (2, 1, 1)),
+                                          ((6, 7, 9), (2, 2, 2))])
+def test_repack_row_widths(gpu, shape, radius, tagged):
+    """Repack at 27, 45, 125 and 127 columns (the widest rows are clipped by the
+    grid), from a stencil and from the same tables without the grid tag, in both
+    directions."""
+    print(f"repack {shape} {radius} tagged={tagged}", flush=True)
+    kw = dict(radius=radius, pool_size=1, layout="raster_block")
+    lay, exp = (m.build_layout(shape, (1, 1, 1), **kw) for m in (p3d, ref))
+    if not tagged:
+        lay = p3d.TokenLayout(shape, lay.order, lay.coords, p3d.prepare_geometry(*lay.geometry.tensors[::2], 1))
+    for step in range(2):
+        p = torch.randperm(math.prod(shape), generator=torch.Generator().manual_seed(step))
+        lay, exp = lay.repack(p), exp.repack(p)
+        for a, b in zip(lay.to("cpu").geometry.tensors, exp.geometry.tensors):
+            assert torch.equal(a, b)
