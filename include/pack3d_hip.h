@@ -88,10 +88,10 @@ int p3d_reverse_adjacency(const int32_t* neighbors, int64_t n, int32_t width, in
 
 /* The same checks as p3d_geometry_check with the edges grouped by destination
  * on the way, for p3d_reverse_bucketed: no per-row in-degree array and no global
- * atomic per edge.  work: p3d_bucket_bytes(n, width) bytes of scratch (0 where
- * this path does not take the table: more than 2^20 rows), kept by the caller
- * until p3d_reverse_bucketed has run.  flags as p3d_geometry_check. */
-int64_t p3d_bucket_bytes(int64_t n, int32_t width);
+ * atomic per edge.  work: scratch of the size that p3d_bucket_bytes gives
+ * (0 where this path does not take the table: more than 2^20 rows), kept by the
+ * caller until p3d_reverse_bucketed has run.  flags as p3d_geometry_check. */
+int p3d_bucket_bytes(int64_t n, int32_t width, int64_t* bytes);
 int p3d_geometry_check_bucketed(const void* neighbors, int32_t nb_is64, int64_t n, int32_t width,
                                 const void* blocks, int32_t blocks_is64, int64_t fine, int32_t slots,
                                 int32_t pool_size, int32_t* neighbors32, int32_t* blocks32, int32_t* cover,

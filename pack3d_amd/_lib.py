@@ -85,7 +85,7 @@ SIGNATURES = {
     "p3d_geometry_check": ([_P, c_int32, c_int64, c_int32, _P, c_int32, c_int64, c_int32, c_int32,
                             _P, _P, _P, _P, _P, _P], c_int32),
     "p3d_reverse_adjacency": ([_P, c_int64, c_int32, _P, _P, c_int32, _P], c_int32),
-    "p3d_bucket_bytes": ([c_int64, c_int32], c_int64),
+    "p3d_bucket_bytes": ([c_int64, c_int32, ctypes.POINTER(c_int64)], c_int32),
     "p3d_geometry_check_bucketed": ([_P, c_int32, c_int64, c_int32, _P, c_int32, c_int64, c_int32, c_int32,
                                      _P, _P, _P, _P, _P, _P], c_int32),
     "p3d_reverse_bucketed": ([_P, c_int64, c_int32, _P, c_int32, _P], c_int32),

@@ -406,6 +406,11 @@ struct Buckets {
 
 inline int64_t bucket_count(int64_t n) { return cdiv(n, kBucketRows); }
 
+int64_t bucket_bytes(int64_t n, int32_t width) {
+    if (n < 1 || width < 1 || width > 128 || n * width >= ((int64_t)1 << 31) || bucket_count(n) > kMaxBuckets) return 0;
+    return (3 * bucket_count(n) + 1 + n * width) * (int64_t)sizeof(int32_t);
+}
+
 Buckets buckets_in(void* work, int64_t n) {
     Buckets b;
     b.n_buckets = (int32_t)bucket_count(n);
@@ -769,16 +774,17 @@ extern "C" int p3d_geometry_check(const void* neighbors, int32_t nb_is64, int64_
     return check_launch("p3d_geometry_check");
 }
 
-extern "C" int64_t p3d_bucket_bytes(int64_t n, int32_t width) {
-    if (n < 1 || width < 1 || width > 128 || n * width >= ((int64_t)1 << 31) || bucket_count(n) > kMaxBuckets) return 0;
-    return (3 * bucket_count(n) + 1 + n * width) * (int64_t)sizeof(int32_t);
+extern "C" int p3d_bucket_bytes(int64_t n, int32_t width, int64_t* bytes) {
+    P3D_REQUIRE(bytes, "null output");
+    *bytes = bucket_bytes(n, width);
+    return P3D_OK;
 }
 
 extern "C" int p3d_geometry_check_bucketed(const void* neighbors, int32_t nb_is64, int64_t n, int32_t width,
                                            const void* blocks, int32_t blocks_is64, int64_t fine, int32_t slots,
                                            int32_t pool_size, int32_t* neighbors32, int32_t* blocks32,
                                            int32_t* cover, void* work, int32_t* flags, void* stream) {
-    P3D_REQUIRE(p3d_bucket_bytes(n, width) > 0 && fine >= 1 && slots >= 1 && slots <= 64, "invalid geometry shape");
+    P3D_REQUIRE(bucket_bytes(n, width) > 0 && fine >= 1 && slots >= 1 && slots <= 64, "invalid geometry shape");
     P3D_REQUIRE(pool_size >= 1 && pool_size <= 32, "pool_size must be an integer in [1,32]");
     P3D_REQUIRE(neighbors && blocks && neighbors32 && blocks32 && cover && work && flags, "null argument");
     hipStream_t s = as_stream(stream);
@@ -806,7 +812,7 @@ extern "C" int p3d_geometry_check_bucketed(const void* neighbors, int32_t nb_is6
 
 extern "C" int p3d_reverse_bucketed(void* work, int64_t n, int32_t width, int32_t* reverse, int32_t rwidth,
                                     void* stream) {
-    P3D_REQUIRE(p3d_bucket_bytes(n, width) > 0 && rwidth >= 1 && rwidth <= 128, "invalid reverse adjacency shape");
+    P3D_REQUIRE(bucket_bytes(n, width) > 0 && rwidth >= 1 && rwidth <= 128, "invalid reverse adjacency shape");
     P3D_REQUIRE(work && reverse, "null argument");
     const Buckets b = buckets_in(work, n);
     const size_t lds = (size_t)kBucketRows * (rwidth + 1) * sizeof(int32_t);

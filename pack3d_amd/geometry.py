@@ -17,6 +17,7 @@ on a HIP device; ``.to("cpu")`` copies it out for inspection.
 """
 from __future__ import annotations
 
+import ctypes
 import itertools
 import math
 import weakref
@@ -154,7 +155,9 @@ def prepare_geometry(neighbors: Tensor, blocks: Tensor, pool_size: int) -> Pack3
     flags = torch.empty(8, dtype=torch.int32, device=device)
     # Edges grouped by destination in scratch memory, or (past 2^20 rows) one
     # atomic per edge on an in-degree array.
-    work_bytes = _lib.lib().p3d_bucket_bytes(n, width)
+    work_bytes = ctypes.c_int64()
+    _lib.call("p3d_bucket_bytes", n, width, ctypes.byref(work_bytes))
+    work_bytes = work_bytes.value
     tables = (nb_in.data_ptr(), int(nb_in.dtype == torch.int64), n, width, bl_in.data_ptr(),
               int(bl_in.dtype == torch.int64), fine, slots, pool_size, nb32.data_ptr(), bl32.data_ptr())
     stream = _lib.stream_of(device)
