@@ -501,11 +501,12 @@ int p3d_transpose_rows(p3d_view src, void* dst, int32_t batch, int32_t heads, in
  * rows; e.g. the q and kl column ranges of the projections' gradients). */
 int p3d_finish_bwd(const p3d_bwd_args* args, const p3d_rope* rope, p3d_view dq, p3d_view dkl, void* stream);
 
-/* Pooling backward (kernels.py:240-270): from the split partials of dsk / dsv,
+/* Pooling backward (kernels.py:240-270): from the split partials of dsk / dsv
+ * (scratch: with more than 16 splits they are summed into the first, in place),
  * writes dkg (gradient of the UNROTATED kg: R^T applied) and dvg into
  * [B,G,N,D] views of dtype (16-byte aligned rows), and per-summary partials
  * dw_part [B*G*Mp, D] and db_part [B*G*Mp, slots]. */
-int p3d_pool_bwd(const p3d_pool_args* pool, const float* dsk_part, const float* dsv_part, int32_t splits,
+int p3d_pool_bwd(const p3d_pool_args* pool, float* dsk_part, float* dsv_part, int32_t splits,
                  p3d_view dkg, p3d_view dvg, float* dw_part, float* db_part, void* stream);
 
 /* ---- self-tests (no counterpart in the reference) ---------------------- */

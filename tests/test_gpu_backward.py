@@ -381,3 +381,22 @@ def test_full_size_allen15_layer_gradients_match_oracle(gpu):
         err = rel_l2(got.float().cpu(), exp)
         print(f"  {name}: rel_l2={err:.3g}", flush=True)
         assert err < TOL[torch.bfloat16], (name, err)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("n,d,heads,kv_heads", [(1087, 64, 4, 1), (1088, 16, 4, 1), (1152, 128, 8, 2)])
+def test_every_gradient_many_splits(gpu, dtype, n, d, heads, kv_heads):
+    """Few summaries and many query splits of the summary dK/dV pass (17 and
+    18, so that the partials are summed before the pooling backward; the last
+    split ragged or empty), transposed stages by DMA (n a multiple of 8) and
+    by registers."""
+    from pack3d_amd.core import _splits
+    print(f"backward splits n{n} d{d} {dtype}", flush=True)
+    inputs, nb, blocks, pool = make_case(n, d, 1, heads, kv_heads, 16, 16, dtype=dtype)
+    og, hg = ref.prepare_geometry(nb, blocks, pool), p3d.prepare_geometry(nb.to(gpu), blocks.to(gpu), pool)
+    assert _splits(n, og.num_summaries, kv_heads, heads // kv_heads, d) > 16
+    xs = [t.to(gpu).requires_grad_() for t in inputs]
+    rs = [t.detach().clone().requires_grad_() for t in inputs]
+    y, e = p3d.pack3d_hip(*xs, hg), ref.pack3d_reference(*rs, og)
+    up = torch.randn(e.shape, generator=torch.Generator().manual_seed(7)).to(dtype)
+    _compare(torch.autograd.grad(y, xs, up.to(gpu)), torch.autograd.grad(e, rs, up), dtype, f"splits {n} {d}")
