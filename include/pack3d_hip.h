@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define P3D_ABI_VERSION 20
+#define P3D_ABI_VERSION 21
 
 enum p3d_status { P3D_OK = 0, P3D_EINVAL = 1, P3D_EHIP = 2, P3D_EUNSUPPORTED = 3 };
 enum p3d_dtype { P3D_F32 = 0, P3D_F16 = 1, P3D_BF16 = 2 };
@@ -402,13 +402,14 @@ int p3d_weight_grad(const void* dy, int64_t ldy, const void* x, int64_t ldx, flo
 
 /* p3d_weight_grad of three linear maps that share their input x (the
  * layer's to_q, to_kv and gate, attention.py:64-67,85) in one pass over x:
- * dw [out0 + out1 + out2, in_features] fp32 holds dW of dy0, then of dy1,
- * then of dy2, each dy with its own row stride.  Same rules as
+ * dw [out0 + out1 + out2, in_features] holds dW of dy0, then of dy1, then of
+ * dy2, each dy with its own row stride; summed in fp32, dw_dtype is fp32 or
+ * the inputs' type (rounded once).  Same rules as
  * p3d_weight_grad; the out counts positive multiples of 8. */
 int p3d_weight_grad3(const void* dy0, int64_t ld0, int32_t out0, const void* dy1, int64_t ld1, int32_t out1,
-                     const void* dy2, int64_t ld2, int32_t out2, const void* x, int64_t ldx, float* dw,
-                     float* workspace, int64_t rows, int32_t in_features, int32_t splits, int32_t dtype,
-                     void* stream);
+                     const void* dy2, int64_t ld2, int32_t out2, const void* x, int64_t ldx, void* dw,
+                     int32_t dw_dtype, float* workspace, int64_t rows, int32_t in_features, int32_t splits,
+                     int32_t dtype, void* stream);
 
 /* ---- backward (replaces kernels.py:313-356, autograd.py:19-28) --------- */
 
@@ -504,10 +505,59 @@ int p3d_finish_bwd(const p3d_bwd_args* args, const p3d_rope* rope, p3d_view dq, 
 /* Pooling backward (kernels.py:240-270): from the split partials of dsk / dsv
  * (scratch: with more than 16 splits they are summed into the first, in place),
  * writes dkg (gradient of the UNROTATED kg: R^T applied) and dvg into
- * [B,G,N,D] views of dtype (16-byte aligned rows), and per-summary partials
- * dw_part [B*G*Mp, D] and db_part [B*G*Mp, slots]. */
+ * [B,G,N,D] views of dtype (16-byte aligned rows), and partial sums of the
+ * parameter gradients, dw_part [parts, D] and db_part [parts, slots] (the
+ * caller sums the rows; parts = min(B*G*Mp, 2048) lets every wave of a large
+ * launch have one). */
 int p3d_pool_bwd(const p3d_pool_args* pool, float* dsk_part, float* dsv_part, int32_t splits,
-                 p3d_view dkg, p3d_view dvg, float* dw_part, float* db_part, void* stream);
+                 p3d_view dkg, p3d_view dvg, float* dw_part, float* db_part, int32_t parts, void* stream);
+
+/* ---- small passes of the 16-bit training step --------------------------- */
+
+/* One sum of a p3d_sum_rows call: dst[c] (of dtype) = sum over rows of
+ * src[r * stride + c], c < cols, in fp32 and a fixed order. */
+typedef struct p3d_sum_job {
+    const float* src;
+    void* dst;
+    int64_t rows, stride;
+    int32_t cols, dtype;
+} p3d_sum_job;
+
+/* Up to 8 sums of partial gradients in one launch.  jobs is a host array. */
+int p3d_sum_rows(const p3d_sum_job* jobs, int32_t count, void* stream);
+
+/* part[p][c] = sum of column c of x [rows, cols] (16-bit, row stride ldx a
+ * multiple of 8, cols a multiple of 8 up to 256) over the p-th of `parts`
+ * equal row ranges, in fp32: the gate bias gradient before p3d_sum_rows. */
+int p3d_column_sums(const void* x, int64_t ldx, int64_t rows, int32_t cols, int32_t dtype, float* part,
+                    int32_t parts, void* stream);
+
+/* Second entry of the softmax over each of `count` pairs of 16-bit logits
+ * (attention.py:85), in fp32, written as gate_dtype. */
+int p3d_gate_fwd(const void* logits, int32_t dtype, void* gate, int32_t gate_dtype, int64_t count, void* stream);
+
+/* Its backward: dlogits [batch * tokens, 2 heads] of the logits' type from
+ * dgate [batch, heads, tokens] (view strides sb, sh, sn in elements), and the
+ * column sums of the unrounded dlogits (the gradient of a bias that the logits
+ * hold) as part [ceil(batch * tokens / 256), 2 heads], summed by the caller. */
+int p3d_gate_bwd(const void* logits, int32_t dtype, p3d_view dgate, int32_t dgate_dtype, void* dlogits,
+                 float* part, int32_t batch, int32_t heads, int64_t tokens, void* stream);
+
+/* One contiguous tensor of a p3d_cast call. */
+typedef struct p3d_cast_job {
+    const void* src;
+    void* dst;
+    int64_t count;
+    int32_t src_dtype, dst_dtype;
+} p3d_cast_job;
+
+/* Up to 8 casts in one launch.  jobs is a host array. */
+int p3d_cast(const p3d_cast_job* jobs, int32_t count, void* stream);
+
+/* wt [dim][k_pad] = [w0; w1; w2]^T of 16-bit matrices w_i [out_i, dim], zero in
+ * the columns past the last row: the weights operand of p3d_input_grad. */
+int p3d_concat_transpose(const void* w0, int32_t out0, const void* w1, int32_t out1, const void* w2, int32_t out2,
+                         int32_t dim, void* wt, int32_t k_pad, void* stream);
 
 /* ---- self-tests (no counterpart in the reference) ---------------------- */
 

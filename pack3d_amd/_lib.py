@@ -25,7 +25,7 @@ class View(ctypes.Structure):
     _fields_ = [("data", c_void_p), ("sb", c_int64), ("sh", c_int64), ("sn", c_int64)]
 
 
-ABI_VERSION = 20  # P3D_ABI_VERSION in include/pack3d_hip.h
+ABI_VERSION = 21  # P3D_ABI_VERSION in include/pack3d_hip.h
 
 
 class Rope(ctypes.Structure):
@@ -77,6 +77,16 @@ class ProjectArgs(ctypes.Structure):
                 ("eps", c_float)]
 
 
+class SumJob(ctypes.Structure):
+    _fields_ = [("src", c_void_p), ("dst", c_void_p), ("rows", c_int64), ("stride", c_int64), ("cols", c_int32),
+                ("dtype", c_int32)]
+
+
+class CastJob(ctypes.Structure):
+    _fields_ = [("src", c_void_p), ("dst", c_void_p), ("count", c_int64), ("src_dtype", c_int32),
+                ("dst_dtype", c_int32)]
+
+
 _P = c_void_p
 SIGNATURES = {
     "p3d_last_error": ([], ctypes.c_char_p),
@@ -115,8 +125,8 @@ SIGNATURES = {
     "p3d_copy_rows": ([View, View, c_int64, c_int32, c_int64, c_int32, c_int32, _P], c_int32),
     "p3d_input_grad": ([_P, c_int64, c_int32, _P, c_int64, c_int32, _P, c_int64, c_int32, _P, c_int32, _P, c_int64,
                         c_int32, c_int32, _P], c_int32),
-    "p3d_weight_grad3": ([_P, c_int64, c_int32, _P, c_int64, c_int32, _P, c_int64, c_int32, _P, c_int64, _P, _P,
-                          c_int64, c_int32, c_int32, c_int32, _P], c_int32),
+    "p3d_weight_grad3": ([_P, c_int64, c_int32, _P, c_int64, c_int32, _P, c_int64, c_int32, _P, c_int64, _P, c_int32,
+                          _P, c_int64, c_int32, c_int32, c_int32, _P], c_int32),
     "p3d_weight_grad": ([_P, c_int64, _P, c_int64, _P, _P, c_int64, c_int32, c_int32, c_int32, c_int32, _P], c_int32),
     "p3d_mix_bwd": ([ctypes.POINTER(BwdArgs), _P], c_int32),
     "p3d_local_bwd_indexed": ([ctypes.POINTER(BwdArgs), _P, c_int32, _P, c_int32, _P], c_int32),
@@ -126,7 +136,13 @@ SIGNATURES = {
     "p3d_global_bwd_dkv": ([ctypes.POINTER(BwdArgs), _P], c_int32),
     "p3d_transpose_rows": ([View, _P, c_int32, c_int32, c_int32, c_int32, c_int32, _P], c_int32),
     "p3d_finish_bwd": ([ctypes.POINTER(BwdArgs), ctypes.POINTER(Rope), View, View, _P], c_int32),
-    "p3d_pool_bwd": ([ctypes.POINTER(PoolArgs), _P, _P, c_int32, View, View, _P, _P, _P], c_int32),
+    "p3d_pool_bwd": ([ctypes.POINTER(PoolArgs), _P, _P, c_int32, View, View, _P, _P, c_int32, _P], c_int32),
+    "p3d_sum_rows": ([ctypes.POINTER(SumJob), c_int32, _P], c_int32),
+    "p3d_column_sums": ([_P, c_int64, c_int64, c_int32, c_int32, _P, c_int32, _P], c_int32),
+    "p3d_gate_fwd": ([_P, c_int32, _P, c_int32, c_int64, _P], c_int32),
+    "p3d_gate_bwd": ([_P, c_int32, View, c_int32, _P, _P, c_int32, c_int32, c_int64, _P], c_int32),
+    "p3d_cast": ([ctypes.POINTER(CastJob), c_int32, _P], c_int32),
+    "p3d_concat_transpose": ([_P, c_int32, _P, c_int32, _P, c_int32, c_int32, _P, c_int32, _P], c_int32),
 }
 
 _lock = threading.Lock()
@@ -211,6 +227,14 @@ def view3(t: torch.Tensor) -> View:
     """A [B, H, N] tensor (the gate) as a p3d_view."""
     sb, sh, sn = t.stride()
     return View(t.data_ptr(), sb, sh, sn)
+
+
+def sum_rows(jobs, device):
+    """One p3d_sum_rows launch: jobs of (src fp32 [rows, >= cols] with unit
+    column stride, out of any shape with cols elements, contiguous)."""
+    args = (SumJob * len(jobs))(*[SumJob(src.data_ptr(), out.data_ptr(), src.shape[0], src.stride(0), out.numel(),
+                                         DTYPES[out.dtype]) for src, out in jobs])
+    call("p3d_sum_rows", args, len(jobs), stream_of(device))
 
 
 def require_device(t: torch.Tensor, what="tensor"):

@@ -28,8 +28,8 @@ from torch import nn
 
 from . import _lib
 from .core import SUPPORTED_HEAD_DIMS, ForwardPlan, _projection_views, _validate_inputs, pack3d_hip_projections
-from .linear import (InputProjections, LayerNormTrain, OutputResidual, OutputResidualWide, compute_dtype,
-                     layer_norm_train_supported, wide_residual_supported)
+from .linear import (GateProbability, InputProjections, LayerNormTrain, OutputResidual, OutputResidualWide,
+                     compute_dtype, layer_norm_train_supported, wide_residual_supported)
 from .geometry import TokenLayout, blocks_consecutive
 from .rope import axial_rope, balanced_pairs, packed_rope
 
@@ -249,8 +249,11 @@ class PACK3DAttention(nn.Module):
             else:
                 xn = layer_norm(self.norm, x)
             qp, kvp, gl = InputProjections.apply(xn, self.to_q.weight, self.to_kv.weight, self.gate.weight,
-                                                 self.gate.bias, dt)
-            gate = gl.view(b, n, self.heads, 2).softmax(-1)[..., 1].transpose(1, 2)
+                                                 self.gate.bias.detach(), dt)
+            # torch's softmax gives fp32 under autocast and the logits' type
+            # otherwise; the bias gradient comes with the logits' gradient.
+            gate = GateProbability.apply(gl, self.gate.bias, self.heads,
+                                         torch.float32 if torch.is_autocast_enabled("cuda") else gl.dtype)
         else:
             xn = layer_norm(self.norm, x)
             qp, kvp, gl = self.to_q(xn), self.to_kv(xn), self.gate(xn)

@@ -376,15 +376,16 @@ def backward(dy, q, kl, vl, kg, vg, weight, bias, gate, sl, sg, sk, svt, sk_norm
                               _lib.view(kg), _lib.view(vg), geometry.blocks.data_ptr(), w32.data_ptr(),
                               b32.data_ptr(), pool_rope.struct(), sk.data_ptr(), svt.data_ptr(),
                               sk_norm_max.data_ptr())
-    dwp = empty(b * g * mp, d, dtype=f32)
-    dbp = empty(b * g * mp, slots, dtype=f32)
+    # One row of partials per pooling wave; all four parameter sums in one launch.
+    pool_parts = min(b * g * mp, 2048)
+    dwp, dbp = empty(pool_parts, d, dtype=f32), empty(pool_parts, slots, dtype=f32)
     _lib.call("p3d_pool_bwd", pool_args, bufs["dskp"].data_ptr(), bufs["dsvp"].data_ptr(), splits,
-              _lib.view(dkg), _lib.view(dvg), dwp.data_ptr(), dbp.data_ptr(), stream)
+              _lib.view(dkg), _lib.view(dvg), dwp.data_ptr(), dbp.data_ptr(), pool_parts, stream)
     keep += [w32, b32]
-    dweight = dwp.sum(0).to(weight.dtype)
-    dbias = dbp.sum(0).to(bias.dtype)
-    dsl = bufs["dslp"].sum(0).to(sl.dtype)
-    dsg = bufs["dsgp"].sum(0).to(sg.dtype)
+    sums = [(part, empty(*p.shape, dtype=p.dtype if p.dtype in _lib.DTYPES else f32))
+            for part, p in ((dwp, weight), (dbp, bias), (bufs["dslp"], sl), (bufs["dsgp"], sg))]
+    _lib.sum_rows(sums, dev)
+    dweight, dbias, dsl, dsg = (out.to(p.dtype) for (_, out), p in zip(sums, (weight, bias, sl, sg)))
     dgate = bufs["dgate"] if bufs["dgate"].dtype == gate.dtype else bufs["dgate"].to(gate.dtype)
     return dq, dkl, dvl, dkg, dvg, dweight, dbias, dgate, dsl, dsg
 

@@ -690,8 +690,9 @@ struct PoolBwdDev {
     const float *dsk_part, *dsv_part;
     int splits;
     p3d_view dkg, dvg;  // [B, G, N, D] views, storage type, 16-byte aligned rows
-    float *dw_part;    // [B * G * Mp, D]
-    float *db_part;    // [B * G * Mp, V]
+    float *dw_part;    // [parts, D]: one row per wave, zero past the launched waves
+    float *db_part;    // [parts, V]
+    int parts;
 };
 
 template <typename T, int D, bool TAB_LDS>
@@ -733,7 +734,16 @@ __global__ __launch_bounds__(256) void k_pool_bwd(PoolDev a, PoolBwdDev bd) {
         const int f = fs + lane_block;
         return (lane < a.bps * a.V && f < f_end) ? a.blocks[(int64_t)f * a.V + lane_slot] : -1;
     };
-    for (unsigned item = blockIdx.x * waves + wave; item < total; item += stride) {
+    // The parameter gradients accumulate over the wave's items, so that the sum
+    // over partials that follows reads a row per wave instead of one per summary.
+    float dwacc[C::SJ][CPD];
+#pragma unroll
+    for (int j = 0; j < C::SJ; ++j)
+#pragma unroll
+        for (int c = 0; c < CPD; ++c) dwacc[j][c] = 0.f;
+    float dbacc = 0.f;
+    const unsigned wid = blockIdx.x * waves + wave;
+    for (unsigned item = wid; item < total; item += stride) {
         const int g = (int)(item % a.G);
         const unsigned bm = item / a.G;
         const int m = (int)(bm % a.Mp), b = (int)(bm / a.Mp);
@@ -744,12 +754,6 @@ __global__ __launch_bounds__(256) void k_pool_bwd(PoolDev a, PoolBwdDev bd) {
             const uint64_t filled = __ballot(slot_token(fs, f_end) >= 0);
             if (filled) count += blocks_filled(filled, a.bps, a.V);
         }
-        float dwacc[C::SJ][CPD];
-#pragma unroll
-        for (int j = 0; j < C::SJ; ++j)
-#pragma unroll
-            for (int c = 0; c < CPD; ++c) dwacc[j][c] = 0.f;
-        float dbacc = 0.f;
         if (count > 0) {
             const float inv = 1.f / (float)count;
             for (int c = lane; c < D; c += 64) {
@@ -869,8 +873,12 @@ __global__ __launch_bounds__(256) void k_pool_bwd(PoolDev a, PoolBwdDev bd) {
             column_sums_w<C, T>(krows, lw, lane, dwacc);
             wave_lds_sync();  // the next fine block overwrites the rows
         }
-        // Partials of this item: dw (column dwords of group 0) and db (one per slot).
-        float* dwp = bd.dw_part + (int64_t)item * D;
+    }
+    // Slot s's bias gradient sums the lanes holding slot s of any block.
+    for (int o = a.gsz; o < 64; o <<= 1) dbacc += __shfl_xor(dbacc, o);
+    // Partials of this wave: dw (column dwords of group 0) and db (one per slot).
+    if (wid < (unsigned)bd.parts) {
+        float* dwp = bd.dw_part + (int64_t)wid * D;
 #pragma unroll
         for (int j = 0; j < C::SJ; ++j) {
             const int u = lane + 64 * j;
@@ -878,9 +886,11 @@ __global__ __launch_bounds__(256) void k_pool_bwd(PoolDev a, PoolBwdDev bd) {
 #pragma unroll
                 for (int c = 0; c < CPD; ++c) dwp[u * CPD + c] = dwacc[j][c];
         }
-        // Slot s's bias gradient sums the lanes holding slot s of any block.
-        for (int o = a.gsz; o < 64; o <<= 1) dbacc += __shfl_xor(dbacc, o);
-        if (lane < a.V) bd.db_part[(int64_t)item * a.V + lane] = dbacc;
+        if (lane < a.V) bd.db_part[(int64_t)wid * a.V + lane] = dbacc;
+    }
+    for (unsigned q = wid + stride; q < (unsigned)bd.parts; q += stride) {
+        for (int c = lane; c < D; c += 64) bd.dw_part[(int64_t)q * D + c] = 0.f;
+        if (lane < a.V) bd.db_part[(int64_t)q * a.V + lane] = 0.f;
     }
 }
 
@@ -1108,15 +1118,16 @@ void launch_pool_bwd_t(const PoolDev& d, const PoolBwdDev& bd, int64_t items, hi
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     int waves = pool_waves(fixed + tab_bytes, per_wave);
-    while (waves > 1 && cdiv(items, waves) < cus) waves >>= 1;  // as in the forward
+    while (waves > 1 && (cdiv(items, waves) < cus || waves > bd.parts)) waves >>= 1;  // as in the forward
     const size_t smem = fixed + tab_bytes + per_wave * waves;
     if (tab_lds)
         (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pool_bwd<T, D, true>, 64 * waves, smem);
     else
         (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pool_bwd<T, D, false>, 64 * waves, smem);
     const int64_t resident = (int64_t)std::max(1, cus) * std::max(1, per_cu);
-    const int64_t needed = cdiv(items, waves);
-    const int64_t rounds = cdiv(needed, resident);
+    // Every wave that has an item needs its own row of partials.
+    const int64_t needed = cdiv(items, waves), most = bd.parts >= items ? needed : bd.parts / waves;
+    const int64_t rounds = cdiv(needed, std::min(resident, most));
     const unsigned blocks = (unsigned)cdiv(needed, rounds);
     if (tab_lds)
         k_pool_bwd<T, D, true><<<blocks, 64 * waves, smem, s>>>(d, bd);
@@ -1178,14 +1189,15 @@ extern "C" int p3d_rotate(p3d_view x, p3d_view y, int32_t batch, int32_t heads, 
     return check_launch("p3d_rotate");
 }
 
-extern "C" int p3d_pool_bwd(const p3d_pool_args* args, float* dsk_part, float* dsv_part, int32_t splits, p3d_view dkg, p3d_view dvg, float* dw_part, float* db_part,
+extern "C" int p3d_pool_bwd(const p3d_pool_args* args, float* dsk_part, float* dsv_part, int32_t splits,
+                            p3d_view dkg, p3d_view dvg, float* dw_part, float* db_part, int32_t parts,
                             void* stream) {
     PoolDev d;
     if (int rc = fill_pool(args, d)) return rc;
     P3D_REQUIRE(dsk_part && dsv_part && dw_part && db_part, "null pointer argument");
     P3D_REQUIRE(view_ok(dkg, dtype_size(args->dtype)) && view_ok(dvg, dtype_size(args->dtype)),
                 "dkg / dvg rows must be 16-byte aligned");
-    P3D_REQUIRE(splits >= 1, "splits must be positive");
+    P3D_REQUIRE(splits >= 1 && parts >= 1, "splits and parts must be positive");
     const int64_t items = (int64_t)d.B * d.G * d.Mp;
     hipStream_t s = as_stream(stream);
     // Up to 16 splits the pooling waves add them as they go (two rounds of
@@ -1196,7 +1208,7 @@ extern "C" int p3d_pool_bwd(const p3d_pool_args* args, float* dsk_part, float* d
                                                                                              slice4);
         splits = 1;
     }
-    PoolBwdDev bd{dsk_part, dsv_part, splits, dkg, dvg, dw_part, db_part};
+    PoolBwdDev bd{dsk_part, dsv_part, splits, dkg, dvg, dw_part, db_part, parts};
     switch (args->head_dim) {
         case 16: launch_pool_bwd<16>(d, bd, args->dtype, items, s); break;
         case 32: launch_pool_bwd<32>(d, bd, args->dtype, items, s); break;

@@ -173,26 +173,46 @@ __global__ __launch_bounds__(64 * kWgWaves) void k_wgrad(WgSrc<T> dy, const T* x
         }
 }
 
-// dw[e] = sum over splits of part[s][e] in a fixed order: thread group j of
-// a block (64 elements x 4 groups) sums splits j, j + 4, ... in increasing
-// order, then group 0 adds the four partial sums in order (deterministic).
-constexpr int kRedElems = 64, kRedGroups = 4;
-__global__ __launch_bounds__(kRedElems * kRedGroups) void k_wgrad_reduce(const float* part, float* dw, int64_t count,
-                                                                         int splits) {
-    __shared__ float sums[kRedGroups][kRedElems];
+// dw[e] = sum over splits of part[s][e] in a fixed order (deterministic),
+// rounded once to dw's type: thread group j of a block (64 elements x G
+// groups) sums splits j, j + G, ... in increasing order, eight loads issued
+// together, then the groups are added pairwise.  16 groups where there are
+// more than 64 splits (256 of a 192 x 192 gradient, 38 MB: 18 us with 4 groups
+// and one load at a time, 9 us), else 4, whose threads all have work (25 of a
+// 1,040 x 512 gradient, 53 MB: 9 us against 24 us with 16 groups).
+constexpr int kRedElems = 64;
+template <typename TO, int G>
+__global__ __launch_bounds__(kRedElems * G) void k_wgrad_reduce(const float* part, TO* dw, int64_t count, int splits) {
+    __shared__ float sums[G][kRedElems];
     const int le = threadIdx.x % kRedElems, grp = threadIdx.x / kRedElems;
     const int64_t e = (int64_t)blockIdx.x * kRedElems + le;
     float s = 0.f;
     if (e < count)
-        for (int k = grp; k < splits; k += kRedGroups) s += part[(int64_t)k * count + e];
+        for (int k = grp; k < splits; k += 8 * G) {
+            float v[8];
+#pragma unroll
+            for (int i = 0; i < 8; ++i) v[i] = part[(int64_t)min(k + i * G, splits - 1) * count + e];
+#pragma unroll
+            for (int i = 0; i < 8; ++i)
+                if (k + i * G < splits) s += v[i];
+        }
     sums[grp][le] = s;
     __syncthreads();
-    if (grp == 0 && e < count) {
-        float t = sums[0][le];
 #pragma unroll
-        for (int j = 1; j < kRedGroups; ++j) t += sums[j][le];
-        dw[e] = t;
+    for (int h = G / 2; h >= 1; h /= 2) {
+        if (grp < h) sums[grp][le] += sums[grp + h][le];
+        __syncthreads();
     }
+    if (grp == 0 && e < count) dw[e] = from_f32<TO>(sums[0][le]);
+}
+
+template <typename TO>
+void launch_reduce(const float* part, TO* dw, int64_t count, int splits, hipStream_t s) {
+    const unsigned blocks = (unsigned)cdiv(count, kRedElems);
+    if (splits > 64)
+        k_wgrad_reduce<TO, 16><<<blocks, kRedElems * 16, 0, s>>>(part, dw, count, splits);
+    else
+        k_wgrad_reduce<TO, 4><<<blocks, kRedElems * 4, 0, s>>>(part, dw, count, splits);
 }
 
 // Input widths the kernel takes: a multiple of 32 up to 256 (one column
@@ -202,8 +222,8 @@ inline bool wgrad_cols_ok(int I) {
 }
 
 template <typename T>
-int launch_wgrad(const WgSrc<T>& dy, const void* x, int64_t ldx, float* dw, float* part, int64_t rows, int O, int I,
-                 int splits, hipStream_t s) {
+int launch_wgrad(const WgSrc<T>& dy, const void* x, int64_t ldx, void* dw, int dw_dtype, float* part, int64_t rows,
+                 int O, int I, int splits, hipStream_t s) {
     const int64_t per = cdiv(cdiv(rows, splits), kWgTokMax) * kWgTokMax;
     const int used = (int)cdiv(rows, per);
     // Past 256 input columns the columns go to blocks of 256 (grid z), each
@@ -222,7 +242,10 @@ int launch_wgrad(const WgSrc<T>& dy, const void* x, int64_t ldx, float* dw, floa
         default: return fail(P3D_EUNSUPPORTED, "in_features must be a multiple of 32, at most 256");
     }
     const int64_t count = (int64_t)O * I;
-    k_wgrad_reduce<<<(unsigned)cdiv(count, kRedElems), kRedElems * kRedGroups, 0, s>>>(part, dw, count, used);
+    if (dw_dtype == P3D_F32)
+        launch_reduce(part, (float*)dw, count, used, s);
+    else  // the inputs' own type
+        launch_reduce(part, (T*)dw, count, used, s);
     return check_launch("p3d_weight_grad");
 }
 
@@ -246,20 +269,21 @@ extern "C" int p3d_weight_grad(const void* dy, int64_t ldy, const void* x, int64
     P3D_REQUIRE(cdiv(out_features, kWgRows) < 65536 && splits < 65536, "grid too large");
     if (dtype == P3D_F16) {
         const WgSrc<_Float16> src{{(const _Float16*)dy, nullptr, nullptr}, {ldy, 0, 0}, {out_features, out_features}};
-        return launch_wgrad<_Float16>(src, x, ldx, dw, workspace, rows, out_features, in_features, splits,
+        return launch_wgrad<_Float16>(src, x, ldx, dw, P3D_F32, workspace, rows, out_features, in_features, splits,
                                       as_stream(stream));
     }
     const WgSrc<__bf16> src{{(const __bf16*)dy, nullptr, nullptr}, {ldy, 0, 0}, {out_features, out_features}};
-    return launch_wgrad<__bf16>(src, x, ldx, dw, workspace, rows, out_features, in_features, splits,
+    return launch_wgrad<__bf16>(src, x, ldx, dw, P3D_F32, workspace, rows, out_features, in_features, splits,
                                 as_stream(stream));
 }
 
 extern "C" int p3d_weight_grad3(const void* dy0, int64_t ld0, int32_t out0, const void* dy1, int64_t ld1,
                                 int32_t out1, const void* dy2, int64_t ld2, int32_t out2, const void* x, int64_t ldx,
-                                float* dw, float* workspace, int64_t rows, int32_t in_features, int32_t splits,
-                                int32_t dtype, void* stream) {
+                                void* dw, int32_t dw_dtype, float* workspace, int64_t rows, int32_t in_features,
+                                int32_t splits, int32_t dtype, void* stream) {
     P3D_REQUIRE(dy0 && dy1 && dy2 && x && dw && workspace, "null pointer argument");
     P3D_REQUIRE(dtype == P3D_F16 || dtype == P3D_BF16, "dtype must be fp16 or bf16");
+    P3D_REQUIRE(dw_dtype == P3D_F32 || dw_dtype == dtype, "dw is fp32 or of the inputs' type");
     P3D_REQUIRE(rows >= 1 && splits >= 1, "need at least one row and one split");
     P3D_REQUIRE(out0 >= 8 && out1 >= 8 && out2 >= 8 && out0 % 8 == 0 && out1 % 8 == 0 && out2 % 8 == 0 &&
                     (int64_t)out0 + out1 + out2 < (1 << 24),
@@ -276,9 +300,10 @@ extern "C" int p3d_weight_grad3(const void* dy0, int64_t ld0, int32_t out0, cons
         const WgSrc<_Float16> src{{(const _Float16*)dy0, (const _Float16*)dy1, (const _Float16*)dy2},
                                   {ld0, ld1, ld2},
                                   {out0, out0 + out1}};
-        return launch_wgrad<_Float16>(src, x, ldx, dw, workspace, rows, O, in_features, splits, as_stream(stream));
+        return launch_wgrad<_Float16>(src, x, ldx, dw, dw_dtype, workspace, rows, O, in_features, splits,
+                                      as_stream(stream));
     }
     const WgSrc<__bf16> src{{(const __bf16*)dy0, (const __bf16*)dy1, (const __bf16*)dy2}, {ld0, ld1, ld2},
                             {out0, out0 + out1}};
-    return launch_wgrad<__bf16>(src, x, ldx, dw, workspace, rows, O, in_features, splits, as_stream(stream));
+    return launch_wgrad<__bf16>(src, x, ldx, dw, dw_dtype, workspace, rows, O, in_features, splits, as_stream(stream));
 }

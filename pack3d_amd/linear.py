@@ -16,6 +16,7 @@ in fp32 (torch's autocast path rounds them to the compute type first).
 from __future__ import annotations
 
 import torch
+from torch.autograd.function import once_differentiable
 
 from . import _lib
 
@@ -34,7 +35,12 @@ MIN_ROWS_PER_SPLIT = 512
 
 def splits_for(rows, out_features, in_features):
     blocks = -(-out_features // WG_ROWS) * max(1, in_features // WG_COLS)
-    return max(1, min(max(1, WORKGROUPS // blocks), rows // MIN_ROWS_PER_SPLIT))
+    # Small gradients may be split finer, as long as a split's partials (written
+    # and read, 8 bytes an element) stay below the bytes of its rows of dy and
+    # x: 4,096 rows of 64 x 64 run on 32 workgroups instead of 8 (21 -> 9 us).
+    rows_per = max(128, min(MIN_ROWS_PER_SPLIT,
+                            4 * out_features * in_features // (out_features + in_features)))
+    return max(1, min(max(1, WORKGROUPS // blocks), rows // rows_per))
 
 
 def compute_dtype(x):
@@ -72,8 +78,10 @@ def input_grad(dys, ws):
         return None
     k = sum(outs)
     k_pad = -(-k // 64) * 64
-    wt = torch.zeros(dim, k_pad, dtype=dt, device=ws[0].device)
-    wt[:, :k] = torch.cat(ws, 0).t()
+    wt = torch.empty(dim, k_pad, dtype=dt, device=ws[0].device)
+    ws = [w.contiguous() for w in ws]
+    _lib.call("p3d_concat_transpose", ws[0].data_ptr(), outs[0], ws[1].data_ptr(), outs[1], ws[2].data_ptr(), outs[2],
+              dim, wt.data_ptr(), k_pad, _lib.stream_of(wt.device))
     dx = torch.empty(rows, dim, dtype=dt, device=ws[0].device)
     _lib.call("p3d_input_grad", dys[0].data_ptr(), dys[0].stride(0), outs[0], dys[1].data_ptr(), dys[1].stride(0),
               outs[1], dys[2].data_ptr(), dys[2].stride(0), outs[2], wt.data_ptr(), k_pad, dx.data_ptr(), rows, dim,
@@ -131,11 +139,12 @@ def weight_grad(dy, x):
     return dw
 
 
-def weight_grads3(dys, x):
+def weight_grads3(dys, x, out_dtype=torch.float32):
     """dW of three linear maps sharing the input x: [dy0^T x; dy1^T x;
-    dy2^T x] in fp32 from one pass over x (``p3d_weight_grad3``), as three
-    tensors; None where the kernel does not take the shapes (the caller
-    then takes them one at a time)."""
+    dy2^T x] summed in fp32 from one pass over x (``p3d_weight_grad3``) and
+    returned as three tensors of out_dtype (fp32 or x's type); None where the
+    kernel does not take the shapes (the caller then takes them one at a
+    time)."""
     rows, in_f = x.shape
     outs = [dy.shape[1] for dy in dys]
     dt = x.dtype
@@ -146,12 +155,88 @@ def weight_grads3(dys, x):
         return None
     total = sum(outs)
     splits = splits_for(rows, total, in_f)
-    dw = torch.empty(total, in_f, dtype=torch.float32, device=x.device)
+    dw = torch.empty(total, in_f, dtype=out_dtype, device=x.device)
     work = torch.empty(splits, total, in_f, dtype=torch.float32, device=x.device)
     _lib.call("p3d_weight_grad3", dys[0].data_ptr(), dys[0].stride(0), outs[0], dys[1].data_ptr(), dys[1].stride(0),
               outs[1], dys[2].data_ptr(), dys[2].stride(0), outs[2], x.data_ptr(), x.stride(0), dw.data_ptr(),
-              work.data_ptr(), rows, in_f, splits, _lib.DTYPES[dt], _lib.stream_of(x.device))
+              _lib.DTYPES[out_dtype], work.data_ptr(), rows, in_f, splits, _lib.DTYPES[dt], _lib.stream_of(x.device))
     return torch.split(dw, outs, 0)
+
+
+def column_sums(x, dtype):
+    """Sum over the rows of a 16-bit x [rows, cols] in fp32, rounded to dtype
+    (``p3d_column_sums`` and one ``p3d_sum_rows``; torch where they do not
+    take the shape)."""
+    rows, cols = x.shape
+    if (x.dtype not in (torch.float16, torch.bfloat16) or dtype not in _lib.DTYPES or not 8 <= cols <= 256 or cols % 8
+            or x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < cols or x.data_ptr() % 16):
+        return x.float().sum(0).to(dtype)
+    parts = max(1, min(512, rows // 128))
+    part = torch.empty(parts, cols, dtype=torch.float32, device=x.device)
+    out = torch.empty(cols, dtype=dtype, device=x.device)
+    _lib.call("p3d_column_sums", x.data_ptr(), x.stride(0), rows, cols, _lib.DTYPES[x.dtype], part.data_ptr(), parts,
+              _lib.stream_of(x.device))
+    _lib.sum_rows([(part, out)], x.device)
+    return out
+
+
+def cast_all(tensors, dt):
+    """The tensors in the 16-bit type dt, contiguous: those of another type cast
+    in one launch (``p3d_cast``)."""
+    out = [t.contiguous() if t.dtype == dt else None for t in tensors]
+    todo = [i for i, t in enumerate(out) if t is None]
+    if any(tensors[i].dtype not in _lib.DTYPES or tensors[i].numel() == 0 for i in todo) or len(todo) > 8:
+        return [t.to(dt).contiguous() for t in tensors]
+    if todo:
+        jobs = (_lib.CastJob * len(todo))()
+        keep = []
+        for job, i in zip(jobs, todo):
+            src = tensors[i].contiguous()
+            keep.append(src)
+            out[i] = torch.empty(src.shape, dtype=dt, device=src.device)
+            job.src, job.dst, job.count = src.data_ptr(), out[i].data_ptr(), src.numel()
+            job.src_dtype, job.dst_dtype = _lib.DTYPES[src.dtype], _lib.DTYPES[dt]
+        _lib.call("p3d_cast", jobs, len(todo), _lib.stream_of(out[todo[0]].device))
+    return out
+
+
+class GateProbability(torch.autograd.Function):
+    """The gate of attention.py:85 from its 16-bit logits gl [B, N, 2 H] (pairs
+    per head): the second entry of each pair's softmax as [B, H, N] (a transposed
+    view), in out_dtype.  Computed in fp32 from the logits in both directions,
+    one kernel each (``p3d_gate_fwd`` / ``p3d_gate_bwd``).  bias: the bias that
+    gl already holds, whose gradient is summed from the unrounded logit
+    gradients in the same pass (the product that made gl then takes the bias
+    detached); None where the product's own backward gives it."""
+
+    @staticmethod
+    def forward(ctx, gl, bias, heads, out_dtype):
+        gl = gl.contiguous()
+        b, n = gl.shape[0], gl.shape[1]
+        gate = torch.empty(b, n, heads, dtype=out_dtype, device=gl.device)
+        _lib.call("p3d_gate_fwd", gl.data_ptr(), _lib.DTYPES[gl.dtype], gate.data_ptr(), _lib.DTYPES[out_dtype],
+                  gate.numel(), _lib.stream_of(gl.device))
+        ctx.save_for_backward(gl)
+        ctx.meta = (heads, None if bias is None else bias.dtype)
+        return gate.transpose(1, 2)
+
+    @staticmethod
+    @once_differentiable
+    def backward(ctx, dgate):
+        (gl,) = ctx.saved_tensors
+        heads, bias_dtype = ctx.meta
+        b, n = gl.shape[0], gl.shape[1]
+        dgl = torch.empty_like(gl)
+        part = torch.empty(-(-b * n // 256), 2 * heads, dtype=torch.float32, device=gl.device)
+        _lib.call("p3d_gate_bwd", gl.data_ptr(), _lib.DTYPES[gl.dtype], _lib.view3(dgate), _lib.DTYPES[dgate.dtype],
+                  dgl.data_ptr(), part.data_ptr(), b, heads, n, _lib.stream_of(gl.device))
+        dbias = None
+        if bias_dtype is not None and ctx.needs_input_grad[1]:
+            dbias = torch.empty(2 * heads, dtype=bias_dtype if bias_dtype in _lib.DTYPES else torch.float32,
+                                device=gl.device)
+            _lib.sum_rows([(part, dbias)], gl.device)
+            dbias = dbias.to(bias_dtype)
+        return dgl, dbias, None, None
 
 
 def _rows(t):
@@ -217,14 +302,17 @@ class LayerNormTrain(torch.autograd.Function):
             dy2 = dy2.float()
         dx = torch.empty_like(x2)
         dr = None if dres is None else _rows(dres).to(dx.dtype).contiguous()
-        parts = max(1, min(1024, rows // 256))
+        # Row ranges of the affine partials, and with them workgroups: 256 rows
+        # each left 64 workgroups at 16,384 rows (72 us at dim 512; 18 us).
+        parts = max(1, min(1024, rows // 32))
         part = torch.empty(parts, 2, dim, dtype=torch.float32, device=x2.device)
         _lib.call("p3d_layer_norm_bwd", dy2.data_ptr(), 0 if dr is None else dr.data_ptr(), x2.data_ptr(),
                   weight.data_ptr(), _lib.DTYPES[weight.dtype], mean.data_ptr(), rstd.data_ptr(), dx.data_ptr(),
                   part.data_ptr(), rows, dim, _lib.DTYPES[dy2.dtype], _lib.DTYPES[x2.dtype], _lib.DTYPES[dx.dtype],
                   parts, _lib.stream_of(x2.device))
-        sums = part.sum(0)
-        return dx.view(shape), sums[0].to(weight.dtype), sums[1].to(b_dt), None, None, None
+        dw, db = (torch.empty(dim, dtype=t, device=x2.device) for t in (weight.dtype, b_dt))
+        _lib.sum_rows([(part[:, 0], dw), (part[:, 1], db)], x2.device)
+        return dx.view(shape), dw, db, None, None, None
 
 
 class InputProjections(torch.autograd.Function):
@@ -237,14 +325,14 @@ class InputProjections(torch.autograd.Function):
     @staticmethod
     def forward(ctx, x, wq, wkv, wg, bg, dt):
         x16 = _rows(x).to(dt).contiguous()
-        ws = [w.to(dt) for w in (wq, wkv, wg)]
-        made = project_linear(x16, ws, bg)
+        *ws, bg16 = cast_all((wq, wkv, wg, bg), dt)
+        made = project_linear(x16, ws, bg16)
         if made is not None:
             q, kv, gl = made
         else:
             q = torch.mm(x16, ws[0].t())
             kv = torch.mm(x16, ws[1].t())
-            gl = torch.addmm(bg.to(dt), x16, ws[2].t())
+            gl = torch.addmm(bg16, x16, ws[2].t())
         ctx.save_for_backward(x16, *ws)
         ctx.meta = (x.shape, x.dtype, wq.dtype, wkv.dtype, wg.dtype, bg.dtype)
         lead = x.shape[:-1]
@@ -265,7 +353,8 @@ class InputProjections(torch.autograd.Function):
         if wide:
             dx = torch.zeros(x16.shape, dtype=torch.float32, device=x16.device)
         # The three weight gradients from one pass over x16 where the kernel takes them.
-        dws = None if any(dy is None for dy in dys) else weight_grads3(dys, x16)
+        same = x16.dtype if wq_dt == wkv_dt == wg_dt == x16.dtype else torch.float32
+        dws = None if any(dy is None for dy in dys) else weight_grads3(dys, x16, same)
         grads = []
         for i, (dy, w, w_dt) in enumerate(zip(dys, (wq, wkv, wg), (wq_dt, wkv_dt, wg_dt))):
             if dy is None:
@@ -280,7 +369,7 @@ class InputProjections(torch.autograd.Function):
             grads.append((weight_grad(dy, x16) if dws is None else dws[i]).to(w_dt))
         if dx is None:
             dx = torch.zeros(x16.shape, dtype=x16.dtype, device=x16.device)
-        dbg = None if dgl is None else _rows(dgl).float().sum(0).to(bg_dt)
+        dbg = column_sums(_rows(dgl), bg_dt) if dgl is not None and ctx.needs_input_grad[4] else None
         return dx.view(shape).to(x_dt), grads[0], grads[1], grads[2], dbg, None
 
 
