@@ -51,6 +51,19 @@ struct AttnDev {
     int kl_rotated;    // kl already rotated: the grid kernel rotates q only
 };
 
+// Strips: a grid of one z plane fills only one of a brick's four query planes.
+// There the four planes hold four strips of 8 rows instead: plane z of the
+// kernel is rows 8 z .. 8 z + 7 of the grid (Z = ceil(Y / 8) strips, rz = 0, one
+// brick in y), each with its own halo plane, whose y halo reaches into the
+// neighbouring strips.  A brick then holds 256 queries instead of 64, so a
+// quarter of the workgroups do the summary sweep and the set-up: 128 x 128
+// slices with 8 heads of 64, 150 us with 4 x 8 x 8 bricks, FLAT_FWD us in strips.
+// (STRIPS is a template argument: as a run-time flag it cost the bricks registers.)
+template <bool STRIPS>
+__device__ __forceinline__ int real_y(int gz, int gy) { return STRIPS ? 8 * gz + gy : gy; }
+template <bool STRIPS>
+__device__ __forceinline__ int real_z(int gz) { return STRIPS ? 0 : gz; }
+
 template <typename T>
 __device__ __forceinline__ const T* tp(const char* p) { return reinterpret_cast<const T*>(p); }
 
@@ -600,6 +613,7 @@ struct PlaneStager {
     static constexpr int ITERS = (TASKS + 64 * kWaves - 1) / (64 * kWaves);
     typedef __attribute__((ext_vector_type(2))) T T2;
 
+    template <bool STRIPS>
     __device__ __forceinline__ void stage(const AttnDev& a, const T* KL, const T* VL, int hz, int gz, int Y0,
                                           int X0, const RopeWindow& win, T* Kp, T* Vp, int vps) const {
 #pragma unroll
@@ -608,7 +622,7 @@ struct PlaneStager {
             if (task >= TASKS) break;
             const int piece = task % PPR, grp = task / PPR;
             const int ky = grp / (kPlane / 4), kx0 = 4 * (grp % (kPlane / 4));
-            const int gy = Y0 - a.ry + ky;
+            const int gy = real_y<STRIPS>(gz, Y0 - a.ry + ky);
             const bool row_in = gz >= 0 && gz < a.Z && gy >= 0 && gy < a.Y && ky < 8 + 2 * a.ry;
             // Two halves of 2 keys: loads of a half are issued before it is consumed.
 #pragma unroll
@@ -622,7 +636,7 @@ struct PlaneStager {
                     in[i] = row_in && gx >= 0 && gx < a.X && kx < 8 + 2 * a.rx;
                     kraw[i] = vraw[i] = uint4{0, 0, 0, 0};
                     if (in[i]) {
-                        const int64_t raster = ((int64_t)gz * a.Y + gy) * a.X + gx;
+                        const int64_t raster = ((int64_t)real_z<STRIPS>(gz) * a.Y + gy) * a.X + gx;
                         const int64_t row = a.map ? (int64_t)a.map[raster] : raster;
                         kraw[i] = *reinterpret_cast<const uint4*>(KL + row * a.ksn + piece * EP);
                         vraw[i] = *reinterpret_cast<const uint4*>(VL + row * a.vsn + piece * EP);
@@ -723,14 +737,15 @@ struct PlaneDma {
     static_assert(C::KSTR % EP == 0 && C::KSTR > C::D, "key rows need a spare slot");
 
     // Packed rows of the halo keys of planes [0, planes) (z from Z0 - rz).
+    template <bool STRIPS>
     __device__ __forceinline__ static void fill_rows(const AttnDev& a, int Z0, int Y0, int X0, int planes,
                                                      int* rows) {
         for (int i = threadIdx.x; i < planes * KEYS; i += blockDim.x) {
             const int hz = i / KEYS, k = i - hz * KEYS, ky = k / PW, kx = k - ky * PW;
             const int gz = min(max(Z0 - a.rz + hz, 0), a.Z - 1);
-            const int gy = min(max(Y0 - a.ry + ky, 0), a.Y - 1);
+            const int gy = min(max(real_y<STRIPS>(gz, Y0 - a.ry + ky), 0), a.Y - 1);
             const int gx = min(max(X0 - a.rx + kx, 0), a.X - 1);
-            const int64_t raster = ((int64_t)gz * a.Y + gy) * a.X + gx;
+            const int64_t raster = ((int64_t)real_z<STRIPS>(gz) * a.Y + gy) * a.X + gx;
             rows[i] = a.map ? a.map[raster] : (int)raster;
         }
     }
@@ -878,7 +893,7 @@ __device__ __forceinline__ void plane_chunks(const AttnDev& a, const typename C:
     }
 }
 
-template <typename T, int D, int PW>
+template <typename T, int D, int PW, bool STRIPS>
 __global__ __launch_bounds__(64 * kWaves, 2) void k_attn_grid(AttnDev a) {
     typedef Cfg<T, D> C;
     constexpr int EP = Piece<T>::N;
@@ -909,8 +924,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_attn_grid(AttnDev a) {
     const int planes = 4 + 2 * a.rz;
     const T* KL = tp<T>(a.kl) + b * a.ksb + kvh * a.ksh;
     const T* VL = tp<T>(a.vl) + b * a.vsb + kvh * a.vsh;
-    if (!a.rope.packed) build_rope_window(a, D, Z0 - a.rz, Y0 - a.ry, X0 - a.rx, win);
-    if constexpr (DMA) PD::fill_rows(a, Z0, Y0, X0, planes, rowtab);
+    if (!STRIPS && !a.rope.packed) build_rope_window(a, D, Z0 - a.rz, Y0 - a.ry, X0 - a.rx, win);
+    if constexpr (DMA) PD::template fill_rows<STRIPS>(a, Z0, Y0, X0, planes, rowtab);
     __syncthreads();
     const int uwave = __builtin_amdgcn_readfirstlane(wave);
     if constexpr (DMA) {
@@ -924,13 +939,15 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_attn_grid(AttnDev a) {
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
         const int qz = 2 * nb + (qi >> 4);
-        const int gz = Z0 + qz, gy = Y0 + 4 * wy + qy, gx = X0 + 4 * wx + qx;
+        const int gz = Z0 + qz, gy = real_y<STRIPS>(gz, Y0 + 4 * wy + qy), gx = X0 + 4 * wx + qx;
         qok[nb] = gz < a.Z && gy < a.Y && gx < a.X;
-        const int64_t raster = ((int64_t)gz * a.Y + gy) * a.X + gx;
+        const int64_t raster = ((int64_t)real_z<STRIPS>(gz) * a.Y + gy) * a.X + gx;
         qrow[nb] = qok[nb] ? (a.map ? (int64_t)a.map[raster] : raster) : 0;
         const T* row = tp<T>(a.q) + b * a.qsb + h * a.qsh + qrow[nb] * a.qsn;
-        if (a.rope.packed) {
-            const int64_t pos[3] = {qrow[nb], 0, 0};
+        if (a.rope.packed || STRIPS) {
+            // A brick's strips span more rows than the window holds.
+            int64_t pos[3] = {qrow[nb], 0, 0};
+            if (STRIPS && !a.rope.packed) pos[0] = 0, pos[1] = gy, pos[2] = gx;
             load_q<C>(row, qok[nb], [&](int j) { return rope_cs(a.rope, j, pos); }, g, qf[nb]);
         } else {
             const int wz = qz + a.rz, wy_ = 4 * wy + qy + a.ry, wx_ = 4 * wx + qx + a.rx;
@@ -943,8 +960,8 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_attn_grid(AttnDev a) {
     st[1].reset();
 
     // ---- local pathway: halo planes z = Z0 - rz .. Z0 + 3 + rz
-    const uint32_t kmask[2] = {stencil_mask<C>(a, 0, g, qy, qx, Y0 + 4 * wy, X0 + 4 * wx),
-                               stencil_mask<C>(a, 1, g, qy, qx, Y0 + 4 * wy, X0 + 4 * wx)};
+    uint32_t kmask[2] = {stencil_mask<C>(a, 0, g, qy, qx, Y0 + 4 * wy, X0 + 4 * wx),
+                         stencil_mask<C>(a, 1, g, qy, qx, Y0 + 4 * wy, X0 + 4 * wx)};
     if constexpr (DMA) {
         for (int hz = 0; hz < planes; ++hz) {
             const int gz = Z0 - a.rz + hz;
@@ -957,6 +974,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_attn_grid(AttnDev a) {
                 PD::copy(a, KL, VL, rowtab + (hz + 1) * PD::KEYS, planes_lds + ((hz + 1) & 1) * PD::BUF, uwave,
                          lane);
             if ((unsigned)gz >= (unsigned)a.Z) continue;  // plane outside the grid: nothing to attend
+            if constexpr (STRIPS) {  // the plane's own rows
+                kmask[0] = stencil_mask<C>(a, 0, g, qy, qx, real_y<STRIPS>(gz, 4 * wy), X0 + 4 * wx);
+                kmask[1] = stencil_mask<C>(a, 1, g, qy, qx, real_y<STRIPS>(gz, 4 * wy), X0 + 4 * wx);
+            }
             T* const Kb = reinterpret_cast<T*>(buf);
             const T* const Vb = reinterpret_cast<const T*>(buf + PD::REGION);
             if (!a.kl_rotated) {
@@ -976,9 +997,13 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_attn_grid(AttnDev a) {
         for (int hz = 0; hz < planes; ++hz) {
             const int gz = Z0 - a.rz + hz;
             if (hz) __syncthreads();
-            stager.stage(a, KL, VL, hz, gz, Y0, X0, win, Kp, Vp, VPS);
+            stager.template stage<STRIPS>(a, KL, VL, hz, gz, Y0, X0, win, Kp, Vp, VPS);
             __syncthreads();
             if ((unsigned)gz >= (unsigned)a.Z) continue;  // plane outside the grid: nothing to attend
+            if constexpr (STRIPS) {  // the plane's own rows
+                kmask[0] = stencil_mask<C>(a, 0, g, qy, qx, real_y<STRIPS>(gz, 4 * wy), X0 + 4 * wx);
+                kmask[1] = stencil_mask<C>(a, 1, g, qy, qx, real_y<STRIPS>(gz, 4 * wy), X0 + 4 * wx);
+            }
             plane_chunks<C, kPlane>(a, Kp,
                             [&](int c, int mb, int ks) {
                                 const int k0 = ks * C::KS + C::E * g;  // chunk key (4c + k0/8, k0 % 8) of the footprint
@@ -1094,29 +1119,32 @@ size_t lds_rows() {
 }
 
 template <typename T, int D, int PW>
-void launch_grid_t(const AttnDev& d, dim3 grid, hipStream_t s) {
-    k_attn_grid<T, D, PW><<<grid, 64 * kWaves, lds_grid<T, D, PW>(), s>>>(d);
+void launch_grid_t(const AttnDev& d, bool strips, dim3 grid, hipStream_t s) {
+    if (strips)
+        k_attn_grid<T, D, PW, true><<<grid, 64 * kWaves, lds_grid<T, D, PW>(), s>>>(d);
+    else
+        k_attn_grid<T, D, PW, false><<<grid, 64 * kWaves, lds_grid<T, D, PW>(), s>>>(d);
 }
 
 // Head_dim 64 in a 16-bit type with radius <= 1 stages its halo planes by the
 // LDS DMA on 10-wide planes; everything else takes 12-wide planes.
 template <int D>
-int launch_grid(const AttnDev& d, int dtype, dim3 grid, hipStream_t s) {
+int launch_grid(const AttnDev& d, int dtype, bool strips, dim3 grid, hipStream_t s) {
     constexpr int NARROW = D == 64 ? 10 : 12;
     const bool narrow = NARROW != 12 && d.rz <= 1 && d.ry <= 1 && d.rx <= 1;
     switch (dtype) {
-        case P3D_F32: launch_grid_t<float, D, 12>(d, grid, s); break;
+        case P3D_F32: launch_grid_t<float, D, 12>(d, strips, grid, s); break;
         case P3D_F16:
             if (narrow)
-                launch_grid_t<_Float16, D, NARROW>(d, grid, s);
+                launch_grid_t<_Float16, D, NARROW>(d, strips, grid, s);
             else
-                launch_grid_t<_Float16, D, 12>(d, grid, s);
+                launch_grid_t<_Float16, D, 12>(d, strips, grid, s);
             break;
         default:
             if (narrow)
-                launch_grid_t<__bf16, D, NARROW>(d, grid, s);
+                launch_grid_t<__bf16, D, NARROW>(d, strips, grid, s);
             else
-                launch_grid_t<__bf16, D, 12>(d, grid, s);
+                launch_grid_t<__bf16, D, 12>(d, strips, grid, s);
             break;
     }
     return check_launch("p3d_attn_fwd_grid");
@@ -1149,13 +1177,21 @@ extern "C" int p3d_attn_fwd_grid(const p3d_attn_args* args, void* stream) {
     d.Z = args->grid[0], d.Y = args->grid[1], d.X = args->grid[2];
     d.rz = args->radius[0], d.ry = args->radius[1], d.rx = args->radius[2];
     d.bricks_y = (int)cdiv(d.Y, 8), d.bricks_x = (int)cdiv(d.X, 8);
+    // Strips once the bricks of a one-plane grid are more than the GPU holds at a
+    // time (two workgroups on each of 256 CUs); fewer run side by side, and
+    // four strips in turn would only make each of them longer.  Unrotated
+    // keys take the rotation window, which strips do not build.
+    const bool strips = d.Z == 1 && d.kl_rotated && (int64_t)d.bricks_y * d.bricks_x * d.B * d.H > 512;
+    if (strips) {
+        d.Z = d.bricks_y, d.bricks_y = 1, d.rz = 0;
+    }
     const int64_t bricks = cdiv(d.Z, 4) * d.bricks_y * d.bricks_x;
     P3D_REQUIRE(bricks * d.B * d.H < (1LL << 31), "launch grid too large");
     dim3 grid((unsigned)(bricks * d.B * d.H));
     hipStream_t s = as_stream(stream);
     switch (args->head_dim) {
 #define CASE(DD) \
-    case DD: return launch_grid<DD>(d, args->dtype, grid, s);
+    case DD: return launch_grid<DD>(d, args->dtype, strips, grid, s);
         P3D_HEAD_DIMS(CASE)
 #undef CASE
         default: return fail(P3D_EUNSUPPORTED, "head_dim must be one of 16, 32, 48, 64, 128");

@@ -41,11 +41,20 @@ struct LbDev {
     float scale_log2, scale;   // log2(e)/sqrt(D), 1/sqrt(D)
 };
 
+// A grid of one z plane in strips of 8 rows, as in the forward kernel: plane z
+// of a brick is rows 8 z .. 8 z + 7 of the grid with a halo plane of its own
+// (Z counts strips, rz = 0, one brick in y).  128 x 128 slices with 8 / 2 heads of
+// 64: dQ 102 -> FLAT_DQ us, dK/dV 88 -> FLAT_DKV us.
+template <bool STRIPS>
+__device__ __forceinline__ int real_y(int gz, int gy) { return STRIPS ? 8 * gz + gy : gy; }
+
 template <typename T>
 __device__ __forceinline__ const T* tp(const char* p) { return reinterpret_cast<const T*>(p); }
 
+// gy: the grid's own row (real_y) where the planes are strips.
+template <bool STRIPS>
 __device__ __forceinline__ int64_t packed_row(const LbDev& a, int gz, int gy, int gx) {
-    const int64_t raster = ((int64_t)gz * a.Y + gy) * a.X + gx;
+    const int64_t raster = ((int64_t)(STRIPS ? 0 : gz) * a.Y + gy) * a.X + gx;
     return a.map ? (int64_t)a.map[raster] : raster;
 }
 
@@ -72,6 +81,12 @@ __device__ __forceinline__ uint32_t chunk_mask(const LbDev& a, int c, int g, int
         m |= (ok ? 1u : 0u) << r;
     }
     return m;
+}
+
+template <typename C>
+__device__ __forceinline__ void chunk_masks(const LbDev& a, int g, int py, int px, int Yw, int Xw, uint32_t (&m)[2]) {
+#pragma unroll
+    for (int c = 0; c < 2; ++c) m[c] = chunk_mask<C>(a, c, g, py, px, Yw, Xw);
 }
 
 // Plane position of chunk c's tile row kappa (natural order) in a wave footprint.
@@ -118,7 +133,7 @@ __device__ __forceinline__ void fit_fp16(float* ds, int& shift, f32x16* acc) {
 // Stage one halo plane of two row tensors: rows (stride KSTR) of both and the
 // transposes (stride TPS) of the tensors selected by TRANS_A / TRANS_B.
 // Positions outside the grid or the halo are zero.
-template <typename C, bool TRANS_A, bool TRANS_B>
+template <typename C, bool TRANS_A, bool TRANS_B, bool STRIPS>
 __device__ __forceinline__ void stage_plane(const LbDev& a, const typename C::T_* A, int64_t asn,
                                             const typename C::T_* Bt, int64_t bsn, int gz, int Y0, int X0,
                                             typename C::T_* Ar, typename C::T_* Br, typename C::T_* At,
@@ -129,12 +144,12 @@ __device__ __forceinline__ void stage_plane(const LbDev& a, const typename C::T_
     for (int task = threadIdx.x; task < TASKS; task += 64 * kWaves) {
         const int piece = task % PPR, pos = task / PPR;
         const int ky = pos / kPlane, kx = pos - ky * kPlane;
-        const int gy = Y0 - a.ry + ky, gx = X0 - a.rx + kx;
+        const int gy = real_y<STRIPS>(gz, Y0 - a.ry + ky), gx = X0 - a.rx + kx;
         const bool in = (unsigned)gz < (unsigned)a.Z && (unsigned)gy < (unsigned)a.Y && (unsigned)gx < (unsigned)a.X &&
                         ky < 8 + 2 * a.ry && kx < 8 + 2 * a.rx;
         uint4 ra = uint4{0, 0, 0, 0}, rb = uint4{0, 0, 0, 0};
         if (in) {
-            const int64_t row = packed_row(a, gz, gy, gx);
+            const int64_t row = packed_row<STRIPS>(a, gz, gy, gx);
             ra = *reinterpret_cast<const uint4*>(A + row * asn + piece * EP);
             rb = *reinterpret_cast<const uint4*>(Bt + row * bsn + piece * EP);
         }
@@ -282,13 +297,14 @@ struct BwdPlaneDma {
     static_assert(2 * BUF <= 128 * 1024, "copy destinations below 128 KB");
 
     // Packed rows of the halo positions of planes [0, planes) (z from Z0 - rz).
+    template <bool STRIPS>
     __device__ __forceinline__ static void fill_rows(const LbDev& a, int Z0, int Y0, int X0, int planes, int* rows) {
         for (int i = threadIdx.x; i < planes * kPlaneKeys; i += blockDim.x) {
             const int hz = i / kPlaneKeys, k = i - hz * kPlaneKeys, ky = k / kPlane, kx = k - ky * kPlane;
             const int gz = min(max(Z0 - a.rz + hz, 0), a.Z - 1);
-            const int gy = min(max(Y0 - a.ry + ky, 0), a.Y - 1);
+            const int gy = min(max(real_y<STRIPS>(gz, Y0 - a.ry + ky), 0), a.Y - 1);
             const int gx = min(max(X0 - a.rx + kx, 0), a.X - 1);
-            rows[i] = (int)packed_row(a, gz, gy, gx);
+            rows[i] = (int)packed_row<STRIPS>(a, gz, gy, gx);
         }
     }
 
@@ -329,7 +345,7 @@ struct BwdPlaneDma {
     }
 };
 
-template <typename T, int D>
+template <typename T, int D, bool STRIPS>
 __global__ __launch_bounds__(64 * kWaves) void k_local_dq_grid(LbDev a) {
     typedef Cfg<T, D> C;
     constexpr int EP = Piece<T>::N;
@@ -349,9 +365,9 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dq_grid(LbDev a) {
     const int qy = (qi >> 2) & 3, qx = qi & 3;
     const int qz = 2 * nb + (qi >> 4);
 
-    const int gz = Z0 + qz, gy = Y0 + 4 * wy + qy, gx = X0 + 4 * wx + qx;
+    const int gz = Z0 + qz, gy = real_y<STRIPS>(gz, Y0 + 4 * wy + qy), gx = X0 + 4 * wx + qx;
     const bool qok = gz < a.Z && gy < a.Y && gx < a.X;
-    const int64_t qrow = qok ? packed_row(a, gz, gy, gx) : 0;
+    const int64_t qrow = qok ? packed_row<STRIPS>(a, gz, gy, gx) : 0;
     const int64_t qidx = (int64_t)bh * a.N + qrow;
     typename C::Frag qf[C::NT], df[C::NT];
     row_frags<C>(tp<T>(a.q) + b * a.qsb + h * a.qsh + qrow * a.qsn, qok, g, qf);
@@ -369,19 +385,20 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dq_grid(LbDev a) {
 
     const T* KL = tp<T>(a.kl) + b * a.ksb + kvh * a.ksh;
     const T* VL = tp<T>(a.vl) + b * a.vsb + kvh * a.vsh;
-    const uint32_t kmask[2] = {chunk_mask<C>(a, 0, g, qy, qx, Y0 + 4 * wy, X0 + 4 * wx),
-                               chunk_mask<C>(a, 1, g, qy, qx, Y0 + 4 * wy, X0 + 4 * wx)};
+    uint32_t kmask[2];
+    chunk_masks<C>(a, g, qy, qx, Y0 + 4 * wy, X0 + 4 * wx, kmask);  // strips: set again per plane
     zero_pad_rows<C>(Kt, TPS);
     const int planes = 4 + 2 * a.rz;
     for (int hz = 0; hz < planes; ++hz) {
         const int pz = Z0 - a.rz + hz;
         if (hz) __syncthreads();
-        stage_plane<C, true, false>(a, KL, a.ksn, VL, a.vsn, pz, Y0, X0, Kr, Vr, Kt, nullptr, TPS);
+        stage_plane<C, true, false, STRIPS>(a, KL, a.ksn, VL, a.vsn, pz, Y0, X0, Kr, Vr, Kt, nullptr, TPS);
         __syncthreads();
         if ((unsigned)pz >= (unsigned)a.Z) continue;
         // Column block nb holds query planes 2nb and 2nb + 1.
         if (hz < 2 * nb || hz > 2 * nb + 1 + 2 * a.rz) continue;
         const bool zok = (unsigned)(hz - qz) <= (unsigned)(2 * a.rz) && live;
+        if (STRIPS) chunk_masks<C>(a, g, qy, qx, real_y<STRIPS>(pz, 4 * wy), X0 + 4 * wx, kmask);
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             if (4 * c >= 4 + 2 * a.ry) continue;
@@ -406,7 +423,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dq_grid(LbDev a) {
 }
 
 // k_local_dq_grid with the planes copied by the LDS DMA (kBwdPlaneDma types).
-template <typename T, int D>
+template <typename T, int D, bool STRIPS>
 __global__ __launch_bounds__(64 * kWaves) void k_local_dq_grid_dma(LbDev a) {
     typedef Cfg<T, D> C;
     typedef BwdPlaneDma<C, false> PD;
@@ -425,14 +442,14 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dq_grid_dma(LbDev a) {
     const int planes = 4 + 2 * a.rz;
     const T* KL = tp<T>(a.kl) + b * a.ksb + kvh * a.ksh;
     const T* VL = tp<T>(a.vl) + b * a.vsb + kvh * a.vsh;
-    PD::fill_rows(a, Z0, Y0, X0, planes, rowtab);
+    PD::template fill_rows<STRIPS>(a, Z0, Y0, X0, planes, rowtab);
     __syncthreads();
     const int uwave = __builtin_amdgcn_readfirstlane(wave);
     if ((unsigned)(Z0 - a.rz) < (unsigned)a.Z) PD::copy(KL, a.ksn, VL, a.vsn, rowtab, smem, uwave, lane);
 
-    const int gz = Z0 + qz, gy = Y0 + 4 * wy + qy, gx = X0 + 4 * wx + qx;
+    const int gz = Z0 + qz, gy = real_y<STRIPS>(gz, Y0 + 4 * wy + qy), gx = X0 + 4 * wx + qx;
     const bool qok = gz < a.Z && gy < a.Y && gx < a.X;
-    const int64_t qrow = qok ? packed_row(a, gz, gy, gx) : 0;
+    const int64_t qrow = qok ? packed_row<STRIPS>(a, gz, gy, gx) : 0;
     const int64_t qidx = (int64_t)bh * a.N + qrow;
     typename C::Frag qf[C::NT], df[C::NT];
     row_frags<C>(tp<T>(a.q) + b * a.qsb + h * a.qsh + qrow * a.qsn, qok, g, qf);
@@ -447,8 +464,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dq_grid_dma(LbDev a) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[mb][r] = 0.f;
     int shift = 0;
-    const uint32_t kmask[2] = {chunk_mask<C>(a, 0, g, qy, qx, Y0 + 4 * wy, X0 + 4 * wx),
-                               chunk_mask<C>(a, 1, g, qy, qx, Y0 + 4 * wy, X0 + 4 * wx)};
+    uint32_t kmask[2];
+    chunk_masks<C>(a, g, qy, qx, Y0 + 4 * wy, X0 + 4 * wx, kmask);  // strips: set again per plane
     for (int hz = 0; hz < planes; ++hz) {
         const int pz = Z0 - a.rz + hz;
         // Plane hz has landed, and every wave is done with plane hz - 1,
@@ -464,6 +481,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dq_grid_dma(LbDev a) {
         const T* Kb = reinterpret_cast<const T*>(smem + (hz & 1) * PD::BUF);
         const T* Vb = reinterpret_cast<const T*>(smem + (hz & 1) * PD::BUF + PD::REGION);
         const bool zok = (unsigned)(hz - qz) <= (unsigned)(2 * a.rz) && live;
+        if (STRIPS) chunk_masks<C>(a, g, qy, qx, real_y<STRIPS>(pz, 4 * wy), X0 + 4 * wx, kmask);
 #pragma unroll
         for (int c = 0; c < 2; ++c) {
             if (4 * c >= 4 + 2 * a.ry) continue;
@@ -490,10 +508,11 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dq_grid_dma(LbDev a) {
 // lse (log2 units; +inf where the position has no gradient: outside the grid
 // or the halo, or an all-masked row) and Delta of halo position p of plane
 // pz for query head plane bh; rows: that plane's row table.
+template <bool STRIPS>
 __device__ __forceinline__ void plane_side(const LbDev& a, int64_t bh, int pz, int Y0, int X0, int p,
                                            const int* rows, float& l2, float& dl) {
     const int py = p / kPlane, px = p - py * kPlane;
-    const int qy = Y0 - a.ry + py, qx = X0 - a.rx + px;
+    const int qy = real_y<STRIPS>(pz, Y0 - a.ry + py), qx = X0 - a.rx + px;
     const bool in = (unsigned)pz < (unsigned)a.Z && (unsigned)qy < (unsigned)a.Y && (unsigned)qx < (unsigned)a.X &&
                     py < 8 + 2 * a.ry && px < 8 + 2 * a.rx;
     l2 = INFINITY, dl = 0.f;
@@ -505,7 +524,7 @@ __device__ __forceinline__ void plane_side(const LbDev& a, int64_t bh, int pz, i
     }
 }
 
-template <typename T, int D>
+template <typename T, int D, bool STRIPS>
 __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid(LbDev a) {
     typedef Cfg<T, D> C;
     constexpr int EP = Piece<T>::N;
@@ -528,9 +547,9 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid(LbDev a) {
     const int ky = (ki >> 2) & 3, kx = ki & 3;
     const int kz = 2 * nb + (ki >> 4);
 
-    const int gz = Z0 + kz, gy = Y0 + 4 * wy + ky, gx = X0 + 4 * wx + kx;
+    const int gz = Z0 + kz, gy = real_y<STRIPS>(gz, Y0 + 4 * wy + ky), gx = X0 + 4 * wx + kx;
     const bool kok = gz < a.Z && gy < a.Y && gx < a.X;
-    const int64_t krow = kok ? packed_row(a, gz, gy, gx) : 0;
+    const int64_t krow = kok ? packed_row<STRIPS>(a, gz, gy, gx) : 0;
     typename C::Frag kf[C::NT], vf[C::NT];
     row_frags<C>(tp<T>(a.kl) + b * a.ksb + kvh * a.ksh + krow * a.ksn, kok, g, kf);
     row_frags<C>(tp<T>(a.vl) + b * a.vsb + kvh * a.vsh + krow * a.vsn, kok, g, vf);
@@ -541,8 +560,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid(LbDev a) {
         for (int r = 0; r < 16; ++r) acck[mb][r] = accv[mb][r] = 0.f;
     int shift = 0;
 
-    const uint32_t qmask[2] = {chunk_mask<C>(a, 0, g, ky, kx, Y0 + 4 * wy, X0 + 4 * wx),
-                               chunk_mask<C>(a, 1, g, ky, kx, Y0 + 4 * wy, X0 + 4 * wx)};
+    uint32_t qmask[2];
+    chunk_masks<C>(a, g, ky, kx, Y0 + 4 * wy, X0 + 4 * wx, qmask);  // strips: set again per plane
     zero_pad_rows<C>(Qt, TPS);
     zero_pad_rows<C>(Dt, TPS);
     const int planes = 4 + 2 * a.rz;
@@ -554,15 +573,15 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid(LbDev a) {
         for (int hz = 0; hz < planes; ++hz) {
             const int pz = Z0 - a.rz + hz;
             __syncthreads();
-            stage_plane<C, true, true>(a, Q, a.qsn, DO, D, pz, Y0, X0, Qr, Dr, Qt, Dt, TPS);
+            stage_plane<C, true, true, STRIPS>(a, Q, a.qsn, DO, D, pz, Y0, X0, Qr, Dr, Qt, Dt, TPS);
             for (int p = tid; p < kPlaneKeys; p += 64 * kWaves) {
                 const int py = p / kPlane, px = p - py * kPlane;
-                const int qy = Y0 - a.ry + py, qx = X0 - a.rx + px;
+                const int qy = real_y<STRIPS>(pz, Y0 - a.ry + py), qx = X0 - a.rx + px;
                 const bool in = (unsigned)pz < (unsigned)a.Z && (unsigned)qy < (unsigned)a.Y &&
                                 (unsigned)qx < (unsigned)a.X && py < 8 + 2 * a.ry && px < 8 + 2 * a.rx;
                 float l2 = INFINITY, dl = 0.f;
                 if (in) {
-                    const int64_t qidx = bh * a.N + packed_row(a, pz, qy, qx);
+                    const int64_t qidx = bh * a.N + packed_row<STRIPS>(a, pz, qy, qx);
                     const float l = a.lse[qidx];
                     l2 = l == -INFINITY ? INFINITY : l * kLog2e;  // all-masked rows carry no gradient
                     dl = a.delta[qidx];
@@ -574,6 +593,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid(LbDev a) {
             if ((unsigned)pz >= (unsigned)a.Z) continue;
             if (hz < 2 * nb || hz > 2 * nb + 1 + 2 * a.rz) continue;
             const bool zok = (unsigned)(hz - kz) <= (unsigned)(2 * a.rz);
+            if (STRIPS) chunk_masks<C>(a, g, ky, kx, real_y<STRIPS>(pz, 4 * wy), X0 + 4 * wx, qmask);
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
                 if (4 * c >= 4 + 2 * a.ry) continue;
@@ -609,7 +629,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid(LbDev a) {
 // The (query head, plane) steps of the kv group run as one sequence; a
 // step's lse / Delta are loaded into registers while the step before it is
 // processed and written into its buffer after that.
-template <typename T, int D>
+template <typename T, int D, bool STRIPS>
 __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid_dma(LbDev a) {
     typedef Cfg<T, D> C;
     typedef BwdPlaneDma<C, true> PD;
@@ -627,7 +647,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid_dma(LbDev a) {
     const int kz = 2 * nb + (ki >> 4);
     const int planes = 4 + 2 * a.rz;
     const int steps = rep * planes;
-    PD::fill_rows(a, Z0, Y0, X0, planes, rowtab);
+    PD::template fill_rows<STRIPS>(a, Z0, Y0, X0, planes, rowtab);
     __syncthreads();
     const int uwave = __builtin_amdgcn_readfirstlane(wave);
     const int h0 = kvh * rep;
@@ -643,7 +663,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid_dma(LbDev a) {
         const int hh = i / planes, hz = i - hh * planes;
         l2 = INFINITY, dl = 0.f;
         if (tid < kPlaneKeys)
-            plane_side(a, (int64_t)b * a.H + h0 + hh, Z0 - a.rz + hz, Y0, X0, tid, rowtab + hz * kPlaneKeys, l2, dl);
+            plane_side<STRIPS>(a, (int64_t)b * a.H + h0 + hh, Z0 - a.rz + hz, Y0, X0, tid, rowtab + hz * kPlaneKeys, l2, dl);
     };
     auto side_store = [&](int i, float l2, float dl) __attribute__((always_inline)) {
         if (tid < kPlaneKeys) {
@@ -659,9 +679,9 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid_dma(LbDev a) {
         side_store(0, l2, dl);
     }
 
-    const int gz = Z0 + kz, gy = Y0 + 4 * wy + ky, gx = X0 + 4 * wx + kx;
+    const int gz = Z0 + kz, gy = real_y<STRIPS>(gz, Y0 + 4 * wy + ky), gx = X0 + 4 * wx + kx;
     const bool kok = gz < a.Z && gy < a.Y && gx < a.X;
-    const int64_t krow = kok ? packed_row(a, gz, gy, gx) : 0;
+    const int64_t krow = kok ? packed_row<STRIPS>(a, gz, gy, gx) : 0;
     typename C::Frag kf[C::NT], vf[C::NT];
     row_frags<C>(tp<T>(a.kl) + b * a.ksb + kvh * a.ksh + krow * a.ksn, kok, g, kf);
     row_frags<C>(tp<T>(a.vl) + b * a.vsb + kvh * a.vsh + krow * a.vsn, kok, g, vf);
@@ -671,8 +691,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid_dma(LbDev a) {
 #pragma unroll
         for (int r = 0; r < 16; ++r) acck[mb][r] = accv[mb][r] = 0.f;
     int shift = 0;
-    const uint32_t qmask[2] = {chunk_mask<C>(a, 0, g, ky, kx, Y0 + 4 * wy, X0 + 4 * wx),
-                               chunk_mask<C>(a, 1, g, ky, kx, Y0 + 4 * wy, X0 + 4 * wx)};
+    uint32_t qmask[2];
+    chunk_masks<C>(a, g, ky, kx, Y0 + 4 * wy, X0 + 4 * wx, qmask);  // strips: set again per plane
     for (int i = 0; i < steps; ++i) {
         const int hz = i % planes;
         const int pz = Z0 - a.rz + hz;
@@ -693,6 +713,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid_dma(LbDev a) {
             const float* lse2s = reinterpret_cast<const float*>(buf + 2 * PD::REGION);
             const float* dlts = lse2s + kPlaneKeys;
             const bool zok = (unsigned)(hz - kz) <= (unsigned)(2 * a.rz);
+            if (STRIPS) chunk_masks<C>(a, g, ky, kx, real_y<STRIPS>(pz, 4 * wy), X0 + 4 * wx, qmask);
 #pragma unroll
             for (int c = 0; c < 2; ++c) {
                 if (4 * c >= 4 + 2 * a.ry) continue;
@@ -738,30 +759,30 @@ size_t lds_dkv_grid() {
            (size_t)2 * kPlaneKeys * sizeof(float);
 }
 
-template <typename T, int D>
+template <typename T, int D, bool STRIPS>
 int launch_t(const LbDev& d, hipStream_t s) {
     typedef Cfg<T, D> C;
     const int bricks = (int)(cdiv(d.Z, 4) * d.bricks_y * d.bricks_x);
     if constexpr (kBwdPlaneDma<C>) {
         constexpr size_t l1 = BwdPlaneDma<C, false>::BYTES, l2 = BwdPlaneDma<C, true>::BYTES;
         static_assert(l1 <= 160 * 1024 && l2 <= 160 * 1024, "plane buffers within LDS");
-        k_local_dq_grid_dma<T, D><<<dim3(bricks, d.B * d.H), 64 * kWaves, l1, s>>>(d);
-        k_local_dkv_grid_dma<T, D><<<dim3(bricks, d.B * d.G), 64 * kWaves, l2, s>>>(d);
+        k_local_dq_grid_dma<T, D, STRIPS><<<dim3(bricks, d.B * d.H), 64 * kWaves, l1, s>>>(d);
+        k_local_dkv_grid_dma<T, D, STRIPS><<<dim3(bricks, d.B * d.G), 64 * kWaves, l2, s>>>(d);
     } else {
         const size_t l1 = lds_dq_grid<T, D>(), l2 = lds_dkv_grid<T, D>();
         if (l1 > 160 * 1024 || l2 > 160 * 1024) return fail(P3D_EUNSUPPORTED, "p3d_local_bwd_grid: planes exceed LDS");
-        k_local_dq_grid<T, D><<<dim3(bricks, d.B * d.H), 64 * kWaves, l1, s>>>(d);
-        k_local_dkv_grid<T, D><<<dim3(bricks, d.B * d.G), 64 * kWaves, l2, s>>>(d);
+        k_local_dq_grid<T, D, STRIPS><<<dim3(bricks, d.B * d.H), 64 * kWaves, l1, s>>>(d);
+        k_local_dkv_grid<T, D, STRIPS><<<dim3(bricks, d.B * d.G), 64 * kWaves, l2, s>>>(d);
     }
     return P3D_OK;
 }
 
 template <int D>
-int launch_d(const LbDev& d, int dtype, hipStream_t s) {
+int launch_d(const LbDev& d, int dtype, bool strips, hipStream_t s) {
     switch (dtype) {
-        case P3D_F32: return launch_t<float, D>(d, s);
-        case P3D_F16: return launch_t<_Float16, D>(d, s);
-        default: return launch_t<__bf16, D>(d, s);
+        case P3D_F32: return strips ? launch_t<float, D, true>(d, s) : launch_t<float, D, false>(d, s);
+        case P3D_F16: return strips ? launch_t<_Float16, D, true>(d, s) : launch_t<_Float16, D, false>(d, s);
+        default: return strips ? launch_t<__bf16, D, true>(d, s) : launch_t<__bf16, D, false>(d, s);
     }
 }
 
@@ -793,6 +814,11 @@ extern "C" int p3d_local_bwd_grid(const p3d_bwd_args* args, const int32_t grid[3
     d.Z = grid[0], d.Y = grid[1], d.X = grid[2];
     d.rz = radius[0], d.ry = radius[1], d.rx = radius[2];
     d.bricks_y = (int)cdiv(d.Y, 8), d.bricks_x = (int)cdiv(d.X, 8);
+    // Strips on a one-plane grid with more bricks than CUs (one workgroup each).
+    const bool strips = d.Z == 1 && (int64_t)d.bricks_y * d.bricks_x * d.B * d.G > 256;
+    if (strips) {
+        d.Z = d.bricks_y, d.bricks_y = 1, d.rz = 0;
+    }
     d.q = (const char*)x.q.data, d.qsb = x.q.sb, d.qsh = x.q.sh, d.qsn = x.q.sn;
     d.kl = (const char*)x.kl.data, d.ksb = x.kl.sb, d.ksh = x.kl.sh, d.ksn = x.kl.sn;
     d.vl = (const char*)x.vl.data, d.vsb = x.vl.sb, d.vsh = x.vl.sh, d.vsn = x.vl.sn;
@@ -806,11 +832,11 @@ extern "C" int p3d_local_bwd_grid(const p3d_bwd_args* args, const int32_t grid[3
     hipStream_t s = as_stream(stream);
     int rc = P3D_OK;
     switch (x.head_dim) {
-        case 16: rc = launch_d<16>(d, x.dtype, s); break;
-        case 32: rc = launch_d<32>(d, x.dtype, s); break;
-        case 48: rc = launch_d<48>(d, x.dtype, s); break;
-        case 64: rc = launch_d<64>(d, x.dtype, s); break;
-        default: rc = launch_d<128>(d, x.dtype, s); break;
+        case 16: rc = launch_d<16>(d, x.dtype, strips, s); break;
+        case 32: rc = launch_d<32>(d, x.dtype, strips, s); break;
+        case 48: rc = launch_d<48>(d, x.dtype, strips, s); break;
+        case 64: rc = launch_d<64>(d, x.dtype, strips, s); break;
+        default: rc = launch_d<128>(d, x.dtype, strips, s); break;
     }
     if (rc != P3D_OK) return rc;
     return check_launch("p3d_local_bwd_grid");
