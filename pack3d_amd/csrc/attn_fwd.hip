@@ -57,7 +57,7 @@ struct AttnDev {
 // brick in y), each with its own halo plane, whose y halo reaches into the
 // neighbouring strips.  A brick then holds 256 queries instead of 64, so a
 // quarter of the workgroups do the summary sweep and the set-up: 128 x 128
-// slices with 8 heads of 64, 150 us with 4 x 8 x 8 bricks, FLAT_FWD us in strips.
+// slices with 8 heads of 64, 150 us with 4 x 8 x 8 bricks, 133 us in strips.
 // (STRIPS is a template argument: as a run-time flag it cost the bricks registers.)
 template <bool STRIPS>
 __device__ __forceinline__ int real_y(int gz, int gy) { return STRIPS ? 8 * gz + gy : gy; }
