@@ -173,6 +173,13 @@ struct StageDma {
     }
 };
 
+// Types whose key and value fragments of a tile do not fit in registers
+// together load the values once the scores have consumed the keys (held apart
+// by a scheduling barrier: left to itself the scheduler hoists the loads and
+// spills).
+template <typename C>
+constexpr bool kLateValues = C::D >= 128 || sizeof(typename C::T_) == 4;
+
 // One summary stage (two 32-key tiles) on this wave's two column blocks.
 template <typename C, bool BOUND>
 __device__ __forceinline__ void global_stage(const AttnDev& a, int base, const typename C::T_* Ks,
@@ -187,10 +194,14 @@ __device__ __forceinline__ void global_stage(const AttnDev& a, int base, const t
         if (first >= a.M) break;
         typename C::Frag kf[C::NT], vf[C::MB * C::KSTEPS];
         load_kfrags<C>(Ks + (32 * tt + kperm<C::E, C::KS>(qi)) * C::KSTR + C::E * g, kf);
-        load_vfrags<C, true>(Vs, vstride, 32 * tt, lane, vf);
+        if constexpr (!kLateValues<C>) load_vfrags<C, true>(Vs, vstride, 32 * tt, lane, vf);
         f32x16 s[2];
 #pragma unroll
         for (int nb = 0; nb < 2; ++nb) s[nb] = BOUND ? score_tile<C>(kf, qf[nb], negm[nb]) : score_tile<C>(kf, qf[nb]);
+        if constexpr (kLateValues<C>) {
+            __builtin_amdgcn_sched_barrier(0);
+            load_vfrags<C, true>(Vs, vstride, 32 * tt, lane, vf);
+        }
         if (first + 32 > a.M) {
 #pragma unroll
             for (int nb = 0; nb < 2; ++nb)
@@ -853,6 +864,15 @@ constexpr size_t grid_lds_bytes() {
     }
 }
 
+// Workgroups per CU that the register budget is for (one wave per SIMD each).
+// Where the LDS holds only one workgroup (head_dim 128, and fp32 from head_dim
+// 64) a cap for two bought nothing and spilled 88 to 5,764 registers: head_dim
+// 128 in bf16, 16,384 tokens of 4 heads, 181 us with 350 spilled, 115 us with 14.
+// fp32 head_dim 48 keeps two (one spilled register): 297 us against 368 with one
+// workgroup of unspilled waves (18,711 tokens of 4 heads).
+template <typename C, int PW>
+constexpr int kGridGroups = 2 * grid_lds_bytes<C, PW>() <= 160 * 1024 ? 2 : 1;
+
 // Scores and products of one staged plane on this wave's two column blocks
 // (the chunks of its 8 x 8 key footprint).  Kb holds the plane's rotated K
 // rows, PW keys per plane row; vfrag(c, mb, ks) returns the value fragment
@@ -867,10 +887,13 @@ __device__ __forceinline__ void plane_chunks(const AttnDev& a, const typename C:
         const int kap = kperm<C::E, C::KS>(qi);
         typename C::Frag kf[C::NT], vf[C::MB * C::KSTEPS];
         load_kfrags<C>(Kb + ((4 * wy + 4 * c + kap / 8) * PW + 4 * wx + kap % 8) * C::KSTR + C::E * g, kf);
+        auto load_values = [&]() __attribute__((always_inline)) {
 #pragma unroll
-        for (int mb = 0; mb < C::MB; ++mb)
+            for (int mb = 0; mb < C::MB; ++mb)
 #pragma unroll
-            for (int ks = 0; ks < C::KSTEPS; ++ks) vf[mb * C::KSTEPS + ks] = vfrag(c, mb, ks);
+                for (int ks = 0; ks < C::KSTEPS; ++ks) vf[mb * C::KSTEPS + ks] = vfrag(c, mb, ks);
+        };
+        if constexpr (!kLateValues<C>) load_values();
         f32x16 bias;
 #pragma unroll
         for (int r = 0; r < 16; ++r) bias[r] = (kmask[c] >> r) & 1 ? 0.f : -INFINITY;
@@ -888,13 +911,17 @@ __device__ __forceinline__ void plane_chunks(const AttnDev& a, const typename C:
             }
             float p[16];
             soft_probs<C>(st[nb], s, a.scale_log2, p);
+            if constexpr (kLateValues<C>) {
+                __builtin_amdgcn_sched_barrier(0);
+                load_values();
+            }
             soft_accumulate<C>(st[nb], p, vf);
         }
     }
 }
 
 template <typename T, int D, int PW, bool STRIPS>
-__global__ __launch_bounds__(64 * kWaves, 2) void k_attn_grid(AttnDev a) {
+__global__ __launch_bounds__(64 * kWaves, (kGridGroups<Cfg<T, D>, PW>)) void k_attn_grid(AttnDev a) {
     typedef Cfg<T, D> C;
     constexpr int EP = Piece<T>::N;
     constexpr int VPS = kPlaneKeys + EP;  // plane V row stride (elements)
@@ -1036,8 +1063,15 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_attn_grid(AttnDev a) {
     }
 }
 
+template <typename C>
+constexpr size_t rows_lds_bytes() {
+    constexpr int ep = Piece<typename C::T_>::N;
+    return (kPiped<C> ? 3 : 2) * ((size_t)64 * C::KSTR + (size_t)32 * C::MB * (64 + ep)) * sizeof(typename C::T_);
+}
+
 template <typename T, int D>
-__global__ __launch_bounds__(64 * kRowsWaves, 2) void k_attn_rows(AttnDev a) {
+__global__ __launch_bounds__(64 * kRowsWaves, (2 * rows_lds_bytes<Cfg<T, D>>() <= 160 * 1024 ? 2 : 1))
+void k_attn_rows(AttnDev a) {
     typedef Cfg<T, D> C;
     extern __shared__ __align__(16) unsigned char smem[];
     T* lds = reinterpret_cast<T*>(smem);
@@ -1111,13 +1145,6 @@ size_t lds_grid() {
     return grid_lds_bytes<C, PW>();
 }
 
-template <typename T, int D>
-size_t lds_rows() {
-    typedef Cfg<T, D> C;
-    constexpr int ep = Piece<T>::N;
-    return (kPiped<C> ? 3 : 2) * ((size_t)64 * C::KSTR + (size_t)32 * C::MB * (64 + ep)) * sizeof(T);
-}
-
 template <typename T, int D, int PW>
 void launch_grid_t(const AttnDev& d, bool strips, dim3 grid, hipStream_t s) {
     if (strips)
@@ -1153,9 +1180,9 @@ int launch_grid(const AttnDev& d, int dtype, bool strips, dim3 grid, hipStream_t
 template <int D>
 int launch_rows(const AttnDev& d, int dtype, dim3 grid, hipStream_t s) {
     switch (dtype) {
-        case P3D_F32: k_attn_rows<float, D><<<grid, 64 * kRowsWaves, lds_rows<float, D>(), s>>>(d); break;
-        case P3D_F16: k_attn_rows<_Float16, D><<<grid, 64 * kRowsWaves, lds_rows<_Float16, D>(), s>>>(d); break;
-        default: k_attn_rows<__bf16, D><<<grid, 64 * kRowsWaves, lds_rows<__bf16, D>(), s>>>(d); break;
+        case P3D_F32: k_attn_rows<float, D><<<grid, 64 * kRowsWaves, rows_lds_bytes<Cfg<float, D>>(), s>>>(d); break;
+        case P3D_F16: k_attn_rows<_Float16, D><<<grid, 64 * kRowsWaves, rows_lds_bytes<Cfg<_Float16, D>>(), s>>>(d); break;
+        default: k_attn_rows<__bf16, D><<<grid, 64 * kRowsWaves, rows_lds_bytes<Cfg<__bf16, D>>(), s>>>(d); break;
     }
     return check_launch("p3d_attn_fwd_rows");
 }

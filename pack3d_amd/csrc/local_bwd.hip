@@ -189,20 +189,21 @@ __device__ __forceinline__ void row_frags(const typename C::T_* row, bool valid,
     }
 }
 
-// A-operand fragments of a transposed plane buffer for chunk c: row 32 mb + qi
+// A-operand fragment of a transposed plane buffer for chunk c: row 32 mb + qi
 // (channel), contraction index ks * KS + E * g + j = chunk position (natural).
+template <typename C>
+__device__ __forceinline__ typename C::Frag trans_frag(const typename C::T_* Tb, int tps, int wy, int wx, int c, int mb,
+                                                       int ks, int lane) {
+    const int g = lane >> 5, qi = lane & 31;
+    return frag_load8<typename C::T_>(Tb + (32 * mb + qi) * tps + chunk_pos(wy, wx, c, ks * C::KS + C::E * g));
+}
 template <typename C>
 __device__ __forceinline__ void trans_frags(const typename C::T_* Tb, int tps, int wy, int wx, int c, int lane,
                                             typename C::Frag* f) {
-    const int g = lane >> 5, qi = lane & 31;
 #pragma unroll
     for (int mb = 0; mb < C::MB; ++mb)
 #pragma unroll
-        for (int ks = 0; ks < C::KSTEPS; ++ks) {
-            const int k0 = ks * C::KS + C::E * g;
-            f[mb * C::KSTEPS + ks] =
-                frag_load8<typename C::T_>(Tb + (32 * mb + qi) * tps + chunk_pos(wy, wx, c, k0));
-        }
+        for (int ks = 0; ks < C::KSTEPS; ++ks) f[mb * C::KSTEPS + ks] = trans_frag<C>(Tb, tps, wy, wx, c, mb, ks, lane);
 }
 
 // dQ^T += K^T dS^T for chunk c of one plane: kf / vf are the chunk's K and V
@@ -230,19 +231,66 @@ __device__ __forceinline__ void dq_chunk(const typename C::Frag* kf, const typen
     }
 }
 
-// dK^T += q^T dS and dV^T += dO^T P for chunk c of one plane: qa / da are the
-// chunk's q and dO row fragments (lane = query of the tile), qt / dt the
-// transposed fragments (A operands); lse2s / dlts hold the plane's lse (log2
-// units, +inf where a position has no gradient) and Delta.
+// Which of dK and dV a workgroup of the dK/dV kernel computes.  At 16-bit
+// head_dim 128 the two accumulators (128 registers) beside the key and value
+// fragments (64) spill, so there each goes to workgroups of its own: the scores
+// are computed twice (20 against 16 MFMA groups per chunk), nothing spills, and
+// twice as many workgroups run.  16,384 tokens of 2 kv heads: 353 -> 115 us.
+constexpr int kDK = 1, kDV = 2;
+
+// Types whose resident key fragments and accumulators leave no room for a
+// chunk's four sets of query fragments read them in order of use: the rows a
+// few contraction steps at a time, the transposes one step at a time once the
+// scores are done, each group held apart by a scheduling barrier (left to
+// itself the scheduler hoists the loads and spills 94 registers at fp32
+// head_dim 48, 512 -> 253 us for 18,711 tokens of 4 heads, and 217 at 16-bit
+// head_dim 128).
 template <typename C>
-__device__ __forceinline__ void dkv_chunk(const typename C::Frag* qa, const typename C::Frag* da,
-                                          const typename C::Frag* qt, const typename C::Frag* dt,
+constexpr bool kLateFrags = C::D >= 128 || sizeof(typename C::T_) == 4;
+
+// dK^T += q^T dS and dV^T += dO^T P for chunk c of one plane: qrow / drow are
+// the lane's q and dO rows of the chunk (lane = query of the tile, offset by
+// E g), qtf(mb, ks) / dtf(mb, ks) give the transposed fragments (A operands);
+// lse2s / dlts hold the plane's lse (log2 units, +inf where a position has no
+// gradient) and Delta.
+template <typename C, int PARTS = kDK | kDV, typename QT, typename DT>
+__device__ __forceinline__ void dkv_chunk(const typename C::T_* qrow, const typename C::T_* drow, QT qtf, DT dtf,
                                           const typename C::Frag* kf, const typename C::Frag* vf, bool zok,
                                           uint32_t qmask, float scale_log2, const float* lse2s, const float* dlts,
                                           int wy, int wx, int c, int g, int& shift, f32x16* acck, f32x16* accv) {
     typedef typename C::T_ T;
-    const f32x16 s = score_tile<C>(qa, kf);
-    const f32x16 dp = score_tile<C>(da, vf);
+    typedef typename C::Frag Frag;
+    constexpr bool LATE = kLateFrags<C>;
+    Frag qt[LATE ? 1 : C::MB * C::KSTEPS], dt[LATE ? 1 : C::MB * C::KSTEPS];
+    f32x16 s, dp;
+    if constexpr (!LATE) {
+        Frag qa[C::NT], da[C::NT];
+        load_kfrags<C>(qrow, qa);
+        load_kfrags<C>(drow, da);
+#pragma unroll
+        for (int mb = 0; mb < C::MB; ++mb)
+#pragma unroll
+            for (int ks = 0; ks < C::KSTEPS; ++ks) {
+                qt[mb * C::KSTEPS + ks] = qtf(mb, ks);
+                dt[mb * C::KSTEPS + ks] = dtf(mb, ks);
+            }
+        s = score_tile<C>(qa, kf);
+        dp = score_tile<C>(da, vf);
+    } else {
+#pragma unroll
+        for (int r = 0; r < 16; ++r) s[r] = dp[r] = 0.f;
+        constexpr int STEP = C::E == 8 ? 2 : 12;  // contraction steps per group
+        static_assert(C::NT % STEP == 0 || C::E == 1, "whole groups");
+#pragma unroll
+        for (int t0 = 0; t0 < C::NT; t0 += STEP) {
+#pragma unroll
+            for (int t = t0; t < t0 + STEP && t < C::NT; ++t) {
+                s = C::M::mfma(frag_load16<T>(qrow + t * C::KS), kf[t], s);
+                if constexpr (PARTS & kDK) dp = C::M::mfma(frag_load16<T>(drow + t * C::KS), vf[t], dp);
+            }
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
     float p[16], ds[16];
 #pragma unroll
     for (int r = 0; r < 16; ++r) {
@@ -251,15 +299,20 @@ __device__ __forceinline__ void dkv_chunk(const typename C::Frag* qa, const type
         p[r] = ok ? __builtin_amdgcn_exp2f(fmaf(s[r], scale_log2, -lse2s[pos])) : 0.f;
         ds[r] = p[r] * (dp[r] - dlts[pos]);
     }
-    fit_fp16<C>(ds, shift, acck);
+    if constexpr (PARTS & kDK) fit_fp16<C>(ds, shift, acck);
 #pragma unroll
     for (int ks = 0; ks < C::KSTEPS; ++ks) {
-        const typename C::Frag dsf = frag_from_p<T>(ds, ks);
-        const typename C::Frag pf = frag_from_p<T>(p, ks);
+        const Frag dsf = frag_from_p<T>(ds, ks);
+        const Frag pf = frag_from_p<T>(p, ks);
+        if constexpr (LATE && C::E == 8) __builtin_amdgcn_sched_barrier(0);
+        if constexpr (LATE && C::E == 1)
+            if (ks % 8 == 0) __builtin_amdgcn_sched_barrier(0);
 #pragma unroll
         for (int mb = 0; mb < C::MB; ++mb) {
-            acck[mb] = C::M::mfma(qt[mb * C::KSTEPS + ks], dsf, acck[mb]);
-            accv[mb] = C::M::mfma(dt[mb * C::KSTEPS + ks], pf, accv[mb]);
+            if constexpr (PARTS & kDK)
+                acck[mb] = C::M::mfma(LATE ? qtf(mb, ks) : qt[LATE ? 0 : mb * C::KSTEPS + ks], dsf, acck[mb]);
+            if constexpr (PARTS & kDV)
+                accv[mb] = C::M::mfma(LATE ? dtf(mb, ks) : dt[LATE ? 0 : mb * C::KSTEPS + ks], pf, accv[mb]);
         }
     }
 }
@@ -524,8 +577,8 @@ __device__ __forceinline__ void plane_side(const LbDev& a, int64_t bh, int pz, i
     }
 }
 
-template <typename T, int D, bool STRIPS>
-__global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid(LbDev a) {
+template <typename T, int D, bool STRIPS, int PARTS>
+__device__ __forceinline__ void local_dkv(const LbDev& a) {
     typedef Cfg<T, D> C;
     constexpr int EP = Piece<T>::N;
     constexpr int TPS = kPlaneKeys + EP;
@@ -573,7 +626,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid(LbDev a) {
         for (int hz = 0; hz < planes; ++hz) {
             const int pz = Z0 - a.rz + hz;
             __syncthreads();
-            stage_plane<C, true, true, STRIPS>(a, Q, a.qsn, DO, D, pz, Y0, X0, Qr, Dr, Qt, Dt, TPS);
+            stage_plane<C, (PARTS & kDK) != 0, (PARTS & kDV) != 0, STRIPS>(a, Q, a.qsn, DO, D, pz, Y0, X0, Qr, Dr, Qt, Dt,
+                                                                            TPS);
             for (int p = tid; p < kPlaneKeys; p += 64 * kWaves) {
                 const int py = p / kPlane, px = p - py * kPlane;
                 const int qy = real_y<STRIPS>(pz, Y0 - a.ry + py), qx = X0 - a.rx + px;
@@ -598,12 +652,10 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid(LbDev a) {
             for (int c = 0; c < 2; ++c) {
                 if (4 * c >= 4 + 2 * a.ry) continue;
                 const int kap = kperm<C::E, C::KS>(ki);
-                typename C::Frag qa[C::NT], da[C::NT], qt[C::MB * C::KSTEPS], dt[C::MB * C::KSTEPS];
-                load_kfrags<C>(Qr + chunk_pos(wy, wx, c, kap) * C::KSTR + C::E * g, qa);
-                load_kfrags<C>(Dr + chunk_pos(wy, wx, c, kap) * C::KSTR + C::E * g, da);
-                trans_frags<C>(Qt, TPS, wy, wx, c, lane, qt);
-                trans_frags<C>(Dt, TPS, wy, wx, c, lane, dt);
-                dkv_chunk<C>(qa, da, qt, dt, kf, vf, zok, qmask[c], a.scale_log2, lse2s, dlts, wy, wx, c, g, shift,
+                dkv_chunk<C, PARTS>(Qr + chunk_pos(wy, wx, c, kap) * C::KSTR + C::E * g,
+                             Dr + chunk_pos(wy, wx, c, kap) * C::KSTR + C::E * g,
+                             [&](int mb, int ks) { return trans_frag<C>(Qt, TPS, wy, wx, c, mb, ks, lane); },
+                             [&](int mb, int ks) { return trans_frag<C>(Dt, TPS, wy, wx, c, mb, ks, lane); }, kf, vf, zok, qmask[c], a.scale_log2, lse2s, dlts, wy, wx, c, g, shift,
                              acck, accv);
             }
         }
@@ -619,10 +671,25 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid(LbDev a) {
         for (int r = 0; r < 16; ++r) {
             const int c = 32 * mb + acc_row(r, g);
             if (c < D) {
-                dk[c] = acck[mb][r] * out_scale;
-                dv[c] = from_f32<T>(accv[mb][r]);
+                if constexpr (PARTS & kDK) dk[c] = acck[mb][r] * out_scale;
+                if constexpr (PARTS & kDV) dv[c] = from_f32<T>(accv[mb][r]);
             }
         }
+}
+
+template <typename C>
+constexpr bool kSplitDkv = sizeof(typename C::T_) == 2 && C::D >= 128;
+
+template <typename T, int D, bool STRIPS>
+__global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid(LbDev a) {
+    if constexpr (kSplitDkv<Cfg<T, D>>) {
+        if (blockIdx.z == 0)
+            local_dkv<T, D, STRIPS, kDK>(a);
+        else
+            local_dkv<T, D, STRIPS, kDV>(a);
+    } else {
+        local_dkv<T, D, STRIPS, kDK | kDV>(a);
+    }
 }
 
 // k_local_dkv_grid with the planes copied by the LDS DMA (kBwdPlaneDma types).
@@ -718,12 +785,15 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid_dma(LbDev a) {
             for (int c = 0; c < 2; ++c) {
                 if (4 * c >= 4 + 2 * a.ry) continue;
                 const int kap = kperm<C::E, C::KS>(ki);
-                typename C::Frag qa[C::NT], da[C::NT], qt[C::MB * C::KSTEPS], dt[C::MB * C::KSTEPS];
-                load_kfrags<C>(Qb + chunk_pos(wy, wx, c, kap) * C::KSTR + C::E * g, qa);
-                load_kfrags<C>(Db + chunk_pos(wy, wx, c, kap) * C::KSTR + C::E * g, da);
-                PD::tfrags(Qb, wy, wx, c, lane, qt);
-                PD::tfrags(Db, wy, wx, c, lane, dt);
-                dkv_chunk<C>(qa, da, qt, dt, kf, vf, zok, qmask[c], a.scale_log2, lse2s, dlts, wy, wx, c, g, shift,
+                dkv_chunk<C>(Qb + chunk_pos(wy, wx, c, kap) * C::KSTR + C::E * g,
+                             Db + chunk_pos(wy, wx, c, kap) * C::KSTR + C::E * g,
+                             [&](int mb, int ks) {
+                                 return PD::tfrag(Qb, chunk_pos(wy, wx, c, ks * C::KS + C::E * g), mb, lane);
+                             },
+                             [&](int mb, int ks) {
+                                 return PD::tfrag(Db, chunk_pos(wy, wx, c, ks * C::KS + C::E * g), mb, lane);
+                             },
+                             kf, vf, zok, qmask[c], a.scale_log2, lse2s, dlts, wy, wx, c, g, shift,
                              acck, accv);
             }
         }
@@ -772,7 +842,7 @@ int launch_t(const LbDev& d, hipStream_t s) {
         const size_t l1 = lds_dq_grid<T, D>(), l2 = lds_dkv_grid<T, D>();
         if (l1 > 160 * 1024 || l2 > 160 * 1024) return fail(P3D_EUNSUPPORTED, "p3d_local_bwd_grid: planes exceed LDS");
         k_local_dq_grid<T, D, STRIPS><<<dim3(bricks, d.B * d.H), 64 * kWaves, l1, s>>>(d);
-        k_local_dkv_grid<T, D, STRIPS><<<dim3(bricks, d.B * d.G), 64 * kWaves, l2, s>>>(d);
+        k_local_dkv_grid<T, D, STRIPS><<<dim3(bricks, d.B * d.G, kSplitDkv<C> ? 2 : 1), 64 * kWaves, l2, s>>>(d);
     }
     return P3D_OK;
 }
