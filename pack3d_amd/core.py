@@ -273,22 +273,22 @@ def _mix_parts(rows):
 MIN_STAGES = 4
 
 
-def _splits(n, m, bg, rep, d):
+def _splits(n, m, bg, rep):
     """Query splits of the summary dK/dV pass over n queries of rep heads per
-    kv head, m summaries, bg = batch * kv heads and head_dim d.
+    kv head, m summaries and bg = batch * kv heads.
 
     Large problems take at least 1,024 queries a split, which gives every CU
     several workgroups.  Few summaries or few tokens leave most CUs idle there
     (64 workgroups at 16,384 queries and 256 summaries of 2 kv heads, 8 at
     4,096 queries and 128 summaries): shorter splits, down to MIN_STAGES stages
-    a workgroup, up to one round of resident workgroups (two per CU, one at
-    head_dim 128).  dK/dV 323 -> 117 us (head_dim 128, 256 summaries), 88 ->
-    36 us (head_dim 64, 64 summaries), 37 -> 11 us (4,096 queries, head_dim 16),
-    with 3 to 8 us for the sum of the partials."""
+    a workgroup, up to one round of resident workgroups (two per CU).  dK/dV
+    323 -> 117 us (head_dim 128, 256 summaries; 86 us since its stages leave
+    room for a second workgroup), 88 -> 36 us (head_dim 64, 64 summaries), 37 ->
+    11 us (4,096 queries, head_dim 16), with 3 to 8 us for the sum of the
+    partials."""
     blocks = -(-m // 128) * bg
     splits = max(1, min(64, -(-2048 // blocks), -(-n // 1024)))
-    resident = 512 if d <= 64 else 256
-    return max(splits, min(-(-resident // blocks), -(-n * rep // (64 * MIN_STAGES))))
+    return max(splits, min(-(-512 // blocks), -(-n * rep // (64 * MIN_STAGES))))
 
 
 def backward(dy, q, kl, vl, kg, vg, weight, bias, gate, sl, sg, sk, svt, sk_norm_max, o_local, o_global,
@@ -317,7 +317,7 @@ def backward(dy, q, kl, vl, kg, vg, weight, bias, gate, sl, sg, sk, svt, sk_norm
     gate_k = gate if gate.dtype in _lib.DTYPES else gate.float()
     sl32, sg32 = param_f32(sl), param_f32(sg)
     parts = _mix_parts(b * h * n)
-    splits = _splits(n, m, b * g, h // g, d)
+    splits = _splits(n, m, b * g, h // g)
 
     def empty(*shape, dtype=q.dtype):
         return torch.empty(*shape, dtype=dtype, device=dev)

@@ -244,10 +244,21 @@ struct DqDma {
     }
 };
 
-// Stage depth: 64 rows when two stages fit in the 160 KiB of LDS, else 32.
+// Stage depth: 64 rows, or 32 where two stages of 64 exceed `lds` bytes.  The
+// passes want two workgroups per CU (80 KB each), so that one computes while
+// the other waits at its barrier; only fp32 dK/dV, whose waves wait on long
+// MFMAs rather than on memory, is faster with one workgroup of 64-row stages
+// (263 against 327 us, 18,711 queries of 4 heads of 48, 693 summaries).  Same
+// case, dQ: 347 -> 255 us with 32-row stages; dK/dV at bf16 head_dim 128, 16,384
+// queries of 4 heads, 256 summaries: 116 -> 86 us.
 template <typename C, template <typename, int> class Stage>
-constexpr int stage_rows() {
-    return 2 * Stage<C, 64>::SIZE * (int)sizeof(typename C::T_) <= 160 * 1024 ? 64 : 32;
+constexpr int stage_rows(int lds) {
+    return 2 * Stage<C, 64>::SIZE * (int)sizeof(typename C::T_) <= lds ? 64 : 32;
+}
+template <typename C>
+constexpr int dq_rows() {
+    // Head_dim 128 fills the registers of one wave per SIMD: one workgroup.
+    return stage_rows<C, DqStage>(C::D >= 128 && sizeof(typename C::T_) == 2 ? 160 * 1024 : 80 * 1024);
 }
 
 // Zero rows [D, 32 * MB) of a transposed buffer (rows of `stride` elements).
@@ -280,9 +291,9 @@ __device__ __forceinline__ void load_row_frags(const typename C::T_* row, bool v
 // sk / sqrt(d)) (kernels.py:184-206).  Transposed tiles as in the forward:
 // lane = query; dS feeds the dQ^T = sk^T dS^T MFMA as its B operand.
 template <typename T, int D>
-__global__ __launch_bounds__(64 * kWaves, 2) void k_global_dq(BwdDev a) {
+__global__ __launch_bounds__(64 * kWaves, (D >= 128 || (sizeof(T) == 4 && D >= 64) ? 1 : 2)) void k_global_dq(BwdDev a) {
     typedef Cfg<T, D> C;
-    constexpr int SK = stage_rows<C, DqStage>();
+    constexpr int SK = dq_rows<C>();
     typedef DqStage<C, SK> S;
     extern __shared__ __align__(16) unsigned char smem[];
     T* lds = reinterpret_cast<T*>(smem);
@@ -370,7 +381,12 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_global_dq(BwdDev a) {
                 typename C::Frag kf[C::NT], vf[C::NT], tf[C::MB * C::KSTEPS];
                 load_kfrags<C>(cur + (32 * tt + kperm<C::E, C::KS>(qi)) * C::KSTR + C::E * g, kf);
                 load_kfrags<C>(cur + SK * C::KSTR + (32 * tt + kperm<C::E, C::KS>(qi)) * C::KSTR + C::E * g, vf);
-                load_vfrags<C, true>(cur + 2 * SK * C::KSTR, S::TGS, 32 * tt, lane, tf);
+                // Wide types load sk^T once the scores are done (a scheduling
+                // barrier keeps the loads there): all three sets together spill.
+                // 16-bit head_dim 128, 16,384 queries of 4 heads: 124 us with
+                // 284 registers spilled, 37 us.
+                constexpr bool LATE = D >= 128 || sizeof(T) == 4;
+                if constexpr (!LATE) load_vfrags<C, true>(cur + 2 * SK * C::KSTR, S::TGS, 32 * tt, lane, tf);
 #pragma unroll
                 for (int nb = 0; nb < 2; ++nb) {
                     f32x16 s;
@@ -391,6 +407,10 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_global_dq(BwdDev a) {
 #pragma unroll
                         for (int r = 0; r < 16; ++r)
                             if (first + kperm<C::E, C::KS>(acc_row(r, g)) >= a.M) ds[r] = 0.f;
+                    }
+                    if constexpr (LATE) {
+                        __builtin_amdgcn_sched_barrier(0);
+                        load_vfrags<C, true>(cur + 2 * SK * C::KSTR, S::TGS, 32 * tt, lane, tf);
                     }
 #pragma unroll
                     for (int ks = 0; ks < C::KSTEPS; ++ks) {
@@ -592,6 +612,10 @@ struct KvTransDma {
 // (divided by sqrt(d)), before the pooling's 1/count.
 template <typename C, int SK>
 using KvStageR = KvStage<C, SK>;
+template <typename C>
+constexpr int kv_rows() {
+    return stage_rows<C, KvStageR>(sizeof(typename C::T_) == 4 ? 160 * 1024 : 80 * 1024);
+}
 
 // Stand-in for KvTransDma where the transposed regions are staged from registers.
 struct NoTransDma {
@@ -602,7 +626,7 @@ struct NoTransDma {
 template <typename T, int D, bool TDMA>
 __global__ __launch_bounds__(64 * kWaves, 2) void k_global_dkv(BwdDev a) {
     typedef Cfg<T, D> C;
-    constexpr int SK = stage_rows<C, KvStageR>();
+    constexpr int SK = kv_rows<C>();
     typedef KvStage<C, SK, TDMA> S;
     extern __shared__ __align__(16) unsigned char smem[];
     T* lds = reinterpret_cast<T*>(smem);
@@ -866,12 +890,12 @@ int fill_bwd(const p3d_bwd_args& x, BwdDev& d) {
 
 template <typename C>
 size_t lds_dq() {
-    return (size_t)2 * DqStage<C, stage_rows<C, DqStage>()>::SIZE * sizeof(typename C::T_);
+    return (size_t)2 * DqStage<C, dq_rows<C>()>::SIZE * sizeof(typename C::T_);
 }
 
 template <typename C>
 size_t lds_dkv() {
-    return (size_t)2 * KvStage<C, stage_rows<C, KvStageR>()>::SIZE * sizeof(typename C::T_);
+    return (size_t)2 * KvStage<C, kv_rows<C>()>::SIZE * sizeof(typename C::T_);
 }
 
 template <int D>

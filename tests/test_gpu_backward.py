@@ -394,7 +394,7 @@ def test_every_gradient_many_splits(gpu, dtype, n, d, heads, kv_heads):
     print(f"backward splits n{n} d{d} {dtype}", flush=True)
     inputs, nb, blocks, pool = make_case(n, d, 1, heads, kv_heads, 16, 16, dtype=dtype)
     og, hg = ref.prepare_geometry(nb, blocks, pool), p3d.prepare_geometry(nb.to(gpu), blocks.to(gpu), pool)
-    assert _splits(n, og.num_summaries, kv_heads, heads // kv_heads, d) > 16
+    assert _splits(n, og.num_summaries, kv_heads, heads // kv_heads) > 16
     xs = [t.to(gpu).requires_grad_() for t in inputs]
     rs = [t.detach().clone().requires_grad_() for t in inputs]
     y, e = p3d.pack3d_hip(*xs, hg), ref.pack3d_reference(*rs, og)
