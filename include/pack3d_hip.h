@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define P3D_ABI_VERSION 21
+#define P3D_ABI_VERSION 22
 
 enum p3d_status { P3D_OK = 0, P3D_EINVAL = 1, P3D_EHIP = 2, P3D_EUNSUPPORTED = 3 };
 enum p3d_dtype { P3D_F32 = 0, P3D_F16 = 1, P3D_BF16 = 2 };
@@ -444,10 +444,14 @@ typedef struct p3d_bwd_args {
     float* dsg_part;            /* out of mix: [parts, D] partial dsg */
     void* sv_rows;              /* workspace [B,G,Mp,D] (dtype) */
     void* skt;                  /* workspace [B,G,Mp/32,D,32] (dtype) */
-    float* dq_local;            /* out: [B,H,N,D] fp32, rotated space */
-    float* dq_global;           /* out: [B,H,N,D] fp32, rotated space */
-    float* dk_local;            /* out: [B,G,N,D] fp32, rotated space */
-    p3d_view dv_local;          /* out: [B,G,N,D] view (dtype), 16-byte aligned rows */
+    p3d_rope rope;              /* the rotation of q and kl, applied backward to their gradients */
+    void* dq_local;             /* workspace [B,H,N,D] (dtype): local part of dq, rotated space;
+                                   written by the local passes, read by p3d_global_bwd_dq */
+    p3d_view dq;                /* out of p3d_global_bwd_dq: [B,H,N,D] gradient of the unrotated q */
+    p3d_view dk_local;          /* out of the local passes: [B,G,N,D] gradient of the unrotated kl */
+    p3d_view dv_local;          /* out of the local passes: [B,G,N,D]; the three views of dtype,
+                                   16-byte aligned rows (e.g. column ranges of the projections'
+                                   gradients) */
     float* dsk_part;            /* out: [splits,B,G,Mp,D] fp32, true key units */
     float* dsv_part;            /* out: [splits,B,G,Mp,D] fp32 */
     const void* q_t;            /* optional: rotated q transposed, [B*H][D][N] (p3d_transpose_rows) */
@@ -462,7 +466,8 @@ typedef struct p3d_bwd_args {
 int p3d_mix_bwd(const p3d_bwd_args* args, void* stream);
 
 /* Local pathway backward for any validated graph (kernels.py:130-181): dq_local
- * over the neighbour rows, dk_local / dv_local over the reverse adjacency. */
+ * over the neighbour rows, dk_local = R^T round(dk) (R^T the inverse rotation of
+ * rope) and dv_local over the reverse adjacency. */
 int p3d_local_bwd_indexed(const p3d_bwd_args* args, const int32_t* neighbors, int32_t width,
                           const int32_t* reverse, int32_t rwidth, void* stream);
 
@@ -475,12 +480,13 @@ int p3d_local_bwd_indexed(const p3d_bwd_args* args, const int32_t* neighbors, in
 int p3d_local_bwd_grid(const p3d_bwd_args* args, const int32_t grid[3], const int32_t radius[3],
                        const int32_t* raster_to_packed, void* stream);
 
-/* Summary pathway backward (kernels.py:184-237): dq_global and the split
- * partials dsk_part / dsv_part (sv_rows and skt are filled first). */
+/* Summary pathway backward (kernels.py:184-237), after the local pathway's:
+ * dq = R^T round(dq_local + round(dq_global)) (kernels.py:202-206 rounding) and
+ * the split partials dsk_part / dsv_part (sv_rows and skt are filled first). */
 int p3d_global_bwd(const p3d_bwd_args* args, void* stream);
 
 /* The two halves of p3d_global_bwd, for callers that time or order them
- * separately: _dq fills sv_rows and skt and computes dq_global
+ * separately: _dq fills sv_rows and skt and computes dq
  * (kernels.py:179-207, the _global_dq pass); _dkv computes the split
  * partials dsk_part / dsv_part (kernels.py:209-240, the _global_dkv pass)
  * and reads the skt / sv_rows that _dq wrote, so it runs after it on the
@@ -495,12 +501,6 @@ int p3d_global_bwd_dkv(const p3d_bwd_args* args, void* stream);
  * stages them for the summary dK/dV pass. */
 int p3d_transpose_rows(p3d_view src, void* dst, int32_t batch, int32_t heads, int32_t tokens, int32_t head_dim,
                        int32_t dtype, void* stream);
-
-/* dq = R^T round(round(dq_local) + round(dq_global)) and dkl = R^T round(dk_local)
- * (kernels.py:202-206 rounding; R^T the inverse rotation of rope), written
- * into the views dq [B,H,N,D] and dkl [B,G,N,D] of dtype (16-byte aligned
- * rows; e.g. the q and kl column ranges of the projections' gradients). */
-int p3d_finish_bwd(const p3d_bwd_args* args, const p3d_rope* rope, p3d_view dq, p3d_view dkl, void* stream);
 
 /* Pooling backward (kernels.py:240-270): from the split partials of dsk / dsv
  * (scratch: with more than 16 splits they are summed into the first, in place),

@@ -327,8 +327,7 @@ def backward(dy, q, kl, vl, kg, vg, weight, bias, gate, sl, sg, sk, svt, sk_norm
                 dg=empty(b, h, n, dtype=f32), dgate=empty(b, h, n, dtype=gate_k.dtype),
                 dslp=empty(parts, d, dtype=f32), dsgp=empty(parts, d, dtype=f32),
                 sv_rows=empty(b, g, mp, d), skt=empty(b, g, mp // 32, d, 32),
-                dql=empty(b, h, n, d, dtype=f32), dqg=empty(b, h, n, d, dtype=f32),
-                dkl=empty(b, g, n, d, dtype=f32),
+                dql=empty(b, h, n, d),
                 dskp=empty(splits, b, g, mp, d, dtype=f32), dsvp=empty(splits, b, g, mp, d, dtype=f32))
     a = _lib.BwdArgs()
     a.batch, a.heads, a.kv_heads, a.tokens, a.head_dim, a.dtype = b, h, g, n, d, dt
@@ -342,11 +341,11 @@ def backward(dy, q, kl, vl, kg, vg, weight, bias, gate, sl, sg, sk, svt, sk_norm
     a.dol, a.dog, a.delta_local, a.delta_global = (bufs[k].data_ptr() for k in ("dol", "dog", "dl", "dg"))
     a.dgate, a.dsl_part, a.dsg_part = (bufs[k].data_ptr() for k in ("dgate", "dslp", "dsgp"))
     a.sv_rows, a.skt = bufs["sv_rows"].data_ptr(), bufs["skt"].data_ptr()
-    a.dq_local, a.dq_global, a.dk_local = (bufs[k].data_ptr() for k in ("dql", "dqg", "dkl"))
+    a.dq_local, a.rope = bufs["dql"].data_ptr(), rope.struct()
     if out is None:
         out = tuple(empty(b, hh, n, d) for hh in (h, g, g, g, g))
     dq, dkl, dvl, dkg, dvg = out
-    a.dv_local = _lib.view(dvl)
+    a.dq, a.dk_local, a.dv_local = _lib.view(dq), _lib.view(dkl), _lib.view(dvl)
     a.dsk_part, a.dsv_part = bufs["dskp"].data_ptr(), bufs["dsvp"].data_ptr()
     keep += [qr, klr, gate_k, sl32, sg32, dy]
 
@@ -368,7 +367,6 @@ def backward(dy, q, kl, vl, kg, vg, weight, bias, gate, sl, sg, sk, svt, sk_norm
         _lib.call("p3d_transpose_rows", _lib.view(bufs["dog"]), bufs["dog_t"].data_ptr(), b, h, n, d, dt, stream)
         a.q_t, a.dog_t = bufs["q_t"].data_ptr(), bufs["dog_t"].data_ptr()
     _lib.call("p3d_global_bwd_dkv", a, stream)
-    _lib.call("p3d_finish_bwd", a, rope.struct(), _lib.view(dq), _lib.view(dkl), stream)
 
     w32 = param_f32(weight)
     b32 = param_f32(bias)

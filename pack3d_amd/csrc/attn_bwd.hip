@@ -41,9 +41,10 @@ struct BwdDev {
     char* dgate;
     float *dsl_part, *dsg_part;
     char *sv_rows, *skt;
-    float *dq_l, *dq_g, *dk_l;
-    char* dv_l;
-    int64_t dvsb, dvsh, dvsn;
+    RopeDev rope;
+    const char* dq_l;  // [B,H,N,D] storage type
+    char* dq;
+    int64_t dqsb, dqsh, dqsn;
     float *dsk_part, *dsv_part;
     const char *q_t, *dog_t;  // optional: q and dO_G transposed, [B*H][D][N]
 };
@@ -286,10 +287,14 @@ __device__ __forceinline__ void load_row_frags(const typename C::T_* row, bool v
 }
 
 // Global dQ: per query, over all summaries, S = q . sk (log2 units), P =
-// 2^(S - lse_G log2 e), dP = dO_G . sv, dS = P (dP - Delta_G), dQ = ln 2 *
+// 2^(S - lse_G log2 e), dP = dO_G . sv, dS = P (dP - Delta_G), dQ_G = ln 2 *
 // sum dS sk_stored (sk_stored = sk log2(e)/sqrt(d), so ln 2 * sk_stored =
 // sk / sqrt(d)) (kernels.py:184-206).  Transposed tiles as in the forward:
-// lane = query; dS feeds the dQ^T = sk^T dS^T MFMA as its B operand.
+// lane = query; dS feeds the dQ^T = sk^T dS^T MFMA as its B operand.  The
+// epilogue writes the finished gradient dq = R^T round(round(dQ_L) +
+// round(dQ_G)) (kernels.py:202-206 rounding): dQ_L comes from the local pass in
+// the storage type it is rounded to anyway, and dQ_G never reaches memory.  A
+// pass over fp32 copies of both took 181 us at 262,144 tokens (4 heads of 48).
 template <typename T, int D>
 __global__ __launch_bounds__(64 * kWaves, (D >= 128 || (sizeof(T) == 4 && D >= 64) ? 1 : 2)) void k_global_dq(BwdDev a) {
     typedef Cfg<T, D> C;
@@ -297,9 +302,11 @@ __global__ __launch_bounds__(64 * kWaves, (D >= 128 || (sizeof(T) == 4 && D >= 6
     typedef DqStage<C, SK> S;
     extern __shared__ __align__(16) unsigned char smem[];
     T* lds = reinterpret_cast<T*>(smem);
+    int4* meta = reinterpret_cast<int4*>(lds + 2 * S::SIZE);  // the rotation's pairs, for the epilogue
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 5, qi = lane & 31;
     const int bh = blockIdx.y, b = bh / a.H, h = bh % a.H, kvh = h / (a.H / a.G);
     const int64_t bg = (int64_t)b * a.G + kvh;
+    stage_pair_meta(a.rope, D, meta);
 
     typename C::Frag qf[2][C::NT], df[2][C::NT];
     int64_t qrow[2];
@@ -436,13 +443,22 @@ __global__ __launch_bounds__(64 * kWaves, (D >= 128 || (sizeof(T) == 4 && D >= 6
 #pragma unroll
     for (int nb = 0; nb < 2; ++nb) {
         if (!qok[nb]) continue;
-        float* dq = a.dq_g + ((int64_t)bh * a.N + qrow[nb]) * D;
+        const T* dql = tp<T>(a.dq_l) + ((int64_t)bh * a.N + qrow[nb]) * D;
+        T* dq = reinterpret_cast<T*>(a.dq) + b * a.dqsb + h * a.dqsh + qrow[nb] * a.dqsn;
+        int pos[3];
+        rope_position32(a.rope, (int)qrow[nb], pos);
 #pragma unroll
         for (int mb = 0; mb < C::MB; ++mb)
 #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                const int c = 32 * mb + acc_row(r, g);
-                if (c < D) dq[c] = acc[nb][mb][r] * out_scale;
+            for (int q = 0; q < 4; ++q) {  // four consecutive channels: two rotary pairs
+                if (32 * mb + 8 * q >= D) continue;
+                const int c0 = 32 * mb + acc_row(4 * q, g);
+                float x[4];
+                load_quad4<T>(dql + c0, x);
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[i] += round_to<T>(acc[nb][mb][4 * q + i] * out_scale);
+                rotate_back<T, 4>(a.rope, meta, pos, c0, x);
+                store_quad4<T>(dq + c0, x);
             }
     }
 }
@@ -763,60 +779,6 @@ __global__ __launch_bounds__(64 * kWaves, 2) void k_global_dkv(BwdDev a) {
         }
 }
 
-// ------------------------------------------------------------------ finish
-// dQ = R^T round(round(dQ_L) + round(dQ_G)) and dK_L = R^T round(dK_L), each
-// rounded to the storage type; one 16-byte output piece per thread.  Grid y
-// walks the (batch, head) planes of dq and then those of dkl; grid x the
-// pieces of a plane's rows.  The fp32 inputs are read 16 bytes at a time and
-// the rotation's pair descriptors come from LDS.
-template <typename T, int D>
-__global__ __launch_bounds__(256) void k_finish_bwd(BwdDev a, RopeDev rope, int plane0, p3d_view dq, p3d_view dkl) {
-    constexpr int EP = Piece<T>::N;
-    constexpr int PPR = D / EP;  // pieces per row
-    __shared__ int4 meta[D / 2];
-    for (int j = threadIdx.x; j < D / 2; j += blockDim.x) meta[j] = pair_meta(rope.pairs, j);
-    __syncthreads();
-    // Plane p: (b, head) of dq for p < B*H, else (b, kv head) of dkl.  Rows
-    // of a plane times its pieces fit in 31 bits (checked on the host).
-    const int p = plane0 + (int)blockIdx.y;
-    const int idx = (int)blockIdx.x * 256 + (int)threadIdx.x;
-    if (idx >= a.N * PPR) return;
-    const int n = idx / PPR, piece = idx - n * PPR;
-    const bool isq = p < a.B * a.H;
-    const int pp = isq ? p : p - a.B * a.H, heads = isq ? a.H : a.G;
-    const int64_t off = (int64_t)pp * a.N * D + (int64_t)n * D + piece * EP;  // dense fp32 inputs
-    float x[EP];
-    if (isq) {
-        const f32x4* l = reinterpret_cast<const f32x4*>(a.dq_l + off);
-        const f32x4* g = reinterpret_cast<const f32x4*>(a.dq_g + off);
-#pragma unroll
-        for (int v = 0; v < EP / 4; ++v) {
-            const f32x4 lv = l[v], gv = g[v];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) x[4 * v + i] = round_to<T>(round_to<T>(lv[i]) + round_to<T>(gv[i]));
-        }
-    } else {
-        const f32x4* l = reinterpret_cast<const f32x4*>(a.dk_l + off);
-#pragma unroll
-        for (int v = 0; v < EP / 4; ++v) {
-            const f32x4 lv = l[v];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) x[4 * v + i] = round_to<T>(lv[i]);
-        }
-    }
-    int pos[3];
-    rope_position32(rope, n, pos);
-#pragma unroll
-    for (int e = 0; e < EP; e += 2) {
-        const int4 m = meta[(piece * EP + e) >> 1];
-        const float2 cs = rope.table[m.x + m.y * pos[0] + m.z * pos[1] + m.w * pos[2]];
-        rotate_pair(x[e], x[e + 1], cs.x, -cs.y);
-    }
-    const p3d_view& o = isq ? dq : dkl;
-    const int b = pp / heads, h = pp - b * heads;
-    store_piece<T>(reinterpret_cast<T*>(o.data) + b * o.sb + h * o.sh + (int64_t)n * o.sn + piece * EP, x);
-}
-
 // ------------------------------------------------------------ transpose
 // dst[(b H + h) D + c][n] = src[b][h][n][c] for 16-bit rows (N a multiple
 // of 8): a thread loads an 8-row x 8-channel block as eight 16-byte pieces,
@@ -881,8 +843,9 @@ int fill_bwd(const p3d_bwd_args& x, BwdDev& d) {
     d.dgate = (char*)x.dgate;
     d.dsl_part = x.dsl_part, d.dsg_part = x.dsg_part;
     d.sv_rows = (char*)x.sv_rows, d.skt = (char*)x.skt;
-    d.dq_l = x.dq_local, d.dq_g = x.dq_global, d.dk_l = x.dk_local;
-    d.dv_l = (char*)x.dv_local.data, d.dvsb = x.dv_local.sb, d.dvsh = x.dv_local.sh, d.dvsn = x.dv_local.sn;
+    d.rope = rope_dev(x.rope);
+    d.dq_l = (const char*)x.dq_local;
+    d.dq = (char*)x.dq.data, d.dqsb = x.dq.sb, d.dqsh = x.dq.sh, d.dqsn = x.dq.sn;
     d.dsk_part = x.dsk_part, d.dsv_part = x.dsv_part;
     d.q_t = (const char*)x.q_t, d.dog_t = (const char*)x.dog_t;
     return P3D_OK;
@@ -890,7 +853,8 @@ int fill_bwd(const p3d_bwd_args& x, BwdDev& d) {
 
 template <typename C>
 size_t lds_dq() {
-    return (size_t)2 * DqStage<C, dq_rows<C>()>::SIZE * sizeof(typename C::T_);
+    static_assert(2 * DqStage<C, dq_rows<C>()>::SIZE * sizeof(typename C::T_) % 16 == 0, "pair metadata alignment");
+    return (size_t)2 * DqStage<C, dq_rows<C>()>::SIZE * sizeof(typename C::T_) + (size_t)(C::D / 2) * sizeof(int4);
 }
 
 template <typename C>
@@ -975,7 +939,7 @@ int global_bwd_args(const p3d_bwd_args* args, BwdDev& d) {
     if (int rc = fill_bwd(*args, d)) return rc;
     P3D_REQUIRE(args->splits >= 1, "splits must be positive");
     P3D_REQUIRE(args->sk && args->svt && args->sv_rows && args->skt && args->dog && args->lse_global &&
-                    args->delta_global && args->dq_global && args->dsk_part && args->dsv_part,
+                    args->delta_global && args->dsk_part && args->dsv_part,
                 "null pointer argument");
     return P3D_OK;
 }
@@ -984,6 +948,9 @@ int global_bwd_args(const p3d_bwd_args* args, BwdDev& d) {
 extern "C" int p3d_global_bwd_dq(const p3d_bwd_args* args, void* stream) {
     BwdDev d;
     if (int rc = global_bwd_args(args, d)) return rc;
+    P3D_REQUIRE(args->dq_local && aligned16(args->dq_local) && view_ok(args->dq, dtype_size(args->dtype)),
+                "dq_local and the rows of dq must be 16-byte aligned");
+    P3D_REQUIRE(args->rope.table && args->rope.pairs && (args->rope.packed || args->rope.coords), "bad rope arguments");
     hipStream_t s = as_stream(stream);
     const int64_t te = (int64_t)d.B * d.G * d.Mp * args->head_dim;
     switch (args->dtype) {
@@ -1005,50 +972,6 @@ extern "C" int p3d_global_bwd_dkv(const p3d_bwd_args* args, void* stream) {
 extern "C" int p3d_global_bwd(const p3d_bwd_args* args, void* stream) {
     if (int rc = p3d_global_bwd_dq(args, stream)) return rc;
     return p3d_global_bwd_dkv(args, stream);
-}
-
-template <typename T, int D>
-void launch_finish(const BwdDev& d, const RopeDev& r, const p3d_view& dq, const p3d_view& dkl, hipStream_t s) {
-    constexpr int PPR = D / Piece<T>::N;
-    const unsigned bx = (unsigned)cdiv((int64_t)d.N * PPR, 256);
-    const int planes = d.B * (d.H + d.G);
-    for (int p0 = 0; p0 < planes; p0 += 65535) {
-        const unsigned by = (unsigned)(planes - p0 < 65535 ? planes - p0 : 65535);
-        k_finish_bwd<T, D><<<dim3(bx, by), 256, 0, s>>>(d, r, p0, dq, dkl);
-    }
-}
-
-template <typename T>
-void dispatch_finish(const BwdDev& d, const RopeDev& r, int head_dim, const p3d_view& dq, const p3d_view& dkl,
-                     hipStream_t s) {
-    switch (head_dim) {
-        case 16: launch_finish<T, 16>(d, r, dq, dkl, s); break;
-        case 32: launch_finish<T, 32>(d, r, dq, dkl, s); break;
-        case 48: launch_finish<T, 48>(d, r, dq, dkl, s); break;
-        case 64: launch_finish<T, 64>(d, r, dq, dkl, s); break;
-        default: launch_finish<T, 128>(d, r, dq, dkl, s); break;
-    }
-}
-
-extern "C" int p3d_finish_bwd(const p3d_bwd_args* args, const p3d_rope* rope, p3d_view dq, p3d_view dkl,
-                              void* stream) {
-    P3D_REQUIRE(args && rope, "null argument");
-    BwdDev d;
-    if (int rc = fill_bwd(*args, d)) return rc;
-    P3D_REQUIRE(args->dq_local && args->dq_global && args->dk_local, "null pointer argument");
-    P3D_REQUIRE(rope->table && rope->pairs && (rope->packed || rope->coords), "bad rope arguments");
-    const int ep = 16 / dtype_size(args->dtype);
-    P3D_REQUIRE((int64_t)d.N * (args->head_dim / ep) < ((int64_t)1 << 31), "tokens * pieces per row must be below 2^31");
-    P3D_REQUIRE(view_ok(dq, dtype_size(args->dtype)) && view_ok(dkl, dtype_size(args->dtype)),
-                "dq / dkl rows must be 16-byte aligned");
-    hipStream_t s = as_stream(stream);
-    const RopeDev r = rope_dev(*rope);
-    switch (args->dtype) {
-        case P3D_F32: dispatch_finish<float>(d, r, args->head_dim, dq, dkl, s); break;
-        case P3D_F16: dispatch_finish<_Float16>(d, r, args->head_dim, dq, dkl, s); break;
-        default: dispatch_finish<__bf16>(d, r, args->head_dim, dq, dkl, s); break;
-    }
-    return check_launch("p3d_finish_bwd");
 }
 
 extern "C" int p3d_transpose_rows(p3d_view src, void* dst, int32_t batch, int32_t heads, int32_t tokens,

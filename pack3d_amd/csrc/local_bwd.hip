@@ -34,10 +34,10 @@ struct LbDev {
     const char* dol;          // [B,H,N,D] contiguous
     const float *lse, *delta;  // [B,H,N]
     const int32_t* map;        // raster -> packed row, or null
-    float* dq;                 // [B,H,N,D] fp32
-    float* dk;                 // [B,G,N,D] fp32
-    char* dv;                  // [B,G,N,D] view, storage type
-    int64_t dvsb, dvsh, dvsn;
+    char* dq;                  // [B,H,N,D] storage type, rotated space
+    char *dk, *dv;             // [B,G,N,D] views, storage type; dk rotated back
+    int64_t dksb, dksh, dksn, dvsb, dvsh, dvsn;
+    RopeDev rope;
     float scale_log2, scale;   // log2(e)/sqrt(D), 1/sqrt(D)
 };
 
@@ -398,6 +398,53 @@ struct BwdPlaneDma {
     }
 };
 
+// dQ_L in the storage type: the pass that adds dQ_G rounds it to that type first.
+template <typename C>
+__device__ __forceinline__ void store_dq(const LbDev& a, int64_t qidx, int g, const f32x16* acc, float scale) {
+    typedef typename C::T_ T;
+    T* dq = reinterpret_cast<T*>(a.dq) + qidx * C::D;
+#pragma unroll
+    for (int mb = 0; mb < C::MB; ++mb)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {
+            if (32 * mb + 8 * q >= C::D) continue;
+            float x[4];
+#pragma unroll
+            for (int i = 0; i < 4; ++i) x[i] = acc[mb][4 * q + i] * scale;
+            store_quad4<T>(dq + 32 * mb + acc_row(4 * q, g), x);
+        }
+}
+
+// dk = R^T round(dK) and dv of one key row; meta: the rotation's pairs in LDS.
+template <typename C, int PARTS = 3>
+__device__ __forceinline__ void store_dkv(const LbDev& a, const int4* meta, int b, int kvh, int64_t row, int g,
+                                          const f32x16* acck, const f32x16* accv, float scale) {
+    typedef typename C::T_ T;
+    T* dk = reinterpret_cast<T*>(a.dk) + b * a.dksb + kvh * a.dksh + row * a.dksn;
+    T* dv = reinterpret_cast<T*>(a.dv) + b * a.dvsb + kvh * a.dvsh + row * a.dvsn;
+    int pos[3];
+    rope_position32(a.rope, (int)row, pos);
+#pragma unroll
+    for (int mb = 0; mb < C::MB; ++mb)
+#pragma unroll
+        for (int q = 0; q < 4; ++q) {  // four consecutive channels: two rotary pairs
+            if (32 * mb + 8 * q >= C::D) continue;
+            const int c0 = 32 * mb + acc_row(4 * q, g);
+            float x[4];
+            if constexpr (PARTS & 1) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[i] = acck[mb][4 * q + i] * scale;
+                rotate_back<T, 4>(a.rope, meta, pos, c0, x);
+                store_quad4<T>(dk + c0, x);
+            }
+            if constexpr (PARTS & 2) {
+#pragma unroll
+                for (int i = 0; i < 4; ++i) x[i] = accv[mb][4 * q + i];
+                store_quad4<T>(dv + c0, x);
+            }
+        }
+}
+
 template <typename T, int D, bool STRIPS>
 __global__ __launch_bounds__(64 * kWaves) void k_local_dq_grid(LbDev a) {
     typedef Cfg<T, D> C;
@@ -464,15 +511,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dq_grid(LbDev a) {
         }
     }
     if (!qok) return;
-    float* dq = a.dq + qidx * D;
-    const float out_scale = ldexpf(a.scale, shift);
-#pragma unroll
-    for (int mb = 0; mb < C::MB; ++mb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int c = 32 * mb + acc_row(r, g);
-            if (c < D) dq[c] = acc[mb][r] * out_scale;
-        }
+    store_dq<C>(a, qidx, g, acc, ldexpf(a.scale, shift));
 }
 
 // k_local_dq_grid with the planes copied by the LDS DMA (kBwdPlaneDma types).
@@ -547,15 +586,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dq_grid_dma(LbDev a) {
         }
     }
     if (!qok) return;
-    float* dq = a.dq + qidx * D;
-    const float out_scale = ldexpf(a.scale, shift);
-#pragma unroll
-    for (int mb = 0; mb < C::MB; ++mb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int c = 32 * mb + acc_row(r, g);
-            if (c < D) dq[c] = acc[mb][r] * out_scale;
-        }
+    store_dq<C>(a, qidx, g, acc, ldexpf(a.scale, shift));
 }
 
 // lse (log2 units; +inf where the position has no gradient: outside the grid
@@ -589,6 +620,8 @@ __device__ __forceinline__ void local_dkv(const LbDev& a) {
     T* Dt = Qt + 32 * C::MB * TPS;
     float* lse2s = reinterpret_cast<float*>(Dt + 32 * C::MB * TPS);
     float* dlts = lse2s + kPlaneKeys;
+    int4* meta = reinterpret_cast<int4*>(dlts + kPlaneKeys);  // the rotation's pairs, for the epilogue
+    stage_pair_meta(a.rope, D, meta);
 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 5, ki = lane & 31;
     const int bg = blockIdx.y, b = bg / a.G, kvh = bg % a.G, rep = a.H / a.G;
@@ -661,20 +694,7 @@ __device__ __forceinline__ void local_dkv(const LbDev& a) {
         }
     }
     if (!kok) return;
-    const int64_t kidx = (int64_t)bg * a.N + krow;
-    float* dk = a.dk + kidx * D;
-    T* dv = reinterpret_cast<T*>(a.dv) + b * a.dvsb + kvh * a.dvsh + (int64_t)krow * a.dvsn;
-    const float out_scale = ldexpf(a.scale, shift);
-#pragma unroll
-    for (int mb = 0; mb < C::MB; ++mb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int c = 32 * mb + acc_row(r, g);
-            if (c < D) {
-                if constexpr (PARTS & kDK) dk[c] = acck[mb][r] * out_scale;
-                if constexpr (PARTS & kDV) dv[c] = from_f32<T>(accv[mb][r]);
-            }
-        }
+    store_dkv<C, PARTS>(a, meta, b, kvh, krow, g, acck, accv, ldexpf(a.scale, shift));
 }
 
 template <typename C>
@@ -702,6 +722,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid_dma(LbDev a) {
     typedef BwdPlaneDma<C, true> PD;
     extern __shared__ __align__(16) unsigned char smem[];
     int* const rowtab = reinterpret_cast<int*>(smem + 2 * PD::BUF);
+    int4* meta = reinterpret_cast<int4*>(smem + PD::BYTES);  // the rotation's pairs, for the epilogue
+    stage_pair_meta(a.rope, D, meta);
 
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 5, ki = lane & 31;
     const int bg = blockIdx.y, b = bg / a.G, kvh = bg % a.G, rep = a.H / a.G;
@@ -800,20 +822,7 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid_dma(LbDev a) {
         if (more) side_store(i + 1, l2n, dln);
     }
     if (!kok) return;
-    const int64_t kidx = (int64_t)bg * a.N + krow;
-    float* dk = a.dk + kidx * D;
-    T* dv = reinterpret_cast<T*>(a.dv) + b * a.dvsb + kvh * a.dvsh + (int64_t)krow * a.dvsn;
-    const float out_scale = ldexpf(a.scale, shift);
-#pragma unroll
-    for (int mb = 0; mb < C::MB; ++mb)
-#pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int c = 32 * mb + acc_row(r, g);
-            if (c < D) {
-                dk[c] = acck[mb][r] * out_scale;
-                dv[c] = from_f32<T>(accv[mb][r]);
-            }
-        }
+    store_dkv<C>(a, meta, b, kvh, krow, g, acck, accv, ldexpf(a.scale, shift));
 }
 
 template <typename T, int D>
@@ -826,7 +835,7 @@ template <typename T, int D>
 size_t lds_dkv_grid() {
     typedef Cfg<T, D> C;
     return ((size_t)2 * kPlaneKeys * C::KSTR + (size_t)2 * 32 * C::MB * (kPlaneKeys + Piece<T>::N)) * sizeof(T) +
-           (size_t)2 * kPlaneKeys * sizeof(float);
+           (size_t)2 * kPlaneKeys * sizeof(float) + (size_t)(D / 2) * sizeof(int4);
 }
 
 template <typename T, int D, bool STRIPS>
@@ -834,7 +843,9 @@ int launch_t(const LbDev& d, hipStream_t s) {
     typedef Cfg<T, D> C;
     const int bricks = (int)(cdiv(d.Z, 4) * d.bricks_y * d.bricks_x);
     if constexpr (kBwdPlaneDma<C>) {
-        constexpr size_t l1 = BwdPlaneDma<C, false>::BYTES, l2 = BwdPlaneDma<C, true>::BYTES;
+        constexpr size_t l1 = BwdPlaneDma<C, false>::BYTES;
+        constexpr size_t l2 = BwdPlaneDma<C, true>::BYTES + (D / 2) * sizeof(int4);
+        static_assert(BwdPlaneDma<C, true>::BYTES % 16 == 0, "pair metadata alignment");
         static_assert(l1 <= 160 * 1024 && l2 <= 160 * 1024, "plane buffers within LDS");
         k_local_dq_grid_dma<T, D, STRIPS><<<dim3(bricks, d.B * d.H), 64 * kWaves, l1, s>>>(d);
         k_local_dkv_grid_dma<T, D, STRIPS><<<dim3(bricks, d.B * d.G), 64 * kWaves, l2, s>>>(d);
@@ -877,8 +888,9 @@ extern "C" int p3d_local_bwd_grid(const p3d_bwd_args* args, const int32_t grid[3
                     radius[2] <= 2,
                 "grid radius must be 0..2 per axis");
     P3D_REQUIRE(view_ok(x.q, es) && view_ok(x.kl, es) && view_ok(x.vl, es), "q/k/v rows must be 16-byte aligned");
-    P3D_REQUIRE(x.dol && x.lse_local && x.delta_local && x.dq_local && x.dk_local && view_ok(x.dv_local, es),
-                "null pointer argument");
+    P3D_REQUIRE(x.dol && x.lse_local && x.delta_local && x.dq_local && aligned16(x.dq_local), "null pointer argument");
+    P3D_REQUIRE(view_ok(x.dk_local, es) && view_ok(x.dv_local, es), "dk / dv rows must be 16-byte aligned");
+    P3D_REQUIRE(x.rope.table && x.rope.pairs && (x.rope.packed || x.rope.coords), "bad rope arguments");
     LbDev d{};
     d.B = x.batch, d.H = x.heads, d.G = x.kv_heads, d.N = x.tokens;
     d.Z = grid[0], d.Y = grid[1], d.X = grid[2];
@@ -895,8 +907,9 @@ extern "C" int p3d_local_bwd_grid(const p3d_bwd_args* args, const int32_t grid[3
     d.dol = (const char*)x.dol;
     d.lse = x.lse_local, d.delta = x.delta_local;
     d.map = raster_to_packed;
-    d.dq = x.dq_local, d.dk = x.dk_local, d.dv = (char*)x.dv_local.data;
-    d.dvsb = x.dv_local.sb, d.dvsh = x.dv_local.sh, d.dvsn = x.dv_local.sn;
+    d.dq = (char*)x.dq_local, d.rope = rope_dev(x.rope);
+    d.dk = (char*)x.dk_local.data, d.dksb = x.dk_local.sb, d.dksh = x.dk_local.sh, d.dksn = x.dk_local.sn;
+    d.dv = (char*)x.dv_local.data, d.dvsb = x.dv_local.sb, d.dvsh = x.dv_local.sh, d.dvsn = x.dv_local.sn;
     d.scale = 1.f / sqrtf((float)x.head_dim);
     d.scale_log2 = kLog2e * d.scale;
     hipStream_t s = as_stream(stream);

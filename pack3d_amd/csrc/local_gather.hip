@@ -108,7 +108,7 @@ struct GDev {
     const char *q, *kl, *vl;
     int64_t qsb, qsh, qsn, ksb, ksh, ksn, vsb, vsh, vsn;
     const int32_t* nb;  // [N, W] (query kernels) or the reverse table [N, W] (key kernel)
-    RopeDev rope;       // forward: rotation of q on load
+    RopeDev rope;       // rotation of q on load (forward), of dk back (key kernel)
     const float* sl;
     char* y;
     int64_t ysb, ysh, ysn;
@@ -116,10 +116,9 @@ struct GDev {
     float* lse_l;    // forward output (optional) / backward input: [B,H,N]
     const char* dol;      // backward: dO_L [B,H,N,D] storage type
     const float* delta;   // backward: Delta_L [B,H,N]
-    float* dq;            // backward: [B,H,N,D] fp32
-    float* dk;            // backward: [B,G,N,D] fp32
-    char* dv;             // backward: view, storage type
-    int64_t dvsb, dvsh, dvsn;
+    char* dq;             // backward: [B,H,N,D] storage type, rotated space
+    char *dk, *dv;        // backward: views, storage type; dk rotated back
+    int64_t dksb, dksh, dksn, dvsb, dvsh, dvsn;
     float scale_log2;  // log2(e) / sqrt(D)
     float scale;       // 1 / sqrt(D)
 };
@@ -291,16 +290,14 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_gather_dq(GDev a) {
         }
     }
     if (!sl.ok) return;
-    float* dq = a.dq + qi * D;
+    T* dq = reinterpret_cast<T*>(a.dq) + qi * D;  // rounded as the pass that adds dQ_G takes it
 #pragma unroll
     for (int i = 0; i < C::PPL; ++i) {
         const int c0 = chan<C>(sl.part, i, 0);
         float o[C::EP];
 #pragma unroll
         for (int e = 0; e < C::EP; ++e) o[e] = acc[i * C::EP + e] * a.scale;
-#pragma unroll
-        for (int e = 0; e < C::EP; e += 4)
-            *reinterpret_cast<float4*>(dq + c0 + e) = float4{o[e], o[e + 1], o[e + 2], o[e + 3]};
+        store16<T>(dq + c0, o);
     }
 }
 
@@ -311,6 +308,9 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_gather_dq(GDev a) {
 template <typename T, int D>
 __global__ __launch_bounds__(64 * kWaves) void k_local_gather_dkv(GDev a) {
     typedef GCfg<T, D> C;
+    __shared__ int4 meta[D / 2];  // the rotation's pairs, for the epilogue
+    stage_pair_meta(a.rope, D, meta);
+    __syncthreads();
     const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const int part = lane % C::LPR;
     const int bg = blockIdx.y, b = bg / a.G, g = bg - b * a.G, rep = a.H / a.G;
@@ -372,7 +372,9 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_gather_dkv(GDev a) {
         }
     }
     if (!ok) return;
-    float* dko = a.dk + ((int64_t)bg * a.N + row) * D;
+    T* dko = reinterpret_cast<T*>(a.dk) + b * a.dksb + g * a.dksh + row * a.dksn;
+    int pos[3];
+    rope_position32(a.rope, (int)row, pos);
     T* dvo = reinterpret_cast<T*>(a.dv) + b * a.dvsb + g * a.dvsh + row * a.dvsn;
 #pragma unroll
     for (int i = 0; i < C::PPL; ++i) {
@@ -383,9 +385,8 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_gather_dkv(GDev a) {
             ko[e] = dk[i * C::EP + e] * a.scale;
             vo[e] = dv[i * C::EP + e];
         }
-#pragma unroll
-        for (int e = 0; e < C::EP; e += 4)
-            *reinterpret_cast<float4*>(dko + c0 + e) = float4{ko[e], ko[e + 1], ko[e + 2], ko[e + 3]};
+        rotate_back<T, C::EP>(a.rope, meta, pos, c0, ko);
+        store16<T>(dko + c0, ko);
         store16<T>(dvo + c0, vo);
     }
 }
@@ -507,9 +508,10 @@ extern "C" int p3d_local_bwd_indexed(const p3d_bwd_args* args, const int32_t* ne
     P3D_REQUIRE(neighbors && reverse && width >= 1 && width <= 128 && rwidth >= 1 && rwidth <= 128,
                 "neighbour tables must have 1..128 columns");
     P3D_REQUIRE(view_ok(x.q, es) && view_ok(x.kl, es) && view_ok(x.vl, es), "q/k/v rows must be 16-byte aligned");
-    P3D_REQUIRE(x.dol && x.lse_local && x.delta_local && x.dq_local && x.dk_local && view_ok(x.dv_local, es),
-                "null pointer argument or misaligned dv_local");
-    P3D_REQUIRE(aligned16(x.dol) && aligned16(x.dq_local) && aligned16(x.dk_local), "misaligned gradient buffers");
+    P3D_REQUIRE(x.dol && x.lse_local && x.delta_local && x.dq_local && view_ok(x.dk_local, es) && view_ok(x.dv_local, es),
+                "null pointer argument or misaligned dk_local / dv_local");
+    P3D_REQUIRE(aligned16(x.dol) && aligned16(x.dq_local), "misaligned gradient buffers");
+    P3D_REQUIRE(x.rope.table && x.rope.pairs && (x.rope.packed || x.rope.coords), "bad rope arguments");
     GDev d{};
     d.B = x.batch, d.H = x.heads, d.G = x.kv_heads, d.N = x.tokens;
     d.q = (const char*)x.q.data, d.qsb = x.q.sb, d.qsh = x.q.sh, d.qsn = x.q.sn;
@@ -518,8 +520,9 @@ extern "C" int p3d_local_bwd_indexed(const p3d_bwd_args* args, const int32_t* ne
     d.lse_l = const_cast<float*>(x.lse_local);
     d.dol = (const char*)x.dol;
     d.delta = x.delta_local;
-    d.dq = x.dq_local;
-    d.dk = x.dk_local;
+    d.rope = rope_dev(x.rope);
+    d.dq = (char*)x.dq_local;
+    d.dk = (char*)x.dk_local.data, d.dksb = x.dk_local.sb, d.dksh = x.dk_local.sh, d.dksn = x.dk_local.sn;
     d.dv = (char*)x.dv_local.data, d.dvsb = x.dv_local.sb, d.dvsh = x.dv_local.sh, d.dvsn = x.dv_local.sn;
     d.scale_log2 = kLog2e / sqrtf((float)x.head_dim);
     d.scale = 1.f / sqrtf((float)x.head_dim);

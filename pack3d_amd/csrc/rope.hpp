@@ -76,6 +76,43 @@ __device__ __forceinline__ void rope_position32(const RopeDev& r, int n, int pos
     }
 }
 
+// Gradient of EP consecutive rotated channels, starting at channel c0 (even) of
+// a row at pos, in place: each value rounded to T (the rotated operand is
+// stored in that type), then rotated back.  meta: pair_meta of every pair, in LDS.
+template <typename T, int EP>
+__device__ __forceinline__ void rotate_back(const RopeDev& r, const int4* meta, const int pos[3], int c0, float* x) {
+#pragma unroll
+    for (int e = 0; e < EP; e += 2) {
+        const int4 m = meta[(c0 + e) >> 1];
+        const float2 cs = r.table[m.x + m.y * pos[0] + m.z * pos[1] + m.w * pos[2]];
+        x[e] = to_f32(from_f32<T>(x[e]));
+        x[e + 1] = to_f32(from_f32<T>(x[e + 1]));
+        rotate_pair(x[e], x[e + 1], cs.x, -cs.y);
+    }
+}
+
+// The workgroup's pair metadata (D / 2 entries); a barrier follows before use.
+__device__ __forceinline__ void stage_pair_meta(const RopeDev& r, int D, int4* meta) {
+    for (int j = threadIdx.x; j < D / 2; j += blockDim.x) meta[j] = pair_meta(r.pairs, j);
+}
+
+// Four consecutive elements (8 or 16 bytes, aligned).
+template <typename T>
+__device__ __forceinline__ void store_quad4(T* dst, const float* v) {
+    typedef __attribute__((ext_vector_type(4))) T T4;
+    T4 o;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) o[i] = from_f32<T>(v[i]);
+    *reinterpret_cast<T4*>(dst) = o;
+}
+template <typename T>
+__device__ __forceinline__ void load_quad4(const T* src, float* v) {
+    typedef __attribute__((ext_vector_type(4))) T T4;
+    const T4 o = *reinterpret_cast<const T4*>(src);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) v[i] = to_f32(o[i]);
+}
+
 __device__ __forceinline__ void rope_apply32(const RopeDev& r, const int pos[3], int c0, float* x, int count) {
     for (int e = 0; e < count; e += 2) {
         const int32_t* p = r.pairs + 3 * ((c0 + e) >> 1);
