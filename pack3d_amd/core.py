@@ -375,7 +375,7 @@ def backward(dy, q, kl, vl, kg, vg, weight, bias, gate, sl, sg, sk, svt, sk_norm
                               b32.data_ptr(), pool_rope.struct(), sk.data_ptr(), svt.data_ptr(),
                               sk_norm_max.data_ptr())
     # One row of partials per pooling wave; all four parameter sums in one launch.
-    pool_parts = min(b * g * mp, 2048)
+    pool_parts = min(b * g * mp * geometry.pool_size, 2048)
     dwp, dbp = empty(pool_parts, d, dtype=f32), empty(pool_parts, slots, dtype=f32)
     _lib.call("p3d_pool_bwd", pool_args, bufs["dskp"].data_ptr(), bufs["dsvp"].data_ptr(), splits,
               _lib.view(dkg), _lib.view(dvg), dwp.data_ptr(), dbp.data_ptr(), pool_parts, stream)

@@ -25,6 +25,7 @@ constexpr int kNormSlots = 64;
 
 struct PoolDev {
     int B, G, N, F, V, P, M, Mp;
+    int wpi;       // waves that share an item, each taking every wpi-th of its steps
     int bps, gsz;  // fine blocks per 64-lane pooling step; lanes of a block's slot group (64 if bps is 1)
     float inv_tau, key_scale;
     const char *kg, *vg;
@@ -226,6 +227,7 @@ struct PoolRowCfg {
     static constexpr int NCH = D / 16;               // 16-channel chunks of the butterfly
     static constexpr int PPC = 16 / EP;              // pieces per chunk
     static constexpr int NACC = MF ? NT : NCH;       // per-lane partial sums
+    static_assert(NACC * 256 + 4 <= WAVE_BYTES, "a wave's sums fit in its row buffer");
     static constexpr size_t FIXED = (size_t)(D / 2) * 16 + PFN * 4 + D * 4 + 64 * 4;
 };
 
@@ -450,10 +452,12 @@ __global__ __launch_bounds__((64 * PoolRowCfg<T, D>::MAX_WAVES)) void k_pool_fwd
 
     // Item indices fit in 32 bits (checked on the host), so the wave-uniform
     // item arithmetic is 32-bit scalar code.
+    // Shared items (wpi > 1): block i takes item i, wave w its steps w, w + wpi, ...
     const unsigned total = (unsigned)a.B * a.G * a.Mp;
-    const unsigned stride = gridDim.x * waves;
-    const unsigned it0 = blockIdx.x * waves + wave;
-    if (it0 >= total) return;
+    const unsigned stride = a.wpi > 1 ? total : gridDim.x * waves;
+    const unsigned it0 = a.wpi > 1 ? blockIdx.x : blockIdx.x * waves + wave;
+    const int part = a.wpi > 1 ? wave : 0;
+    if (it0 >= total) return;  // never with shared items, whose waves meet at a barrier
 
     // Waves walk the items from the last one down (item = total - 1 - i for
     // the i-th of the walk): the projections that write kg / vg just before
@@ -493,13 +497,14 @@ __global__ __launch_bounds__((64 * PoolRowCfg<T, D>::MAX_WAVES)) void k_pool_fwd
         constexpr bool ALL_RUNS = decltype(all_runs_tag)::value;
         u32x4 pk[PPR], pv[PPR];
         unsigned it = it0;
-        int fl = 0, ns = steps_of(it);
-        int idx = row_of(it, 0);
+        int fl = part, ns = steps_of(it);
+        const bool any = fl < ns;  // a shared item may have fewer steps than waves
+        int idx = any ? row_of(it, fl) : -1;
         int pos[3];
         rope_position32(a.rope, max(idx, 0), pos);
         pool_fetch<T, D>(a, item_of(it), idx, lane, pk, pv);
-        unsigned it1 = ns > 1 ? it : it + stride;
-        int fl1 = ns > 1 ? 1 : 0;
+        unsigned it1 = fl + a.wpi < ns ? it : it + stride;
+        int fl1 = fl + a.wpi < ns ? fl + a.wpi : 0;
         int idx1 = it1 < total ? row_of(it1, fl1) : -1;
         float acc[C::NACC];
 #pragma unroll
@@ -511,7 +516,7 @@ __global__ __launch_bounds__((64 * PoolRowCfg<T, D>::MAX_WAVES)) void k_pool_fwd
         bool pending = false;
         int pend_bg = 0, pend_m = 0, pend_count = 0;
         float pend[C::NACC];
-        for (;;) {
+        if (any) for (;;) {
             // Stage this step's pieces as rows (slot s at s * RB).
 #pragma unroll
             for (int r = 0; r < PPR; ++r) {
@@ -544,8 +549,8 @@ __global__ __launch_bounds__((64 * PoolRowCfg<T, D>::MAX_WAVES)) void k_pool_fwd
             if (more) {
                 ns1 = steps_of(it1);
                 rope_position32(a.rope, max(idx1, 0), pos1);
-                it2 = fl1 + 1 < ns1 ? it1 : it1 + stride;
-                fl2 = fl1 + 1 < ns1 ? fl1 + 1 : 0;
+                it2 = fl1 + a.wpi < ns1 ? it1 : it1 + stride;
+                fl2 = fl1 + a.wpi < ns1 ? fl1 + a.wpi : 0;
                 if (it2 < total) idx2 = row_of(it2, fl2);
                 pool_fetch<T, D>(a, item_of(it1), idx1, lane, pk, pv);
             }
@@ -645,7 +650,7 @@ __global__ __launch_bounds__((64 * PoolRowCfg<T, D>::MAX_WAVES)) void k_pool_fwd
                     }
                 }
             }
-            if (fl + 1 == ns) {
+            if (fl + a.wpi >= ns) {
                 const unsigned bm = item_of(it) / a.G;
                 pending = true;
                 pend_bg = (int)(bm / a.Mp) * a.G + (int)(item_of(it) % a.G);
@@ -664,7 +669,28 @@ __global__ __launch_bounds__((64 * PoolRowCfg<T, D>::MAX_WAVES)) void k_pool_fwd
             pos[0] = pos1[0], pos[1] = pos1[1], pos[2] = pos1[2];
             it1 = it2, fl1 = fl2, idx1 = idx2;
         }
-        if (pending) store_summary<T, D>(a, pend_bg, pend_m, lane, pend_count, pend);
+        if (a.wpi == 1) {
+            if (pending) store_summary<T, D>(a, pend_bg, pend_m, lane, pend_count, pend);
+            return;
+        }
+        // Shared item: each wave leaves its sums in its own row buffer, and wave 0
+        // (which always has a step) adds them in order and stores the summary.
+        wave_lds_sync();
+        float* mine = reinterpret_cast<float*>(rows);
+        if (wave > 0) {
+#pragma unroll
+            for (int k = 0; k < C::NACC; ++k) mine[64 * k + lane] = any ? pend[k] : 0.f;
+            if (lane == 0) reinterpret_cast<int*>(mine)[64 * C::NACC] = any ? pend_count : 0;
+        }
+        __syncthreads();
+        if (wave > 0) return;
+        for (int w = 1; w < waves; ++w) {
+            const float* other = reinterpret_cast<const float*>(rows + (size_t)w * C::WAVE_BYTES);
+#pragma unroll
+            for (int k = 0; k < C::NACC; ++k) pend[k] += other[64 * k + lane];
+            pend_count += reinterpret_cast<const int*>(other)[64 * C::NACC];
+        }
+        store_summary<T, D>(a, pend_bg, pend_m, lane, pend_count, pend);
     };
     if constexpr (C::MF) {
         if (runs == (1u << PPR) - 1u) {
@@ -743,7 +769,11 @@ __global__ __launch_bounds__(256) void k_pool_bwd(PoolDev a, PoolBwdDev bd) {
         for (int c = 0; c < CPD; ++c) dwacc[j][c] = 0.f;
     float dbacc = 0.f;
     const unsigned wid = blockIdx.x * waves + wave;
-    for (unsigned item = wid; item < total; item += stride) {
+    for (unsigned vi = wid; vi < total * a.wpi; vi += stride) {
+        // A shared item's waves take its steps in turn (each forms its gradient
+        // factors g_k, g_v itself).
+        const unsigned item = vi / a.wpi;
+        const int part = (int)(vi - item * a.wpi);
         const int g = (int)(item % a.G);
         const unsigned bm = item / a.G;
         const int m = (int)(bm % a.Mp), b = (int)(bm / a.Mp);
@@ -789,7 +819,7 @@ __global__ __launch_bounds__(256) void k_pool_bwd(PoolDev a, PoolBwdDev bd) {
         const T* Vv = reinterpret_cast<const T*>(a.vg) + b * a.vsb + g * a.vsh;
         T* DK = reinterpret_cast<T*>(bd.dkg.data) + b * bd.dkg.sb + g * bd.dkg.sh;
         T* DV = reinterpret_cast<T*>(bd.dvg.data) + b * bd.dvg.sb + g * bd.dvg.sh;
-        for (int fs = f0; fs < f_end; fs += a.bps) {
+        for (int fs = f0 + part * a.bps; fs < f_end; fs += a.wpi * a.bps) {
             const int idx = slot_token(fs, f_end);
             if (__ballot(idx >= 0) == 0) continue;
             int pos[3];
@@ -1010,8 +1040,19 @@ inline int pool_waves(size_t fixed, size_t per_wave) {
     return 1;
 }
 
+// Waves per item: long summaries in small numbers (16 blocks of 16 slots are 4
+// steps, 256 of them one wave per CU) are shared, until the waves fill the GPU
+// (8 per CU) or run out of steps.  256 items of 4 steps at head_dim 64: forward
+// 42 -> 22 us, backward 50 -> 34 us.
+inline int waves_per_item(const PoolDev& d, int64_t items, int cus, int most) {
+    const int steps = (int)cdiv(d.P, d.bps);
+    int w = 1;
+    while (2 * w <= steps && 2 * w <= most && items * w < 8 * (int64_t)cus) w *= 2;
+    return w;
+}
+
 template <typename T, int D>
-void launch_pool_t(const PoolDev& d, hipStream_t s) {
+void launch_pool_t(PoolDev d, hipStream_t s) {
     // As many waves per block as the LDS holds row buffers for (at most 12);
     // a persistent grid of as many blocks as stay resident, each striding
     // over the items.
@@ -1026,7 +1067,9 @@ void launch_pool_t(const PoolDev& d, hipStream_t s) {
     int waves = (int)std::min<size_t>(C::MAX_WAVES, (160 * 1024 - fixed) / C::WAVE_BYTES);
     // Few items (long summaries: pool_size 16 gives 16 fine blocks each):
     // fewer waves per block, so that the blocks reach every compute unit.
-    while (waves > 1 && cdiv(items, waves) < cus) waves >>= 1;
+    d.wpi = waves_per_item(d, items, cus, waves);
+    if (d.wpi > 1) waves = d.wpi;
+    while (d.wpi == 1 && waves > 1 && cdiv(items, waves) < cus) waves >>= 1;
     const size_t smem = fixed + (size_t)C::WAVE_BYTES * waves;
     if (tab_lds)
         (void)hipOccupancyMaxActiveBlocksPerMultiprocessor(&per_cu, k_pool_fwd<T, D, true>, 64 * waves, smem);
@@ -1036,7 +1079,7 @@ void launch_pool_t(const PoolDev& d, hipStream_t s) {
     const int64_t needed = cdiv(items, waves);
     // Equal shares: the fewest rounds that cover every item, spread evenly.
     const int64_t rounds = cdiv(needed, resident);
-    const unsigned blocks = (unsigned)cdiv(needed, rounds);
+    const unsigned blocks = d.wpi > 1 ? (unsigned)items : (unsigned)cdiv(needed, rounds);
     if (tab_lds)
         k_pool_fwd<T, D, true><<<blocks, 64 * waves, smem, s>>>(d);
     else
@@ -1088,6 +1131,7 @@ int fill_pool(const p3d_pool_args* args, PoolDev& d) {
     d.P = a.pool_size;
     d.bps = (a.slots <= 32 && (a.slots & (a.slots - 1)) == 0) ? 64 / a.slots : 1;
     d.gsz = d.bps == 1 ? 64 : a.slots;
+    d.wpi = 1;
     d.M = a.summaries;
     d.Mp = (int)cdiv(a.summaries, 32) * 32;
     P3D_REQUIRE((int64_t)a.batch * a.kv_heads * d.Mp < ((int64_t)1 << 31), "batch * kv_heads * summaries too large");
@@ -1109,7 +1153,7 @@ int fill_pool(const p3d_pool_args* args, PoolDev& d) {
 }
 
 template <typename T, int D>
-void launch_pool_bwd_t(const PoolDev& d, const PoolBwdDev& bd, int64_t items, hipStream_t s) {
+void launch_pool_bwd_t(PoolDev d, const PoolBwdDev& bd, int64_t items, hipStream_t s) {
     const bool tab_lds = d.table_entries * 8 <= kTableLdsBytes;
     const size_t tab_bytes = tab_lds ? (size_t)((d.table_entries * 2 + 3) & ~3) * 4 : 0;
     const size_t fixed = (size_t)(D / 2) * 16 + (size_t)D * 4 + 64 * 4;
@@ -1118,6 +1162,8 @@ void launch_pool_bwd_t(const PoolDev& d, const PoolBwdDev& bd, int64_t items, hi
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     int waves = pool_waves(fixed + tab_bytes, per_wave);
+    d.wpi = waves_per_item(d, items, cus, 16);
+    items *= d.wpi;
     while (waves > 1 && (cdiv(items, waves) < cus || waves > bd.parts)) waves >>= 1;  // as in the forward
     const size_t smem = fixed + tab_bytes + per_wave * waves;
     if (tab_lds)
