@@ -390,7 +390,7 @@ int p3d_input_grad(const void* dq, int64_t dq_stride, int32_t q_out, const void*
  * 85,89; torch computes it as dy^T x): dw[o][i] = sum over rows n of
  * dy[n][o] x[n][i] with fp32 accumulation, written as fp32 [out_features,
  * in_features].  dy [rows, out_features] and x [rows, in_features] are
- * fp16 or bf16 with row strides ldy, ldx (elements, multiples of 8, 16-byte
+ * fp16, bf16 or fp32 with row strides ldy, ldx (elements, multiples of 8, 16-byte
  * aligned rows).  The rows are split into `splits` ranges whose fp32
  * partials go to workspace [splits, out_features, in_features] and are then
  * summed in order (deterministic).  out_features a positive multiple of 8;

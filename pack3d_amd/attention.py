@@ -12,7 +12,9 @@ autocast, LayerNorm is ``linear.LayerNormTrain`` and the linear maps are
 ``linear.InputProjections`` (``p3d_project_linear``) and
 ``linear.OutputResidual`` / ``OutputResidualWide``, with weight gradients from
 ``p3d_weight_grad``; for fp32 models without autocast they are the torch
-modules (LayerNorm on the HIP kernel when no gradient is needed).  The
+modules (LayerNorm on the HIP kernel when no gradient is needed), in training
+with the linear maps as ``InputProjections`` / ``OutputResidual`` for their
+weight gradients.  The
 rotation, pooling, local and global attention and their fusion run in
 ``libpack3d_hip.so``, and so does ``x + to_out(y)`` in the no-grad fp16 /
 bf16 forward and under autocast over an fp32 input (``p3d_out_residual``;
@@ -29,7 +31,7 @@ from torch import nn
 from . import _lib
 from .core import SUPPORTED_HEAD_DIMS, ForwardPlan, _projection_views, _validate_inputs, pack3d_hip_projections
 from .linear import (GateProbability, InputProjections, LayerNormTrain, OutputResidual, OutputResidualWide,
-                     compute_dtype, layer_norm_train_supported, wide_residual_supported)
+                     compute_dtype, fp32_training, layer_norm_train_supported, wide_residual_supported)
 from .geometry import TokenLayout, blocks_consecutive
 from .rope import axial_rope, balanced_pairs, packed_rope
 
@@ -256,7 +258,11 @@ class PACK3DAttention(nn.Module):
                                          torch.float32 if torch.is_autocast_enabled("cuda") else gl.dtype)
         else:
             xn = layer_norm(self.norm, x)
-            qp, kvp, gl = self.to_q(xn), self.to_kv(xn), self.gate(xn)
+            if self._fp32_linear(x):
+                qp, kvp, gl = InputProjections.apply(xn, self.to_q.weight, self.to_kv.weight, self.gate.weight,
+                                                     self.gate.bias, torch.float32)
+            else:
+                qp, kvp, gl = self.to_q(xn), self.to_kv(xn), self.gate(xn)
             gate = gl.view(b, n, self.heads, 2).softmax(-1)[..., 1].transpose(1, 2)
         return qp, kvp, gate, res
 
@@ -295,9 +301,26 @@ class PACK3DAttention(nn.Module):
             if res is not None:  # LayerNormTrain's dt copy of x, owned by this step
                 return OutputResidual.apply(res, o, self.to_out.weight, dt, True).view(b, n, self.dim)
             return OutputResidual.apply(x.reshape(b * n, self.dim), o, self.to_out.weight, dt).view(b, n, self.dim)
+        if self._fp32_linear(x):
+            return OutputResidual.apply(x.reshape(b * n, self.dim), o, self.to_out.weight,
+                                        torch.float32).view(b, n, self.dim)
         if x.is_cuda and torch.is_autocast_enabled("cuda") and x.dtype != torch.get_autocast_dtype("cuda"):
             return x + self.to_out(o).view(b, n, self.dim)
         return torch.addmm(x.reshape(b * n, self.dim), o, self.to_out.weight.t()).view(b, n, self.dim)
+
+    def _fp32_linear(self, x):
+        """Whether fp32 training runs the linear maps as InputProjections /
+        OutputResidual: plain fp32 modules on which nothing is registered that
+        the functions would skip."""
+        mods = (self.to_q, self.to_kv, self.gate, self.to_out)
+        params = [m.weight for m in mods] + [self.gate.bias]
+        if not torch.is_grad_enabled() or any(p is None for p in params):
+            return False
+        return (any(p.requires_grad for p in (x, *params)) and fp32_training(x, params)
+                and not any(m.bias is not None for m in (self.to_q, self.to_kv, self.to_out))
+                and not nn.modules.module._has_any_global_hook()
+                and all(type(m) is nn.Linear and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
+                                                      or m._backward_pre_hooks) for m in mods))
 
     def _hip_linear(self, x):
         """Whether the linear maps run as InputProjections / OutputResidual

@@ -18,6 +18,12 @@
 // transposed reads per fragment, so nothing is transposed on the way in.
 // Each wave then multiplies its 32 x 16-token A fragment with the I / 32
 // shared x fragments: D = dy^T x, 32 rows by I columns per wave.
+//
+// fp32 takes the same tiles at 32 tokens a stage; its operands (two tokens of
+// one column per 64 lanes) are plain reads of two tile rows.  It is bound by
+// the fp32 MFMA: 18,711 tokens of to_q, to_kv and the gate at width 192 take
+// 91 us and to_out 50 us, where the library's four products, on a few dozen
+// workgroups, took 403 us.
 #include "common.hpp"
 
 namespace p3d {
@@ -26,8 +32,8 @@ namespace {
 constexpr int kWgWaves = 8;
 constexpr int kWgRows = 32 * kWgWaves;  // output rows per workgroup
 // Tokens per stage for x of 32 IT columns.
-template <int IT>
-constexpr int wg_tok() { return IT >= 4 ? 64 : 32; }
+template <typename T, int IT>
+constexpr int wg_tok() { return sizeof(T) == 2 && IT >= 4 ? 64 : 32; }
 constexpr int kWgTokMax = 64;
 constexpr int kWgMaxCols = 256;  // input columns per workgroup
 
@@ -35,7 +41,11 @@ constexpr int kWgMaxCols = 256;  // input columns per workgroup
 // stride in dwords is 16 mod 32, so the four consecutive rows that a 16-lane
 // block reads through one transposed load start in four distinct 16-bank
 // ranges; rows stay 16-byte aligned.
-constexpr int tile_stride(int w) { return w + 2 * ((16 - (w / 2) % 32 + 32) % 32); }
+// fp32: 32 mod 64 dwords, so that the two rows of a fragment cover the banks.
+template <typename T>
+constexpr int tile_stride(int w) {
+    return sizeof(T) == 2 ? w + 2 * ((16 - (w / 2) % 32 + 32) % 32) : w + (32 - w % 64 + 64) % 64;
+}
 
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef short v8s __attribute__((ext_vector_type(8)));
@@ -59,8 +69,13 @@ __device__ __forceinline__ typename Mma<T>::Frag frag_tr(const T* tile, int stri
     return __builtin_bit_cast(typename Mma<T>::Frag, v);
 }
 
-template <int IT>
-constexpr int wgrad_stage_elems() { return wg_tok<IT>() * (tile_stride(kWgRows) + tile_stride(32 * IT)); }
+template <>
+__device__ __forceinline__ float frag_tr<float>(const float* tile, int stride, int k0, int c0, int lane) {
+    return tile[(k0 + (lane >> 5)) * stride + c0 + (lane & 31)];
+}
+
+template <typename T, int IT>
+constexpr int wgrad_stage_elems() { return wg_tok<T, IT>() * (tile_stride<T>(kWgRows) + tile_stride<T>(32 * IT)); }
 
 // dy as up to three column blocks of output rows: rows [0, end[0]) from
 // src[0], [end[0], end[1]) from src[1], [end[1], O) from src[2], each with its
@@ -77,19 +92,20 @@ struct WgSrc {
 // spread evenly over the row blocks, so that a last block of a few rows does
 // not cost a whole workgroup's pass) and input columns [blockIdx.z * I, + I)
 // of I_total, written to part[blockIdx.y][o][blockIdx.z * I + i].  Two
-// stages of dynamic LDS (2 * wgrad_stage_elems<IT>() elements).
+// stages of dynamic LDS (2 * wgrad_stage_elems<T, IT>() elements).
 template <typename T, int IT>
 __global__ __launch_bounds__(64 * kWgWaves) void k_wgrad(WgSrc<T> dy, const T* x, int64_t ldx, float* part,
                                                         int64_t rows, int O, int rpb, int64_t per, int I_total) {
     typedef Mma<T> M;
     constexpr int I = 32 * IT;
-    constexpr int SA = tile_stride(kWgRows), SB = tile_stride(I);
-    constexpr int STAGE = wgrad_stage_elems<IT>();         // elements
-    constexpr int kWgTok = wg_tok<IT>();
-    constexpr int PA = kWgTok * (kWgRows / 8) / (64 * kWgWaves);            // dy pieces per thread
-    constexpr int BP = kWgTok * (I / 8);                                     // x pieces per stage
+    constexpr int EP = Piece<T>::N;
+    constexpr int SA = tile_stride<T>(kWgRows), SB = tile_stride<T>(I);
+    constexpr int STAGE = wgrad_stage_elems<T, IT>();      // elements
+    constexpr int kWgTok = wg_tok<T, IT>();
+    constexpr int PA = kWgTok * (kWgRows / EP) / (64 * kWgWaves);           // dy pieces per thread
+    constexpr int BP = kWgTok * (I / EP);                                    // x pieces per stage
     constexpr int PB = (BP + 64 * kWgWaves - 1) / (64 * kWgWaves);           // x pieces per thread
-    static_assert(PA * 64 * kWgWaves == kWgTok * (kWgRows / 8), "dy stage pieces must divide evenly");
+    static_assert(PA * 64 * kWgWaves == kWgTok * (kWgRows / EP), "dy stage pieces must divide evenly");
     extern __shared__ __align__(16) unsigned char wg_smem[];
     T* lds = reinterpret_cast<T*>(wg_smem);
     const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 5;
@@ -102,9 +118,9 @@ __global__ __launch_bounds__(64 * kWgWaves) void k_wgrad(WgSrc<T> dy, const T* x
     auto fetch = [&](int64_t t0) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < PA; ++i) {
-            const int p = tid + i * 64 * kWgWaves, r = p / (kWgRows / 8), c = (p % (kWgRows / 8)) * 8;
+            const int p = tid + i * 64 * kWgWaves, r = p / (kWgRows / EP), c = (p % (kWgRows / EP)) * EP;
             const int64_t n = t0 + r;
-            const int o = ob + c;  // 8 rows of one source (the blocks are multiples of 8)
+            const int o = ob + c;  // a piece of one source (the blocks are multiples of 8)
             const int sel = o < dy.end[0] ? 0 : (o < dy.end[1] ? 1 : 2);
             const int o_src = o - (sel == 0 ? 0 : dy.end[sel - 1]);
             ra[i] = u32x4{0, 0, 0, 0};
@@ -113,7 +129,7 @@ __global__ __launch_bounds__(64 * kWgWaves) void k_wgrad(WgSrc<T> dy, const T* x
         }
 #pragma unroll
         for (int i = 0; i < PB; ++i) {
-            const int p = tid + i * 64 * kWgWaves, r = p / (I / 8), c = (p % (I / 8)) * 8;
+            const int p = tid + i * 64 * kWgWaves, r = p / (I / EP), c = (p % (I / EP)) * EP;
             const int64_t n = t0 + r;
             rb[i] = u32x4{0, 0, 0, 0};
             if (p < BP && n < n1) rb[i] = *reinterpret_cast<const u32x4*>(x + n * ldx + c);
@@ -122,12 +138,12 @@ __global__ __launch_bounds__(64 * kWgWaves) void k_wgrad(WgSrc<T> dy, const T* x
     auto stage = [&](T* st) __attribute__((always_inline)) {
 #pragma unroll
         for (int i = 0; i < PA; ++i) {
-            const int p = tid + i * 64 * kWgWaves, r = p / (kWgRows / 8), c = (p % (kWgRows / 8)) * 8;
+            const int p = tid + i * 64 * kWgWaves, r = p / (kWgRows / EP), c = (p % (kWgRows / EP)) * EP;
             *reinterpret_cast<u32x4*>(st + r * SA + c) = ra[i];
         }
 #pragma unroll
         for (int i = 0; i < PB; ++i) {
-            const int p = tid + i * 64 * kWgWaves, r = p / (I / 8), c = (p % (I / 8)) * 8;
+            const int p = tid + i * 64 * kWgWaves, r = p / (I / EP), c = (p % (I / EP)) * EP;
             if (p < BP) *reinterpret_cast<u32x4*>(st + kWgTok * SA + r * SB + c) = rb[i];
         }
     };
@@ -150,11 +166,11 @@ __global__ __launch_bounds__(64 * kWgWaves) void k_wgrad(WgSrc<T> dy, const T* x
             // of the dy tile: no branch around the MFMAs, whose accumulators would
             // otherwise be copied between register files at the join.
 #pragma unroll
-            for (int ks = 0; ks < kWgTok / 16; ++ks) {
-                const typename M::Frag fa = frag_tr<T>(cur, SA, 16 * ks, 32 * wave, lane);
+            for (int ks = 0; ks < kWgTok / M::KS; ++ks) {
+                const typename M::Frag fa = frag_tr<T>(cur, SA, M::KS * ks, 32 * wave, lane);
 #pragma unroll
                 for (int t = 0; t < IT; ++t)
-                    acc[t] = M::mfma(fa, frag_tr<T>(cur + kWgTok * SA, SB, 16 * ks, 32 * t, lane), acc[t]);
+                    acc[t] = M::mfma(fa, frag_tr<T>(cur + kWgTok * SA, SB, M::KS * ks, 32 * t, lane), acc[t]);
             }
             if (more) stage(lds + (buf ^ 1) * STAGE);
             __syncthreads();
@@ -234,7 +250,7 @@ int launch_wgrad(const WgSrc<T>& dy, const void* x, int64_t ldx, void* dw, int d
     switch (Ib / 32) {
 #define CASE(IT)                                                                                                  \
     case IT:                                                                                                      \
-        k_wgrad<T, IT><<<grid, 64 * kWgWaves, 2 * wgrad_stage_elems<IT>() * sizeof(T), s>>>(                      \
+        k_wgrad<T, IT><<<grid, 64 * kWgWaves, 2 * wgrad_stage_elems<T, IT>() * sizeof(T), s>>>(                   \
             dy, (const T*)x, ldx, part, rows, O, rpb, per, I);                                                         \
         break;
         CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
@@ -258,7 +274,7 @@ extern "C" int p3d_weight_grad(const void* dy, int64_t ldy, const void* x, int64
                                int64_t rows, int32_t out_features, int32_t in_features, int32_t splits, int32_t dtype,
                                void* stream) {
     P3D_REQUIRE(dy && x && dw && workspace, "null pointer argument");
-    P3D_REQUIRE(dtype == P3D_F16 || dtype == P3D_BF16, "dtype must be fp16 or bf16");
+    P3D_REQUIRE(dtype >= P3D_F32 && dtype <= P3D_BF16, "unknown dtype");
     P3D_REQUIRE(rows >= 1 && splits >= 1, "need at least one row and one split");
     P3D_REQUIRE(out_features >= 8 && out_features % 8 == 0, "out_features must be a positive multiple of 8");
     P3D_REQUIRE(wgrad_cols_ok(in_features),
@@ -267,6 +283,11 @@ extern "C" int p3d_weight_grad(const void* dy, int64_t ldy, const void* x, int64
                 "row strides must cover the rows and keep 16-byte alignment");
     P3D_REQUIRE(aligned16(dy) && aligned16(x), "dy and x must be 16-byte aligned");
     P3D_REQUIRE(cdiv(out_features, kWgRows) < 65536 && splits < 65536, "grid too large");
+    if (dtype == P3D_F32) {
+        const WgSrc<float> src{{(const float*)dy, nullptr, nullptr}, {ldy, 0, 0}, {out_features, out_features}};
+        return launch_wgrad<float>(src, x, ldx, dw, P3D_F32, workspace, rows, out_features, in_features, splits,
+                                   as_stream(stream));
+    }
     if (dtype == P3D_F16) {
         const WgSrc<_Float16> src{{(const _Float16*)dy, nullptr, nullptr}, {ldy, 0, 0}, {out_features, out_features}};
         return launch_wgrad<_Float16>(src, x, ldx, dw, P3D_F32, workspace, rows, out_features, in_features, splits,
@@ -282,7 +303,7 @@ extern "C" int p3d_weight_grad3(const void* dy0, int64_t ld0, int32_t out0, cons
                                 void* dw, int32_t dw_dtype, float* workspace, int64_t rows, int32_t in_features,
                                 int32_t splits, int32_t dtype, void* stream) {
     P3D_REQUIRE(dy0 && dy1 && dy2 && x && dw && workspace, "null pointer argument");
-    P3D_REQUIRE(dtype == P3D_F16 || dtype == P3D_BF16, "dtype must be fp16 or bf16");
+    P3D_REQUIRE(dtype >= P3D_F32 && dtype <= P3D_BF16, "unknown dtype");
     P3D_REQUIRE(dw_dtype == P3D_F32 || dw_dtype == dtype, "dw is fp32 or of the inputs' type");
     P3D_REQUIRE(rows >= 1 && splits >= 1, "need at least one row and one split");
     P3D_REQUIRE(out0 >= 8 && out1 >= 8 && out2 >= 8 && out0 % 8 == 0 && out1 % 8 == 0 && out2 % 8 == 0 &&
@@ -296,6 +317,12 @@ extern "C" int p3d_weight_grad3(const void* dy0, int64_t ld0, int32_t out0, cons
     P3D_REQUIRE(aligned16(dy0) && aligned16(dy1) && aligned16(dy2) && aligned16(x), "dy and x must be 16-byte aligned");
     const int O = out0 + out1 + out2;
     P3D_REQUIRE(cdiv(O, kWgRows) < 65536 && splits < 65536, "grid too large");
+    if (dtype == P3D_F32) {
+        const WgSrc<float> src{{(const float*)dy0, (const float*)dy1, (const float*)dy2}, {ld0, ld1, ld2},
+                               {out0, out0 + out1}};
+        return launch_wgrad<float>(src, x, ldx, dw, dw_dtype, workspace, rows, O, in_features, splits,
+                                   as_stream(stream));
+    }
     if (dtype == P3D_F16) {
         const WgSrc<_Float16> src{{(const _Float16*)dy0, (const _Float16*)dy1, (const _Float16*)dy2},
                                   {ld0, ld1, ld2},

@@ -1,5 +1,5 @@
-"""The layer's linear maps under autograd in fp16 / bf16, with the weight
-gradients from the HIP kernel ``p3d_weight_grad``.
+"""The layer's linear maps under autograd, with the weight gradients from the
+HIP kernel ``p3d_weight_grad``.
 
 For y = x W^T the weight gradient dW = dy^T x contracts over every token
 (262,144 at 64^3) into a small matrix; the library GEMM runs it with a
@@ -33,14 +33,27 @@ WORKGROUPS = 256
 MIN_ROWS_PER_SPLIT = 512
 
 
-def splits_for(rows, out_features, in_features):
+def splits_for(rows, out_features, in_features, dtype=torch.bfloat16):
     blocks = -(-out_features // WG_ROWS) * max(1, in_features // WG_COLS)
     # Small gradients may be split finer, as long as a split's partials (written
     # and read, 8 bytes an element) stay below the bytes of its rows of dy and
     # x: 4,096 rows of 64 x 64 run on 32 workgroups instead of 8 (21 -> 9 us).
     rows_per = max(128, min(MIN_ROWS_PER_SPLIT,
                             4 * out_features * in_features // (out_features + in_features)))
+    # The fp32 products take 16 times as long and the partials no longer: 128
+    # rows fill the GPU (18,711 rows of 192 x 192 on 147 workgroups instead of
+    # 42, 105 -> 50 us; 968 x 192 on 236 instead of 132, 147 -> 91 us).
+    if dtype == torch.float32:
+        rows_per = 128
     return max(1, min(max(1, WORKGROUPS // blocks), rows // rows_per))
+
+
+def fp32_training(x, params):
+    """Whether fp32 training takes InputProjections and OutputResidual (for their
+    weight gradients; LayerNorm and the gate stay torch's): a CUDA fp32 x and
+    fp32 parameters, without autocast."""
+    return (x.is_cuda and x.dtype == torch.float32 and not torch.is_autocast_enabled("cuda")
+            and all(type(p) in (torch.Tensor, torch.nn.Parameter) and p.dtype == torch.float32 for p in params))
 
 
 def compute_dtype(x):
@@ -118,20 +131,26 @@ def project_linear(x16, ws, bg):
     return q, kv, gl
 
 
+def _differentiated(*tensors):
+    """fp32 backward passes under create_graph stay on torch ops, as they were."""
+    return (torch.is_grad_enabled() and tensors[0].dtype == torch.float32
+            and any(t.requires_grad for t in tensors))
+
+
 def weight_grad(dy, x):
-    """dW = dy^T x in fp32 for dy [rows, out], x [rows, in] of one 16-bit type
+    """dW = dy^T x in fp32 for dy [rows, out], x [rows, in] of one type
     (``p3d_weight_grad``; torch's product in fp32 where the kernel does not
-    take the shape)."""
+    take the shape, or where the gradient is itself to be differentiated)."""
     rows, out_f = dy.shape
     in_f = x.shape[1]
-    if not weight_grad_supported(out_f, in_f) or dy.dtype != x.dtype or dy.dtype not in (torch.float16,
-                                                                                           torch.bfloat16):
+    if (not weight_grad_supported(out_f, in_f) or dy.dtype != x.dtype or dy.dtype not in _lib.DTYPES
+            or _differentiated(dy, x)):
         return torch.mm(dy.t().float(), x.float())
     dy = dy if dy.stride(1) == 1 and dy.stride(0) % 8 == 0 else dy.contiguous()
     x = x if x.stride(1) == 1 and x.stride(0) % 8 == 0 else x.contiguous()
     if dy.data_ptr() % 16 or x.data_ptr() % 16:
         dy, x = dy.clone(), x.clone()
-    splits = splits_for(rows, out_f, in_f)
+    splits = splits_for(rows, out_f, in_f, dy.dtype)
     dw = torch.empty(out_f, in_f, dtype=torch.float32, device=dy.device)
     work = torch.empty(splits, out_f, in_f, dtype=torch.float32, device=dy.device)
     _lib.call("p3d_weight_grad", dy.data_ptr(), dy.stride(0), x.data_ptr(), x.stride(0), dw.data_ptr(),
@@ -148,13 +167,13 @@ def weight_grads3(dys, x, out_dtype=torch.float32):
     rows, in_f = x.shape
     outs = [dy.shape[1] for dy in dys]
     dt = x.dtype
-    if (dt not in (torch.float16, torch.bfloat16) or not all(weight_grad_supported(o, in_f) for o in outs)
+    if (dt not in _lib.DTYPES or not all(weight_grad_supported(o, in_f) for o in outs) or _differentiated(x, *dys)
             or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16
             or any(dy.dtype != dt or dy.shape[0] != rows or dy.stride(1) != 1 or dy.stride(0) % 8
                    or dy.data_ptr() % 16 for dy in dys)):
         return None
     total = sum(outs)
-    splits = splits_for(rows, total, in_f)
+    splits = splits_for(rows, total, in_f, dt)
     dw = torch.empty(total, in_f, dtype=out_dtype, device=x.device)
     work = torch.empty(splits, total, in_f, dtype=torch.float32, device=x.device)
     _lib.call("p3d_weight_grad3", dys[0].data_ptr(), dys[0].stride(0), outs[0], dys[1].data_ptr(), dys[1].stride(0),
@@ -316,9 +335,9 @@ class LayerNormTrain(torch.autograd.Function):
 
 
 class InputProjections(torch.autograd.Function):
-    """(x Wq^T, x Wkv^T, x Wg^T + bg) of the normalised tokens x in the 16-bit
-    type dt (attention.py:64-67,85): x is rounded to dt once and shared by
-    the three products; the backward returns dx in x's dtype (the three
+    """(x Wq^T, x Wkv^T, x Wg^T + bg) of the normalised tokens x in the type
+    dt, 16-bit, or fp32 for an fp32 model (attention.py:64-67,85): x is rounded
+    to dt once and shared by the three products; the backward returns dx in x's dtype (the three
     input gradients summed in fp32) and fp32 weight gradients cast to the
     parameters' dtypes."""
 
@@ -333,7 +352,9 @@ class InputProjections(torch.autograd.Function):
             q = torch.mm(x16, ws[0].t())
             kv = torch.mm(x16, ws[1].t())
             gl = torch.addmm(bg16, x16, ws[2].t())
-        ctx.save_for_backward(x16, *ws)
+        # x itself where it is what the products read, so that a differentiated
+        # backward reaches it.
+        ctx.save_for_backward(x if x.dtype == dt and x.is_contiguous() else x16, *ws)
         ctx.meta = (x.shape, x.dtype, wq.dtype, wkv.dtype, wg.dtype, bg.dtype)
         lead = x.shape[:-1]
         return q.view(*lead, -1), kv.view(*lead, -1), gl.view(*lead, -1)
@@ -341,11 +362,12 @@ class InputProjections(torch.autograd.Function):
     @staticmethod
     def backward(ctx, dq, dkv, dgl):
         x16, wq, wkv, wg = ctx.saved_tensors
+        x16 = _rows(x16)
         shape, x_dt, wq_dt, wkv_dt, wg_dt, bg_dt = ctx.meta
         # dx = dq Wq + dkv Wkv + dgl Wg: for an fp32 x (autocast) the three
         # products are summed in fp32 as autograd would; for a 16-bit x the
         # GEMMs accumulate into one buffer of that type.
-        wide = x_dt == torch.float32
+        wide = x_dt == torch.float32 and x16.dtype != x_dt
         dys = [None if dy is None else _rows(dy).to(x16.dtype) for dy in (dq, dkv, dgl)]
         # One kernel for the three products where it takes the shapes (16-bit x).
         dx = None if wide else input_grad(dys, (wq, wkv, wg))
@@ -354,7 +376,8 @@ class InputProjections(torch.autograd.Function):
             dx = torch.zeros(x16.shape, dtype=torch.float32, device=x16.device)
         # The three weight gradients from one pass over x16 where the kernel takes them.
         same = x16.dtype if wq_dt == wkv_dt == wg_dt == x16.dtype else torch.float32
-        dws = None if any(dy is None for dy in dys) else weight_grads3(dys, x16, same)
+        every = all(ctx.needs_input_grad[1:4]) and not any(dy is None for dy in dys)
+        dws = weight_grads3(dys, x16, same) if every else None
         grads = []
         for i, (dy, w, w_dt) in enumerate(zip(dys, (wq, wkv, wg), (wq_dt, wkv_dt, wg_dt))):
             if dy is None:
@@ -365,7 +388,11 @@ class InputProjections(torch.autograd.Function):
             elif dx is None:
                 dx = torch.mm(dy, w)
             elif not fused:
-                dx.addmm_(dy, w)  # in place: no copy of dx into a new result
+                # in place: no copy of dx into a new result
+                dx = torch.addmm(dx, dy, w) if _differentiated(dy, w) else dx.addmm_(dy, w)
+            if not ctx.needs_input_grad[1 + i]:
+                grads.append(None)
+                continue
             grads.append((weight_grad(dy, x16) if dws is None else dws[i]).to(w_dt))
         if dx is None:
             dx = torch.zeros(x16.shape, dtype=x16.dtype, device=x16.device)
@@ -412,7 +439,7 @@ class OutputResidualWide(torch.autograd.Function):
 
 
 class OutputResidual(torch.autograd.Function):
-    """x + y Wo^T in the 16-bit type dt (attention.py:89 with a 16-bit x):
+    """x + y Wo^T in the type dt (attention.py:89 with an x of that type):
     x [rows, dim], y [rows, k].  The product accumulates into the residual in
     place: into x itself when the caller owns it (x_owned: x is already a dt
     copy, such as the one LayerNormTrain returns; it is marked dirty and
@@ -447,4 +474,4 @@ class OutputResidual(torch.autograd.Function):
         d16 = dout.to(y16.dtype)
         dy = torch.mm(d16, wo16).to(y_dt)
         dx = None if x_dt is None else dout.to(x_dt)
-        return dx, dy, weight_grad(d16, y16).to(wo_dt), None, None
+        return dx, dy, weight_grad(d16, y16).to(wo_dt) if ctx.needs_input_grad[2] else None, None, None
