@@ -6,46 +6,53 @@
 // and each writes an fp32 partial; a second kernel sums the partials in a
 // fixed order (deterministic).
 //
-// A workgroup owns 256 output rows (8 waves x 32) and a token range, taken
-// TOK tokens per stage.  A stage of dy [TOK tokens x 256 rows] and of x [TOK
-// tokens x I] is loaded with 16-byte row pieces (the next stage in flight
-// while the current one is multiplied) and stored row-major in LDS.  The
-// pass is bound by the bytes in flight per CU: from I = 128 on, one
-// workgroup fits per CU and its stages take 64 tokens (32-token stages ran
-// 15% slower at I = 192); narrower x keeps 32-token stages and several
-// workgroups per CU.  The MFMA operands need 8 consecutive tokens of one column per lane; they come
-// out of the row-major tiles through ds_read_b64_tr_b16, two 8-byte
-// transposed reads per fragment, so nothing is transposed on the way in.
+// A workgroup owns 256 output rows (8 waves x 32) and a token range, taken 32
+// tokens per stage (16 in fp32).  The pass is bound by the bytes in flight per
+// CU, so the stages of dy [tokens x 256 rows] and of x [tokens x I] are copied to
+// LDS by DMA, two stages ahead of the one that is multiplied: through registers,
+// a stage at a time, 262,144 tokens took 253 us for 968 x 192 and 64 us for
+// 192 x 192, now 153 and 46 us (32,768 tokens of 1,040 x 512: 90 -> 65 us).
+// Three and four buffers of 32 tokens and two of 64 are alike.  The MFMA
+// operands need 8 consecutive tokens of one column per lane; they come out of the
+// row-major tiles through ds_read_b64_tr_b16, two 8-byte transposed reads per
+// fragment, so nothing is transposed on the way in.
 // Each wave then multiplies its 32 x 16-token A fragment with the I / 32
 // shared x fragments: D = dy^T x, 32 rows by I columns per wave.
 //
-// fp32 takes the same tiles at 32 tokens a stage; its operands (two tokens of
-// one column per 64 lanes) are plain reads of two tile rows.  It is bound by
+// In fp32 the operands (two tokens of one column per 64 lanes) are plain reads of
+// two tile rows.  It is bound by
 // the fp32 MFMA: 18,711 tokens of to_q, to_kv and the gate at width 192 take
 // 91 us and to_out 50 us, where the library's four products, on a few dozen
 // workgroups, took 403 us.
-#include "common.hpp"
+#include "attn_common.hpp"
 
 namespace p3d {
 namespace {
 
 constexpr int kWgWaves = 8;
+constexpr int kWgThreads = 64 * kWgWaves;
 constexpr int kWgRows = 32 * kWgWaves;  // output rows per workgroup
-// Tokens per stage for x of 32 IT columns.
-template <typename T, int IT>
-constexpr int wg_tok() { return sizeof(T) == 2 && IT >= 4 ? 64 : 32; }
-constexpr int kWgTokMax = 64;
-constexpr int kWgMaxCols = 256;  // input columns per workgroup
+constexpr int kWgTokMax = 64;           // splits are multiples of this many tokens
+constexpr int kWgMaxCols = 256;         // input columns per workgroup
 
-// Row stride (elements of a 16-bit type) of an LDS tile w elements wide: the
-// stride in dwords is 16 mod 32, so the four consecutive rows that a 16-lane
-// block reads through one transposed load start in four distinct 16-bank
-// ranges; rows stay 16-byte aligned.
-// fp32: 32 mod 64 dwords, so that the two rows of a fragment cover the banks.
+// Tiles of one stage in LDS: TOK rows of 256 dy columns, then TOK rows of x's
+// columns rounded up to 128 or 256, in 16-byte pieces without padding (the DMA
+// writes 64 pieces of a wave in a row).  Piece c of row r lies at c ^ swizzle(r),
+// so that the rows a fragment reads together start in different banks: four rows
+// of 64 bytes (16-bit types), two of 128 (fp32).
+template <typename T, int IT>
+struct WgCfg {
+    static constexpr int EP = Piece<T>::N;
+    static constexpr int TOK = sizeof(T) == 2 ? 32 : 16;
+    static constexpr int BUFS = 3;
+    static constexpr int AP = kWgRows / EP;                // pieces of a dy row
+    static constexpr int XP = (IT <= 4 ? 128 : 256) / EP;  // and of an x row
+    static constexpr int NA = TOK * AP / kWgThreads, NX = TOK * XP / kWgThreads;  // copies per thread
+    static constexpr int STAGE = TOK * (AP + XP) * 16;     // bytes
+    static_assert(NA * kWgThreads == TOK * AP && NX * kWgThreads == TOK * XP, "a stage is whole copies");
+};
 template <typename T>
-constexpr int tile_stride(int w) {
-    return sizeof(T) == 2 ? w + 2 * ((16 - (w / 2) % 32 + 32) % 32) : w + (32 - w % 64 + 64) % 64;
-}
+__device__ __forceinline__ int wg_swizzle(int row) { return sizeof(T) == 2 ? 4 * (row & 3) : 8 * (row & 1); }
 
 typedef short v4s __attribute__((ext_vector_type(4)));
 typedef short v8s __attribute__((ext_vector_type(8)));
@@ -57,25 +64,24 @@ typedef short v8s __attribute__((ext_vector_type(8)));
 // B + 4a + e of each 16-lane block element e of the 8-byte windows addressed
 // by lanes B + a + 4j (j = 0..3) as its values j, so lane L addresses row
 // k0 + 8 (L / 32) + (L % 16) / 4 (four rows further for the second read) at
-// column c0 + 16 ((L / 16) % 2) + 4 (L % 4).
+// column c0 + 16 ((L / 16) % 2) + 4 (L % 4).  pieces: of a tile row.
 template <typename T>
-__device__ __forceinline__ typename Mma<T>::Frag frag_tr(const T* tile, int stride, int k0, int c0, int lane) {
+__device__ __forceinline__ typename Mma<T>::Frag frag_tr(const T* tile, int pieces, int k0, int c0, int lane) {
     const int row = k0 + 8 * (lane >> 5) + ((lane & 15) >> 2);
     const int col = c0 + 16 * ((lane >> 4) & 1) + 4 * (lane & 3);
+    const T* p = tile + (row * pieces + ((col / 8) ^ wg_swizzle<T>(row))) * 8 + col % 8;
     typedef __attribute__((address_space(3))) v4s* lds_v4s;
-    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(tile + row * stride + col));
-    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(tile + (row + 4) * stride + col));
+    const v4s lo = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)p);
+    const v4s hi = __builtin_amdgcn_ds_read_tr16_b64_v4i16((lds_v4s)(p + 4 * pieces * 8));  // same swizzle
     const v8s v = {lo[0], lo[1], lo[2], lo[3], hi[0], hi[1], hi[2], hi[3]};
     return __builtin_bit_cast(typename Mma<T>::Frag, v);
 }
 
 template <>
-__device__ __forceinline__ float frag_tr<float>(const float* tile, int stride, int k0, int c0, int lane) {
-    return tile[(k0 + (lane >> 5)) * stride + c0 + (lane & 31)];
+__device__ __forceinline__ float frag_tr<float>(const float* tile, int pieces, int k0, int c0, int lane) {
+    const int row = k0 + (lane >> 5), col = c0 + (lane & 31);
+    return tile[(row * pieces + ((col / 4) ^ wg_swizzle<float>(row))) * 4 + col % 4];
 }
-
-template <typename T, int IT>
-constexpr int wgrad_stage_elems() { return wg_tok<T, IT>() * (tile_stride<T>(kWgRows) + tile_stride<T>(32 * IT)); }
 
 // dy as up to three column blocks of output rows: rows [0, end[0]) from
 // src[0], [end[0], end[1]) from src[1], [end[1], O) from src[2], each with its
@@ -87,64 +93,81 @@ struct WgSrc {
     int end[2];
 };
 
-// Partial dW of token range [blockIdx.y * per, + per) for output rows
-// [blockIdx.x * rpb, + rpb) (rpb a multiple of 32, at most 256: the rows are
-// spread evenly over the row blocks, so that a last block of a few rows does
-// not cost a whole workgroup's pass) and input columns [blockIdx.z * I, + I)
-// of I_total, written to part[blockIdx.y][o][blockIdx.z * I + i].  Two
-// stages of dynamic LDS (2 * wgrad_stage_elems<T, IT>() elements).
+// The tiles of dW (row blocks x column blocks) of each token range.  by_xcd:
+// workgroups go to the eight XCDs in turn, so the tiles of a range, which read
+// the same rows of dy and x, take ids 8 apart and share one XCD's L2 (ids past
+// the last range leave at once).  32,768 rows of 1,040 x 512 (10 tiles): 71 us
+// spread over the XCDs, 65 us so; 262,144 of 968 x 192 (4 tiles): 160 and 153
+// us.  Fewer than 8 ranges would leave XCDs idle and keep the tiles spread.
+struct WgGrid {
+    int row_blocks, col_blocks, splits;
+    bool by_xcd;
+};
+
+// Partial dW of token range [split * per, + per) for output rows [ob, ob + rpb)
+// (rpb a multiple of 32, at most 256: the rows are spread evenly over the row
+// blocks, so that a last block of a few rows does not cost a whole workgroup's
+// pass) and input columns [cb * I, + I) of I_total, written to
+// part[split][o][cb * I + i].
+// BUFS stages of dynamic LDS.
 template <typename T, int IT>
-__global__ __launch_bounds__(64 * kWgWaves) void k_wgrad(WgSrc<T> dy, const T* x, int64_t ldx, float* part,
-                                                        int64_t rows, int O, int rpb, int64_t per, int I_total) {
+__global__ __launch_bounds__(kWgThreads) void k_wgrad(WgSrc<T> dy, const T* x, int64_t ldx, float* part, int64_t rows,
+                                                      int O, int rpb, int64_t per, int I_total, WgGrid wg) {
     typedef Mma<T> M;
-    constexpr int I = 32 * IT;
-    constexpr int EP = Piece<T>::N;
-    constexpr int SA = tile_stride<T>(kWgRows), SB = tile_stride<T>(I);
-    constexpr int STAGE = wgrad_stage_elems<T, IT>();      // elements
-    constexpr int kWgTok = wg_tok<T, IT>();
-    constexpr int PA = kWgTok * (kWgRows / EP) / (64 * kWgWaves);           // dy pieces per thread
-    constexpr int BP = kWgTok * (I / EP);                                    // x pieces per stage
-    constexpr int PB = (BP + 64 * kWgWaves - 1) / (64 * kWgWaves);           // x pieces per thread
-    static_assert(PA * 64 * kWgWaves == kWgTok * (kWgRows / EP), "dy stage pieces must divide evenly");
+    typedef WgCfg<T, IT> C;
+    constexpr int I = 32 * IT, EP = C::EP, NP = C::NA + C::NX;
     extern __shared__ __align__(16) unsigned char wg_smem[];
-    T* lds = reinterpret_cast<T*>(wg_smem);
-    const int tid = threadIdx.x, wave = tid >> 6, lane = tid & 63, g = lane >> 5;
-    const int ob = blockIdx.x * rpb;
-    const int64_t n0 = (int64_t)blockIdx.y * per, n1 = min(rows, n0 + per);
-    x += (int64_t)blockIdx.z * I;  // this workgroup's input columns
+    const int tid = threadIdx.x, lane = tid & 63, g = lane >> 5;
+    const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+    const int tiles = wg.row_blocks * wg.col_blocks, id = blockIdx.x;
+    const int split = wg.by_xcd ? id / 8 / tiles * 8 + id % 8 : id / tiles;
+    const int tile = wg.by_xcd ? id / 8 % tiles : id % tiles;
+    if (split >= wg.splits) return;  // the whole workgroup
+    const int cb = tile / wg.row_blocks, ob = (tile - cb * wg.row_blocks) * rpb;
+    const int64_t n0 = (int64_t)split * per, n1 = min(rows, n0 + per);
+    x += (int64_t)cb * I;  // this workgroup's input columns
     const bool active = 32 * wave < rpb && ob + 32 * wave < O;  // wave-uniform
 
-    u32x4 ra[PA], rb[PB];
-    auto fetch = [&](int64_t t0) __attribute__((always_inline)) {
+    // This thread's pieces of a stage: p-th copy's row, and its source in the
+    // stage to come next (columns past the block's or x's last are read from it:
+    // they only reach output rows and columns that are not stored).
+    int prow[NP];
+    const unsigned char* src[NP];
+    int64_t step[NP];  // bytes per stage
 #pragma unroll
-        for (int i = 0; i < PA; ++i) {
-            const int p = tid + i * 64 * kWgWaves, r = p / (kWgRows / EP), c = (p % (kWgRows / EP)) * EP;
-            const int64_t n = t0 + r;
-            const int o = ob + c;  // a piece of one source (the blocks are multiples of 8)
+    for (int i = 0; i < NP; ++i) {
+        const bool isx = i >= C::NA;
+        const int L = tid + (isx ? i - C::NA : i) * kWgThreads, pieces = isx ? C::XP : C::AP;
+        prow[i] = L / pieces;
+        const int c = ((L % pieces) ^ wg_swizzle<T>(prow[i])) * EP;
+        if (isx) {
+            src[i] = reinterpret_cast<const unsigned char*>(x + (n0 + prow[i]) * ldx + min(c, I - EP));
+            step[i] = C::TOK * ldx * (int64_t)sizeof(T);
+        } else {
+            const int o = ob + min(c, min(rpb, O - ob) - EP);  // a piece of one source (the blocks are multiples of 8)
             const int sel = o < dy.end[0] ? 0 : (o < dy.end[1] ? 1 : 2);
             const int o_src = o - (sel == 0 ? 0 : dy.end[sel - 1]);
-            ra[i] = u32x4{0, 0, 0, 0};
-            if (n < n1 && c < rpb && o < O)
-                ra[i] = *reinterpret_cast<const u32x4*>(dy.src[sel] + n * dy.ld[sel] + o_src);
+            src[i] = reinterpret_cast<const unsigned char*>(dy.src[sel] + (n0 + prow[i]) * dy.ld[sel] + o_src);
+            step[i] = C::TOK * dy.ld[sel] * (int64_t)sizeof(T);
+        }
+    }
+    // Copies stage t0 .. t0 + TOK - 1 into buffer buf: by LDS DMA, or through
+    // registers with zeros past n1 where it is the range's partial last one.
+    auto issue = [&](int64_t t0, int buf) __attribute__((always_inline)) {
+        if (t0 >= n1) return;
+        if (t0 + C::TOK <= n1) {
+#pragma unroll
+            for (int i = 0; i < NP; ++i) {
+                dma_copy16(src[i], lds_address(wg_smem) + buf * C::STAGE + (i * kWgThreads + wave * 64) * 16);
+                src[i] += step[i];
+            }
+            return;
         }
 #pragma unroll
-        for (int i = 0; i < PB; ++i) {
-            const int p = tid + i * 64 * kWgWaves, r = p / (I / EP), c = (p % (I / EP)) * EP;
-            const int64_t n = t0 + r;
-            rb[i] = u32x4{0, 0, 0, 0};
-            if (p < BP && n < n1) rb[i] = *reinterpret_cast<const u32x4*>(x + n * ldx + c);
-        }
-    };
-    auto stage = [&](T* st) __attribute__((always_inline)) {
-#pragma unroll
-        for (int i = 0; i < PA; ++i) {
-            const int p = tid + i * 64 * kWgWaves, r = p / (kWgRows / EP), c = (p % (kWgRows / EP)) * EP;
-            *reinterpret_cast<u32x4*>(st + r * SA + c) = ra[i];
-        }
-#pragma unroll
-        for (int i = 0; i < PB; ++i) {
-            const int p = tid + i * 64 * kWgWaves, r = p / (I / EP), c = (p % (I / EP)) * EP;
-            if (p < BP) *reinterpret_cast<u32x4*>(st + kWgTok * SA + r * SB + c) = rb[i];
+        for (int i = 0; i < NP; ++i) {
+            u32x4 v{0, 0, 0, 0};
+            if (t0 + prow[i] < n1) v = *reinterpret_cast<const u32x4*>(src[i]);
+            *reinterpret_cast<u32x4*>(wg_smem + buf * C::STAGE + (i * kWgThreads + tid) * 16) = v;
         }
     };
 
@@ -153,33 +176,37 @@ __global__ __launch_bounds__(64 * kWgWaves) void k_wgrad(WgSrc<T> dy, const T* x
     for (int t = 0; t < IT; ++t)
 #pragma unroll
         for (int r = 0; r < 16; ++r) acc[t][r] = 0.f;
-    if (n0 < n1) {
-        fetch(n0);
-        stage(lds);
+    constexpr int AHEAD = C::BUFS - 1;  // stages being copied while one is multiplied
+#pragma unroll
+    for (int i = 0; i < AHEAD; ++i) issue(n0 + i * C::TOK, i);
+    int buf = 0;
+    for (int64_t t0 = n0; t0 < n1; t0 += C::TOK) {
+        // This wave's copies of the stage have landed (those of the stages after
+        // it are still counted if all of them are whole), and after the barrier
+        // every wave's; every wave is also done with the stage before, whose buffer
+        // is copied into next.
+        if (t0 + AHEAD * C::TOK <= n1)
+            asm volatile("s_waitcnt vmcnt(%0) lgkmcnt(0)" ::"n"((AHEAD - 1) * NP) : "memory");
+        else
+            dma_wait();
         __syncthreads();
-        int buf = 0;
-        for (int64_t t0 = n0; t0 < n1; t0 += kWgTok) {
-            const bool more = t0 + kWgTok < n1;
-            if (more) fetch(t0 + kWgTok);
-            const T* cur = lds + buf * STAGE;
-            // Waves past the block's last output row multiply the zero columns
-            // of the dy tile: no branch around the MFMAs, whose accumulators would
-            // otherwise be copied between register files at the join.
+        issue(t0 + AHEAD * C::TOK, (buf + AHEAD) % C::BUFS);
+        const T* cur = reinterpret_cast<const T*>(wg_smem + buf * C::STAGE);
+        // Waves past the block's last output row multiply columns of the dy tile
+        // that are not stored: no branch around the MFMAs, whose accumulators would
+        // otherwise be copied between register files at the join.
 #pragma unroll
-            for (int ks = 0; ks < kWgTok / M::KS; ++ks) {
-                const typename M::Frag fa = frag_tr<T>(cur, SA, M::KS * ks, 32 * wave, lane);
+        for (int ks = 0; ks < C::TOK / M::KS; ++ks) {
+            const typename M::Frag fa = frag_tr<T>(cur, C::AP, M::KS * ks, 32 * wave, lane);
 #pragma unroll
-                for (int t = 0; t < IT; ++t)
-                    acc[t] = M::mfma(fa, frag_tr<T>(cur + kWgTok * SA, SB, M::KS * ks, 32 * t, lane), acc[t]);
-            }
-            if (more) stage(lds + (buf ^ 1) * STAGE);
-            __syncthreads();
-            buf ^= 1;
+            for (int t = 0; t < IT; ++t)
+                acc[t] = M::mfma(fa, frag_tr<T>(cur + C::TOK * C::AP * EP, C::XP, M::KS * ks, 32 * t, lane), acc[t]);
         }
+        buf = (buf + 1) % C::BUFS;
     }
     if (!active) return;
     // D row acc_row(r, g) is output row ob + 32 wave + that; column lane % 32 of tile t is input 32 t + lane % 32.
-    float* out = part + (int64_t)blockIdx.y * O * I_total + (int64_t)blockIdx.z * I;
+    float* out = part + (int64_t)split * O * I_total + (int64_t)cb * I;
 #pragma unroll
     for (int t = 0; t < IT; ++t)
 #pragma unroll
@@ -242,16 +269,17 @@ int launch_wgrad(const WgSrc<T>& dy, const void* x, int64_t ldx, void* dw, int d
                  int O, int I, int splits, hipStream_t s) {
     const int64_t per = cdiv(cdiv(rows, splits), kWgTokMax) * kWgTokMax;
     const int used = (int)cdiv(rows, per);
-    // Past 256 input columns the columns go to blocks of 256 (grid z), each
+    // Past 256 input columns the columns go to blocks of 256, each
     // with its own accumulators; dy is read once per block.
     const int cbs = I > kWgMaxCols ? I / kWgMaxCols : 1, Ib = I / cbs;
     const int nrb = (int)cdiv(O, kWgRows), rpb = 32 * (int)cdiv(cdiv(O, nrb), 32);
-    const dim3 grid((unsigned)nrb, (unsigned)used, (unsigned)cbs);
+    const WgGrid wg{nrb, cbs, used, nrb * cbs > 1 && used >= 8};
+    const unsigned grid = (unsigned)(nrb * cbs * (wg.by_xcd ? cdiv(used, 8) * 8 : used));
     switch (Ib / 32) {
 #define CASE(IT)                                                                                                  \
     case IT:                                                                                                      \
-        k_wgrad<T, IT><<<grid, 64 * kWgWaves, 2 * wgrad_stage_elems<T, IT>() * sizeof(T), s>>>(                   \
-            dy, (const T*)x, ldx, part, rows, O, rpb, per, I);                                                         \
+        k_wgrad<T, IT><<<grid, kWgThreads, WgCfg<T, IT>::BUFS * WgCfg<T, IT>::STAGE, s>>>(                       \
+            dy, (const T*)x, ldx, part, rows, O, rpb, per, I, wg);                                                       \
         break;
         CASE(1) CASE(2) CASE(3) CASE(4) CASE(5) CASE(6) CASE(7) CASE(8)
 #undef CASE

@@ -45,7 +45,10 @@ def splits_for(rows, out_features, in_features, dtype=torch.bfloat16):
     # 42, 105 -> 50 us; 968 x 192 on 236 instead of 132, 147 -> 91 us).
     if dtype == torch.float32:
         rows_per = 128
-    return max(1, min(max(1, WORKGROUPS // blocks), rows // rows_per))
+    splits = max(1, min(max(1, WORKGROUPS // blocks), rows // rows_per))
+    # Several tiles to a split go to one XCD (eight of them, in turn): whole
+    # rounds of eight splits load the XCDs alike.
+    return splits // 8 * 8 if blocks > 1 and splits >= 8 else splits
 
 
 def fp32_training(x, params):

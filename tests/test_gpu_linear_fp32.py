@@ -1,4 +1,4 @@
-"""fp32 training's linear maps: p3d_weight_grad / p3d_weight_grad3 on fp32
+"""Weight gradients stage by stage, and fp32 training's linear maps: p3d_weight_grad / p3d_weight_grad3 on fp32
 operands against the product in 64 bits, and InputProjections / OutputResidual
 in fp32 against torch's linear maps, through the layer and differentiated twice.
 
@@ -101,3 +101,23 @@ def test_fp32_maps_differentiated_twice(gpu):
     out2 = x.reshape(-1, 32) + F.linear(q2.reshape(-1, 32), wo)
     for a, b in zip(second((q, kv, gl, out)), second((q2, kv2, gl2, out2))):
         assert rel_l2(a, b) < 1e-5
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("rows,out_f,in_f,splits", [(1, 8, 32, 1), (31, 40, 128, 1), (32, 264, 160, 1), (33, 8, 256, 1),
+                                                    (95, 520, 96, 2), (96, 256, 512, 2), (97, 24, 192, 2),
+                                                    (641, 300 * 8, 64, 9), (1100, 520, 256, 17)])
+def test_weight_grad_stages(gpu, dtype, rows, out_f, in_f, splits):
+    """Ranges of less than a stage, of one, two and three, their partial last
+    stages beside rows of NaN, and several tiles to a range below, at and above
+    eight ranges.  16-bit products are exact in fp32."""
+    print(f"weight grad stages {rows}x{out_f}x{in_f} s{splits} {dtype}", flush=True)
+    gen = torch.Generator(device=gpu).manual_seed(rows + out_f)
+    dy, x = (torch.full((rows + 64, c), float("nan"), device=gpu, dtype=dtype) for c in (out_f, in_f))
+    dy[:rows] = torch.randn(rows, out_f, device=gpu, generator=gen).to(dtype)
+    x[:rows] = torch.randn(rows, in_f, device=gpu, generator=gen).to(dtype)
+    dw, work = torch.empty(out_f, in_f, device=gpu), torch.empty(splits, out_f, in_f, device=gpu)
+    _lib.call("p3d_weight_grad", dy.data_ptr(), out_f, x.data_ptr(), in_f, dw.data_ptr(), work.data_ptr(), rows, out_f,
+              in_f, splits, _lib.DTYPES[dtype], _lib.stream_of(gpu))
+    exp = torch.mm(dy[:rows].double().t(), x[:rows].double())
+    assert rel_l2(dw.double(), exp) <= _bound(rows)
