@@ -323,12 +323,21 @@ def backward(dy, q, kl, vl, kg, vg, weight, bias, gate, sl, sg, sk, svt, sk_norm
         return torch.empty(*shape, dtype=dtype, device=dev)
 
     f32 = torch.float32
-    bufs = dict(dol=empty(b, h, n, d), dog=empty(b, h, n, d), dl=empty(b, h, n, dtype=f32),
-                dg=empty(b, h, n, dtype=f32), dgate=empty(b, h, n, dtype=gate_k.dtype),
-                dslp=empty(parts, d, dtype=f32), dsgp=empty(parts, d, dtype=f32),
-                sv_rows=empty(b, g, mp, d), skt=empty(b, g, mp // 32, d, 32),
-                dql=empty(b, h, n, d),
-                dskp=empty(splits, b, g, mp, d, dtype=f32), dsvp=empty(splits, b, g, mp, d, dtype=f32))
+    rows, summary, esz = b * h * n, b * g * mp * d, q.element_size()
+    # Transposed copies of the rotated q and of dO_G: the summary dK/dV pass
+    # copies its transposed query stages from them by LDS DMA.
+    transposed = q.dtype != f32 and n >= 64 and n % 8 == 0
+    # One row of partials per pooling wave.
+    pool_parts = min(b * g * mp * geometry.pool_size, 2048)
+    work = _lib.Workspace()
+    for name, count, size in (("dol", rows * d, esz), ("dog", rows * d, esz), ("dl", rows, 4), ("dg", rows, 4),
+                              ("dslp", parts * d, 4), ("dsgp", parts * d, 4), ("sv_rows", summary, esz),
+                              ("skt", summary, esz), ("dql", rows * d, esz), ("dskp", splits * summary, 4),
+                              ("dsvp", splits * summary, 4), ("dwp", pool_parts * d, 4), ("dbp", pool_parts * slots, 4),
+                              ("q_t", transposed * rows * d, esz), ("dog_t", transposed * rows * d, esz)):
+        work.take(name, count, size)
+    bufs = work.allocate(dev)
+    dgate = empty(b, h, n, dtype=gate_k.dtype)
     a = _lib.BwdArgs()
     a.batch, a.heads, a.kv_heads, a.tokens, a.head_dim, a.dtype = b, h, g, n, d, dt
     a.summaries, a.gate_dtype, a.parts, a.splits = m, _lib.DTYPES[gate_k.dtype], parts, splits
@@ -338,15 +347,15 @@ def backward(dy, q, kl, vl, kg, vg, weight, bias, gate, sl, sg, sk, svt, sk_norm
     a.o_local, a.o_global = o_local.data_ptr(), o_global.data_ptr()
     a.lse_local, a.lse_global = lse_local.data_ptr(), lse_global.data_ptr()
     a.dy = _lib.view(dy)
-    a.dol, a.dog, a.delta_local, a.delta_global = (bufs[k].data_ptr() for k in ("dol", "dog", "dl", "dg"))
-    a.dgate, a.dsl_part, a.dsg_part = (bufs[k].data_ptr() for k in ("dgate", "dslp", "dsgp"))
-    a.sv_rows, a.skt = bufs["sv_rows"].data_ptr(), bufs["skt"].data_ptr()
-    a.dq_local, a.rope = bufs["dql"].data_ptr(), rope.struct()
+    a.dol, a.dog, a.delta_local, a.delta_global = (bufs[k] for k in ("dol", "dog", "dl", "dg"))
+    a.dgate, a.dsl_part, a.dsg_part = dgate.data_ptr(), bufs["dslp"], bufs["dsgp"]
+    a.sv_rows, a.skt = bufs["sv_rows"], bufs["skt"]
+    a.dq_local, a.rope = bufs["dql"], rope.struct()
     if out is None:
         out = tuple(empty(b, hh, n, d) for hh in (h, g, g, g, g))
     dq, dkl, dvl, dkg, dvg = out
     a.dq, a.dk_local, a.dv_local = _lib.view(dq), _lib.view(dkl), _lib.view(dvl)
-    a.dsk_part, a.dsv_part = bufs["dskp"].data_ptr(), bufs["dsvp"].data_ptr()
+    a.dsk_part, a.dsv_part = bufs["dskp"], bufs["dsvp"]
     keep += [qr, klr, gate_k, sl32, sg32, dy]
 
     _lib.call("p3d_mix_bwd", a, stream)
@@ -359,13 +368,11 @@ def backward(dy, q, kl, vl, kg, vg, weight, bias, gate, sl, sg, sk, svt, sk_norm
         nb, rev = geometry.neighbors, geometry.reverse_neighbors
         _lib.call("p3d_local_bwd_indexed", a, nb.data_ptr(), nb.shape[1], rev.data_ptr(), rev.shape[1], stream)
     _lib.call("p3d_global_bwd_dq", a, stream)
-    if q.dtype != torch.float32 and n >= 64 and n % 8 == 0:
-        # Transposed copies of the rotated q and of dO_G: the summary dK/dV
-        # pass copies its transposed query stages from them by LDS DMA.
-        bufs["q_t"], bufs["dog_t"] = empty(b * h * d * n), empty(b * h * d * n)
-        _lib.call("p3d_transpose_rows", _lib.view(qr), bufs["q_t"].data_ptr(), b, h, n, d, dt, stream)
-        _lib.call("p3d_transpose_rows", _lib.view(bufs["dog"]), bufs["dog_t"].data_ptr(), b, h, n, d, dt, stream)
-        a.q_t, a.dog_t = bufs["q_t"].data_ptr(), bufs["dog_t"].data_ptr()
+    if transposed:
+        _lib.call("p3d_transpose_rows", _lib.view(qr), bufs["q_t"], b, h, n, d, dt, stream)
+        _lib.call("p3d_transpose_rows", _lib.View(bufs["dog"], h * n * d, n * d, d), bufs["dog_t"], b, h, n, d, dt,
+                  stream)
+        a.q_t, a.dog_t = bufs["q_t"], bufs["dog_t"]
     _lib.call("p3d_global_bwd_dkv", a, stream)
 
     w32 = param_f32(weight)
@@ -374,17 +381,16 @@ def backward(dy, q, kl, vl, kg, vg, weight, bias, gate, sl, sg, sk, svt, sk_norm
                               _lib.view(kg), _lib.view(vg), geometry.blocks.data_ptr(), w32.data_ptr(),
                               b32.data_ptr(), pool_rope.struct(), sk.data_ptr(), svt.data_ptr(),
                               sk_norm_max.data_ptr())
-    # One row of partials per pooling wave; all four parameter sums in one launch.
-    pool_parts = min(b * g * mp * geometry.pool_size, 2048)
-    dwp, dbp = empty(pool_parts, d, dtype=f32), empty(pool_parts, slots, dtype=f32)
-    _lib.call("p3d_pool_bwd", pool_args, bufs["dskp"].data_ptr(), bufs["dsvp"].data_ptr(), splits,
-              _lib.view(dkg), _lib.view(dvg), dwp.data_ptr(), dbp.data_ptr(), pool_parts, stream)
+    # All four parameter sums in one launch.
+    _lib.call("p3d_pool_bwd", pool_args, bufs["dskp"], bufs["dsvp"], splits,
+              _lib.view(dkg), _lib.view(dvg), bufs["dwp"], bufs["dbp"], pool_parts, stream)
     keep += [w32, b32]
     sums = [(part, empty(*p.shape, dtype=p.dtype if p.dtype in _lib.DTYPES else f32))
-            for part, p in ((dwp, weight), (dbp, bias), (bufs["dslp"], sl), (bufs["dsgp"], sg))]
+            for part, p in (((bufs["dwp"], pool_parts, d), weight), ((bufs["dbp"], pool_parts, slots), bias),
+                            ((bufs["dslp"], parts, d), sl), ((bufs["dsgp"], parts, d), sg))]
     _lib.sum_rows(sums, dev)
     dweight, dbias, dsl, dsg = (out.to(p.dtype) for (_, out), p in zip(sums, (weight, bias, sl, sg)))
-    dgate = bufs["dgate"] if bufs["dgate"].dtype == gate.dtype else bufs["dgate"].to(gate.dtype)
+    dgate = dgate if dgate.dtype == gate.dtype else dgate.to(gate.dtype)
     return dq, dkl, dvl, dkg, dvg, dweight, dbias, dgate, dsl, dsg
 
 
@@ -436,8 +442,7 @@ def _projection_views(qp, kvp, heads, kv_heads):
     b, n = qp.shape[0], qp.shape[1]
     d = qp.shape[2] // heads
     q = qp.view(b, n, heads, d).transpose(1, 2)
-    kv = kvp.view(b, n, 4, kv_heads, d)
-    return (q, *(kv[:, :, i].transpose(1, 2) for i in range(4)))
+    return (q, *kvp.view(b, n, 4, kv_heads, d).permute(2, 0, 3, 1, 4).unbind(0))
 
 
 def pack3d_hip_projections(qp, kvp, heads, kv_heads, weight, bias, gate, sl, sg, geometry, rope: RopeSpec, *,
