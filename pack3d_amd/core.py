@@ -281,14 +281,15 @@ def _splits(n, m, bg, rep):
     several workgroups.  Few summaries or few tokens leave most CUs idle there
     (64 workgroups at 16,384 queries and 256 summaries of 2 kv heads, 8 at
     4,096 queries and 128 summaries): shorter splits, down to MIN_STAGES stages
-    a workgroup, up to one round of resident workgroups (two per CU).  dK/dV
+    a workgroup, up to one round of resident workgroups (two per CU, none with a
+    third: 21 splits of 24 blocks in fp32, 253 us, where 22 took 266).  dK/dV
     323 -> 117 us (head_dim 128, 256 summaries; 86 us since its stages leave
     room for a second workgroup), 88 -> 36 us (head_dim 64, 64 summaries), 37 ->
     11 us (4,096 queries, head_dim 16), with 3 to 8 us for the sum of the
     partials."""
     blocks = -(-m // 128) * bg
     splits = max(1, min(64, -(-2048 // blocks), -(-n // 1024)))
-    return max(splits, min(-(-512 // blocks), -(-n * rep // (64 * MIN_STAGES))))
+    return max(splits, min(512 // blocks, -(-n * rep // (64 * MIN_STAGES))))
 
 
 def backward(dy, q, kl, vl, kg, vg, weight, bias, gate, sl, sg, sk, svt, sk_norm_max, o_local, o_global,

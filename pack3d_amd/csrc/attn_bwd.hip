@@ -286,6 +286,9 @@ __device__ __forceinline__ void load_row_frags(const typename C::T_* row, bool v
     }
 }
 
+template <typename T>
+constexpr int dq_blocks = sizeof(T) == 4 ? 1 : 2;
+
 // Global dQ: per query, over all summaries, S = q . sk (log2 units), P =
 // 2^(S - lse_G log2 e), dP = dO_G . sv, dS = P (dP - Delta_G), dQ_G = ln 2 *
 // sum dS sk_stored (sk_stored = sk log2(e)/sqrt(d), so ln 2 * sk_stored =
@@ -295,9 +298,16 @@ __device__ __forceinline__ void load_row_frags(const typename C::T_* row, bool v
 // round(dQ_G)) (kernels.py:202-206 rounding): dQ_L comes from the local pass in
 // the storage type it is rounded to anyway, and dQ_G never reaches memory.  A
 // pass over fp32 copies of both took 181 us at 262,144 tokens (4 heads of 48).
+// A wave takes two column blocks of 32 queries, which share the LDS reads that
+// bound the 16-bit types, and one in fp32: bound by the matrix cores it gains from
+// the registers of the second (head_dim 48: 256 with 22 spilled and two waves a SIMD,
+// 133 and three) and from the finer grid (18,711 queries of 4 heads: 592 workgroups
+// for 296 on 256 compute units).  There 268 -> 190 us; 32,768 queries of 4 heads of
+// 128 and 256 summaries 629 -> 340 us.
 template <typename T, int D>
-__global__ __launch_bounds__(64 * kWaves, (D >= 128 || (sizeof(T) == 4 && D >= 64) ? 1 : 2)) void k_global_dq(BwdDev a) {
+__global__ __launch_bounds__(64 * kWaves, (D >= 128 ? 1 : 2)) void k_global_dq(BwdDev a) {
     typedef Cfg<T, D> C;
+    constexpr int NB = dq_blocks<T>;
     constexpr int SK = dq_rows<C>();
     typedef DqStage<C, SK> S;
     extern __shared__ __align__(16) unsigned char smem[];
@@ -308,13 +318,13 @@ __global__ __launch_bounds__(64 * kWaves, (D >= 128 || (sizeof(T) == 4 && D >= 6
     const int64_t bg = (int64_t)b * a.G + kvh;
     stage_pair_meta(a.rope, D, meta);
 
-    typename C::Frag qf[2][C::NT], df[2][C::NT];
-    int64_t qrow[2];
-    bool qok[2];
-    float lse2[2], delta[2];
+    typename C::Frag qf[NB][C::NT], df[NB][C::NT];
+    int64_t qrow[NB];
+    bool qok[NB];
+    float lse2[NB], delta[NB];
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) {
-        const int64_t row = (int64_t)blockIdx.x * 64 * kWaves + 64 * wave + 32 * nb + qi;
+    for (int nb = 0; nb < NB; ++nb) {
+        const int64_t row = (int64_t)blockIdx.x * 32 * NB * kWaves + 32 * NB * wave + 32 * nb + qi;
         qok[nb] = row < a.N;
         qrow[nb] = qok[nb] ? row : 0;
         load_row_frags<C>(tp<T>(a.q) + b * a.qsb + h * a.qsh + qrow[nb] * a.qsn, qok[nb], g, qf[nb]);
@@ -322,9 +332,9 @@ __global__ __launch_bounds__(64 * kWaves, (D >= 128 || (sizeof(T) == 4 && D >= 6
         lse2[nb] = qok[nb] ? a.lse_g[(int64_t)bh * a.N + qrow[nb]] * kLog2e : INFINITY;
         delta[nb] = qok[nb] ? a.dg[(int64_t)bh * a.N + qrow[nb]] : 0.f;
     }
-    f32x16 acc[2][C::MB];
+    f32x16 acc[NB][C::MB];
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb)
+    for (int nb = 0; nb < NB; ++nb)
 #pragma unroll
         for (int mb = 0; mb < C::MB; ++mb)
 #pragma unroll
@@ -346,21 +356,21 @@ __global__ __launch_bounds__(64 * kWaves, (D >= 128 || (sizeof(T) == 4 && D >= 6
     // Only 16-bit types up to head_dim 48 have the registers for both paths
     // (wider ones and fp32 keep the per-query path, which already fills them).
     constexpr bool kFast = sizeof(T) == 2 && D <= 48;
-    float mw = 0.f, cq[2] = {0.f, 0.f}, cd[2] = {0.f, 0.f};
+    float mw = 0.f, cq[NB] = {}, cd[NB] = {};
     bool fast = false;
     if constexpr (kFast) {
         mw = -INFINITY;
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb)
+        for (int nb = 0; nb < NB; ++nb)
             if (qok[nb]) mw = fmaxf(mw, lse2[nb]);
         mw = wave_max(mw);
         if (mw == -INFINITY) mw = 0.f;  // no live query in the wave
         bool spread = false;
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) spread |= qok[nb] && mw - lse2[nb] > 64.f;
+        for (int nb = 0; nb < NB; ++nb) spread |= qok[nb] && mw - lse2[nb] > 64.f;
         fast = __builtin_amdgcn_ballot_w64(spread) == 0;
 #pragma unroll
-        for (int nb = 0; nb < 2; ++nb) {
+        for (int nb = 0; nb < NB; ++nb) {
             cq[nb] = qok[nb] ? __builtin_amdgcn_exp2f(mw - lse2[nb]) : 0.f;
             cd[nb] = -cq[nb] * delta[nb];
         }
@@ -395,7 +405,7 @@ __global__ __launch_bounds__(64 * kWaves, (D >= 128 || (sizeof(T) == 4 && D >= 6
                 constexpr bool LATE = D >= 128 || sizeof(T) == 4;
                 if constexpr (!LATE) load_vfrags<C, true>(cur + 2 * SK * C::KSTR, S::TGS, 32 * tt, lane, tf);
 #pragma unroll
-                for (int nb = 0; nb < 2; ++nb) {
+                for (int nb = 0; nb < NB; ++nb) {
                     f32x16 s;
                     if constexpr (FAST)
                         s = score_tile<C>(kf, qf[nb], minit);
@@ -441,7 +451,7 @@ __global__ __launch_bounds__(64 * kWaves, (D >= 128 || (sizeof(T) == 4 && D >= 6
     // One summary: P = 1 and dS = 0 exactly (kernels.py:198-199), so dQ_G = 0.
     const float out_scale = a.M > 1 ? kLn2 : 0.f;
 #pragma unroll
-    for (int nb = 0; nb < 2; ++nb) {
+    for (int nb = 0; nb < NB; ++nb) {
         if (!qok[nb]) continue;
         const T* dql = tp<T>(a.dq_l) + ((int64_t)bh * a.N + qrow[nb]) * D;
         T* dq = reinterpret_cast<T*>(a.dq) + b * a.dqsb + h * a.dqsh + qrow[nb] * a.dqsn;
@@ -873,7 +883,8 @@ void launch_mix(const BwdDev& d, int dtype, hipStream_t s) {
 
 template <int D>
 void launch_dq(const BwdDev& d, int dtype, hipStream_t s) {
-    const dim3 grid((unsigned)cdiv(d.N, 64 * kWaves), (unsigned)(d.B * d.H));
+    const int nb = dtype == P3D_F32 ? dq_blocks<float> : dq_blocks<_Float16>;
+    const dim3 grid((unsigned)cdiv(d.N, 32 * nb * kWaves), (unsigned)(d.B * d.H));
     switch (dtype) {
         case P3D_F32: k_global_dq<float, D><<<grid, 64 * kWaves, lds_dq<Cfg<float, D>>(), s>>>(d); break;
         case P3D_F16: k_global_dq<_Float16, D><<<grid, 64 * kWaves, lds_dq<Cfg<_Float16, D>>(), s>>>(d); break;
