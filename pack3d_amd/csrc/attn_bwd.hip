@@ -649,8 +649,11 @@ struct NoTransDma {
 };
 
 // TDMA: the transposed regions come by LDS DMA from a.q_t / a.dog_t.
+// fp32 from head_dim 64 on leaves LDS for one workgroup, whose waves may then use
+// the registers of two (head_dim 128 spilled 216: 32,768 queries of 4 heads and 256
+// summaries 1,237 -> 407 us; head_dim 64, 10 spilled, 65,536 and 1,024: 1,295 -> 1,283).
 template <typename T, int D, bool TDMA>
-__global__ __launch_bounds__(64 * kWaves, 2) void k_global_dkv(BwdDev a) {
+__global__ __launch_bounds__(64 * kWaves, (sizeof(T) == 4 && D >= 64 ? 1 : 2)) void k_global_dkv(BwdDev a) {
     typedef Cfg<T, D> C;
     constexpr int SK = kv_rows<C>();
     typedef KvStage<C, SK, TDMA> S;
