@@ -15,8 +15,8 @@
 // token tile's channel blocks (CB = NB; WT = NB / CB waves per tile is 1 for
 // every width taken: split over two waves, each tile's dY rows were read twice
 // and the pass took 25% longer) for the whole contraction.  Widths past 256
-// (384, 512) go to two channel halves on grid y, each workgroup computing one
-// half (its W^T rows, its dx columns), so dY is read once per half; the
+// (384, 512) go to channel shares on grid y, each workgroup computing one
+// (its W^T rows, its dx columns), so dY is read once per share; the
 // registers of a whole 512-channel row would not fit.  The result goes
 // through the wave's LDS tile and leaves as 16-byte row pieces, rounded once
 // from the fp32 sum.
@@ -72,7 +72,7 @@ __global__ __launch_bounds__(64 * kIgWaves, 2) void k_input_grad(IgDev a) {
     const int64_t tok0 = ((int64_t)blockIdx.x * TILES + tile) * 32;
     const int64_t trow = min(tok0 + t, a.rows - 1);  // dead lanes read the last row, their outputs are dropped
     const int chunks = a.k_pad / kIgChunk;
-    // This workgroup's channel half (grid y): W^T rows and dx columns from DIM * blockIdx.y.
+    // This workgroup's channel share (grid y): W^T rows and dx columns from DIM * blockIdx.y.
     const T* wt = tp<T>(a.wt) + (int64_t)blockIdx.y * DIM * a.k_pad;
 
     // W^T chunk c: rows = channels, 64 features each.
@@ -174,24 +174,32 @@ __global__ __launch_bounds__(64 * kIgWaves, 2) void k_input_grad(IgDev a) {
     }
 }
 
-template <typename T, int NB, int CB>
-void launch_ig(const IgDev& d, int halves, hipStream_t s) {
-    constexpr int TILES = kIgWaves / (NB / CB);
-    const int64_t blocks = cdiv(d.rows, 32 * TILES);
-    k_input_grad<T, NB, CB><<<dim3((unsigned)blocks, (unsigned)halves), 64 * kIgWaves, 0, s>>>(d);
+template <typename T, int NB>
+void launch_ig(const IgDev& d, int64_t tiles, int shares, hipStream_t s) {
+    k_input_grad<T, NB, NB><<<dim3((unsigned)tiles, (unsigned)shares), 64 * kIgWaves, 0, s>>>(d);
 }
 
+// A workgroup takes 256 rows and up to 256 channels.  Where that leaves compute
+// units idle, the channels are halved (down to 64, or 96) while the workgroups
+// still fit one a unit: dy is read again for each share, from L2.  16,384 rows of
+// 1,544 features into 512 channels 55 us on 128 workgroups, 50 us on 256; 4,096 of
+// 520 into 256 channels 22 -> 17 us.
 template <typename T>
 int dispatch_ig(const IgDev& d, int dim, hipStream_t s) {
-    switch (dim) {
-        case 64: launch_ig<T, 2, 2>(d, 1, s); break;
-        case 96: launch_ig<T, 3, 3>(d, 1, s); break;
-        case 128: launch_ig<T, 4, 4>(d, 1, s); break;
-        case 192: launch_ig<T, 6, 6>(d, 1, s); break;
-        case 256: launch_ig<T, 8, 8>(d, 1, s); break;
-        case 384: launch_ig<T, 6, 6>(d, 2, s); break;
-        case 512: launch_ig<T, 8, 8>(d, 2, s); break;
-        default: return fail(P3D_EUNSUPPORTED, "p3d_input_grad: dim must be 64, 96, 128, 192, 256, 384 or 512");
+    if (dim != 64 && dim != 96 && dim != 128 && dim != 192 && dim != 256 && dim != 384 && dim != 512)
+        return fail(P3D_EUNSUPPORTED, "p3d_input_grad: dim must be 64, 96, 128, 192, 256, 384 or 512");
+    int dev = 0, cus = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    const int64_t tiles = cdiv(d.rows, 32 * kIgWaves);
+    int shares = dim > 256 ? 2 : 1, nb = dim / 32 / shares;  // channel blocks of 32 per workgroup
+    while (nb > 2 && nb % 2 == 0 && 2 * shares * tiles <= cus) nb /= 2, shares *= 2;
+    switch (nb) {
+        case 2: launch_ig<T, 2>(d, tiles, shares, s); break;
+        case 3: launch_ig<T, 3>(d, tiles, shares, s); break;
+        case 4: launch_ig<T, 4>(d, tiles, shares, s); break;
+        case 6: launch_ig<T, 6>(d, tiles, shares, s); break;
+        default: launch_ig<T, 8>(d, tiles, shares, s); break;
     }
     return P3D_OK;
 }

@@ -21,6 +21,7 @@
 // fragments of 32 different rows.  Outputs are rounded to the storage type,
 // as the linear maps' outputs are; the gate bias is added before that
 // rounding and the pair softmax runs in fp32 on the rounded logits.
+#include <algorithm>
 #include <type_traits>
 
 #include "rope.hpp"
@@ -41,6 +42,7 @@ struct ProjDev {
     int dim, q_out, kv_out, heads;
     int ln_dtype, gate_bias_dtype;
     float eps;
+    int blocks_per_wg;  // output blocks of 32 that a workgroup of k_project takes (blockIdx.y)
 };
 
 template <typename T>
@@ -155,7 +157,7 @@ __attribute__((amdgpu_waves_per_eu(KS <= 8 ? 4 : (KS <= 12 && !LIN ? 3 : 2)))) v
             lb[c] = load_any(a.ln_b, c, a.ln_dtype);
         }
     const int gbase = a.q_out + a.kv_out, nout = gbase + 2 * a.heads;
-    const int nblocks = (nout + 31) / 32;
+    const int ob0 = blockIdx.y * a.blocks_per_wg, obn = min((nout + 31) / 32, ob0 + a.blocks_per_wg);
     // Weight row o of the concatenation [Wq; Wkv; Wg].
     auto wrow = [&](int o) __attribute__((always_inline)) -> const T* {
         return o < a.q_out ? reinterpret_cast<const T*>(a.wq) + (int64_t)o * DIM
@@ -182,9 +184,9 @@ __attribute__((amdgpu_waves_per_eu(KS <= 8 ? 4 : (KS <= 12 && !LIN ? 3 : 2)))) v
             if (pc < PIECES) *reinterpret_cast<u32x4*>(&wbuf[buf][r * WS + c]) = wreg[i];
         }
     };
-    fetch(0);
-    stage(0);
-    fetch(min(1, nblocks - 1));
+    fetch(ob0);
+    stage(ob0 & 1);
+    fetch(min(ob0 + 1, obn - 1));
     __syncthreads();
 
     T* tile = otile[threadIdx.x >> 6];
@@ -274,13 +276,13 @@ __attribute__((amdgpu_waves_per_eu(KS <= 8 ? 4 : (KS <= 12 && !LIN ? 3 : 2)))) v
     // reads), so that every block issues the same loads.
     auto advance = [&](int ob) __attribute__((always_inline)) {
         stage((ob + 1) & 1);
-        fetch(min(ob + 2, nblocks - 1));
+        fetch(min(ob + 2, obn - 1));
         __syncthreads();
     };
     if constexpr (KS != 12 && KS != 16) {
         // One block at a time (the second accumulator set below would spill
         // at these widths).
-        for (int ob = 0; ob < nblocks; ++ob) {
+        for (int ob = ob0; ob < obn; ++ob) {
             epilogue(ob, gemm(ob));
             advance(ob);
         }
@@ -290,10 +292,10 @@ __attribute__((amdgpu_waves_per_eu(KS <= 8 ? 4 : (KS <= 12 && !LIN ? 3 : 2)))) v
     // block ob - 1's epilogue, which then runs under them.  The staged
     // weights of block ob + 1 go into the buffer block ob - 1 read, whose
     // readers all passed the barrier that ended the step before.
-    f32x16 d0 = gemm(0), d1;
-    advance(0);
-    int ob = 1;
-    for (; ob + 1 < nblocks; ob += 2) {
+    f32x16 d0 = gemm(ob0), d1;
+    advance(ob0);
+    int ob = ob0 + 1;
+    for (; ob + 1 < obn; ob += 2) {
         d1 = gemm(ob);
         epilogue(ob - 1, d0);
         advance(ob);
@@ -301,7 +303,7 @@ __attribute__((amdgpu_waves_per_eu(KS <= 8 ? 4 : (KS <= 12 && !LIN ? 3 : 2)))) v
         epilogue(ob, d1);
         advance(ob + 1);
     }
-    if (ob < nblocks) {
+    if (ob < obn) {
         d1 = gemm(ob);
         epilogue(ob - 1, d0);
         epilogue(ob, d1);
@@ -866,9 +868,19 @@ void k_out_residual(const T* __restrict__ y, const T* __restrict__ wo, const R* 
     }
 }
 
+// Where the row tiles leave compute units idle (256 rows a workgroup: 16,384 rows
+// are 64), the output blocks are shared by several workgroups, at least two blocks
+// each; each normalises its rows itself.  16,384 rows of 512 into 1,544 outputs
+// 94 -> 40 us, 32,768 into 1,040 69 -> 48 us, 9,000 of 192 into 968 32 -> 12 us.  Every output is formed alike.
 template <typename T, bool LIN>
-int launch_project(const ProjDev& d, hipStream_t s) {
-    const unsigned blocks = (unsigned)cdiv(cdiv(d.rows, 32), kProjWaves);
+int launch_project(ProjDev d, hipStream_t s) {
+    const int64_t tiles = cdiv(cdiv(d.rows, 32), kProjWaves), nblocks = cdiv(d.q_out + d.kv_out + 2 * d.heads, 32);
+    int dev = 0, cus = 0;
+    (void)hipGetDevice(&dev);
+    (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
+    const int64_t shares = std::max<int64_t>(1, std::min<int64_t>(cus / tiles, nblocks / 2));
+    d.blocks_per_wg = (int)cdiv(nblocks, shares);
+    const dim3 blocks((unsigned)tiles, (unsigned)cdiv(nblocks, d.blocks_per_wg));
     switch (d.dim) {
 #define CASE(DIM)                                                                     \
     case DIM:                                                                         \
