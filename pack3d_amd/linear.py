@@ -373,9 +373,10 @@ class InputProjections(torch.autograd.Function):
         wide = x_dt == torch.float32 and x16.dtype != x_dt
         dys = [None if dy is None else _rows(dy).to(x16.dtype) for dy in (dq, dkv, dgl)]
         # One kernel for the three products where it takes the shapes (16-bit x).
-        dx = None if wide else input_grad(dys, (wq, wkv, wg))
+        need = ctx.needs_input_grad[0]
+        dx = input_grad(dys, (wq, wkv, wg)) if need and not wide else None
         fused = dx is not None
-        if wide:
+        if need and wide:
             dx = torch.zeros(x16.shape, dtype=torch.float32, device=x16.device)
         # The three weight gradients from one pass over x16 where the kernel takes them.
         same = x16.dtype if wq_dt == wkv_dt == wg_dt == x16.dtype else torch.float32
@@ -386,7 +387,9 @@ class InputProjections(torch.autograd.Function):
             if dy is None:
                 grads.append(None)
                 continue
-            if wide:
+            if not need:
+                pass
+            elif wide:
                 dx.add_(torch.mm(dy, w))
             elif dx is None:
                 dx = torch.mm(dy, w)
@@ -397,10 +400,10 @@ class InputProjections(torch.autograd.Function):
                 grads.append(None)
                 continue
             grads.append((weight_grad(dy, x16) if dws is None else dws[i]).to(w_dt))
-        if dx is None:
+        if dx is None and need:
             dx = torch.zeros(x16.shape, dtype=x16.dtype, device=x16.device)
         dbg = column_sums(_rows(dgl), bg_dt) if dgl is not None and ctx.needs_input_grad[4] else None
-        return dx.view(shape).to(x_dt), grads[0], grads[1], grads[2], dbg, None
+        return dx.view(shape).to(x_dt) if need else None, grads[0], grads[1], grads[2], dbg, None
 
 
 def wide_residual_supported(x, k, dim, dt):
@@ -475,6 +478,6 @@ class OutputResidual(torch.autograd.Function):
         y16, wo16 = ctx.saved_tensors
         x_dt, y_dt, wo_dt = ctx.meta
         d16 = dout.to(y16.dtype)
-        dy = torch.mm(d16, wo16).to(y_dt)
+        dy = torch.mm(d16, wo16).to(y_dt) if ctx.needs_input_grad[1] else None
         dx = None if x_dt is None else dout.to(x_dt)
         return dx, dy, weight_grad(d16, y16).to(wo_dt) if ctx.needs_input_grad[2] else None, None, None

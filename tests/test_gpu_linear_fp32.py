@@ -121,3 +121,27 @@ def test_weight_grad_stages(gpu, dtype, rows, out_f, in_f, splits):
               in_f, splits, _lib.DTYPES[dtype], _lib.stream_of(gpu))
     exp = torch.mm(dy[:rows].double().t(), x[:rows].double())
     assert rel_l2(dw.double(), exp) <= _bound(rows)
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+def test_frozen_weights(gpu, dtype):
+    """Only what requires a gradient gets one, with the value it has when all do."""
+    gen = torch.Generator(device=gpu).manual_seed(2)
+
+    def normal(*shape):
+        return torch.randn(*shape, device=gpu, generator=gen).to(dtype)
+
+    args = [normal(100, 64), normal(64, 64), normal(128, 64), normal(8, 64), normal(8)]
+
+    def grads(mask):
+        leaves = [t.clone().requires_grad_(m) for t, m in zip(args, mask)]
+        q, kv, gl = linear.InputProjections.apply(*leaves, dtype)
+        (q.square().sum() + kv.square().sum() + gl.square().sum()).backward()
+        return [t.grad for t in leaves]
+
+    every = grads([True] * 5)
+    for mask in ([False, True, False, False, False], [True, False, True, False, True], [False, False, False, True, False]):
+        for got, exp, m in zip(grads(mask), every, mask):
+            assert (got is None) != m
+            # one rounding to the type: the sums may take another order
+            assert not m or rel_l2(got.float(), exp.float()) < (1e-5 if dtype == torch.float32 else 2.0 ** -7)
