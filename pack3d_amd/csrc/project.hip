@@ -757,7 +757,7 @@ __attribute__((amdgpu_waves_per_eu(2))) void k_project_pool(ProjDev a, PoolFuseD
 template <typename T, int KS, typename R>
 __global__ __launch_bounds__(64 * kProjWaves) __attribute__((amdgpu_waves_per_eu(KS <= 12 ? 4 : 2)))
 void k_out_residual(const T* __restrict__ y, const T* __restrict__ wo, const R* __restrict__ x, R* __restrict__ out,
-                    int64_t rows, int dim) {
+                    int64_t rows, int dim, int blocks_per_wg) {
     constexpr int RP = (int)sizeof(R) / 2;  // 16-byte pieces per 8 outputs
     typedef Mma<T> M;
     typedef typename M::Frag Frag;
@@ -768,7 +768,7 @@ void k_out_residual(const T* __restrict__ y, const T* __restrict__ wo, const R* 
     constexpr int OS = 32 + 4;                      // fp32 output tile row stride
     __shared__ __align__(16) T wbuf[2][32 * WS];
     __shared__ __align__(16) float otile[kProjWaves][32 * OS];
-    const int nblocks = dim / 32;
+    const int ob0 = blockIdx.y * blocks_per_wg, obn = min(dim / 32, ob0 + blocks_per_wg);
     const int lane = threadIdx.x & 63, g = lane >> 5, t = lane & 31;
     const int64_t tok0 = ((int64_t)blockIdx.x * kProjWaves + (threadIdx.x >> 6)) * 32, tok = tok0 + t;
     const bool live = tok < rows;
@@ -798,7 +798,7 @@ void k_out_residual(const T* __restrict__ y, const T* __restrict__ wo, const R* 
     // operations go: stores, next residual, next weights; each wait then
     // falls on loads issued a block earlier.
     u32x4 resv[2][RP];
-    load_res(0, resv);
+    load_res(ob0, resv);
     u32x4 wreg[PPT];
     auto fetch = [&](int ob) __attribute__((always_inline)) {
 #pragma unroll
@@ -815,13 +815,13 @@ void k_out_residual(const T* __restrict__ y, const T* __restrict__ wo, const R* 
             if (pc < PIECES) *reinterpret_cast<u32x4*>(&wbuf[buf][r * WS + c]) = wreg[i];
         }
     };
-    fetch(0);
-    stage(0);
-    fetch(min(1, nblocks - 1));
+    fetch(ob0);
+    stage(ob0 & 1);
+    fetch(min(ob0 + 1, obn - 1));
     __syncthreads();
     settle_loads(wreg, yf, resv);
 
-    for (int ob = 0; ob < nblocks; ++ob) {
+    for (int ob = ob0; ob < obn; ++ob) {
         const T* wb = &wbuf[ob & 1][t * WS + 8 * g];
         f32x16 d;
 #pragma unroll
@@ -858,12 +858,12 @@ void k_out_residual(const T* __restrict__ y, const T* __restrict__ wo, const R* 
                 buffer_store16(orsrc, obytes, (uint32_t)(tt * dim + o0 + h * (8 / RP)) * sizeof(R), tok0 + tt < rows,
                                o[h]);
         }
-        load_res(min(ob + 1, nblocks - 1), resv);
+        load_res(min(ob + 1, obn - 1), resv);
         wave_lds_sync();
         // Unconditional (a stage after the last block fills a buffer no
         // block reads), so that every block issues the same loads.
         stage((ob + 1) & 1);
-        fetch(min(ob + 2, nblocks - 1));
+        fetch(min(ob + 2, obn - 1));
         __syncthreads();
     }
 }
@@ -871,16 +871,22 @@ void k_out_residual(const T* __restrict__ y, const T* __restrict__ wo, const R* 
 // Where the row tiles leave compute units idle (256 rows a workgroup: 16,384 rows
 // are 64), the output blocks are shared by several workgroups, at least two blocks
 // each; each normalises its rows itself.  16,384 rows of 512 into 1,544 outputs
-// 94 -> 40 us, 32,768 into 1,040 69 -> 48 us, 9,000 of 192 into 968 32 -> 12 us.  Every output is formed alike.
-template <typename T, bool LIN>
-int launch_project(ProjDev d, hipStream_t s) {
-    const int64_t tiles = cdiv(cdiv(d.rows, 32), kProjWaves), nblocks = cdiv(d.q_out + d.kv_out + 2 * d.heads, 32);
+// 94 -> 40 us, 32,768 into 1,040 69 -> 48 us, 9,000 of 192 into 968 32 -> 12 us; the
+// output product of 16,384 rows of 512 into 512 37 -> 20 us.  Every output is formed
+// alike.
+dim3 share_blocks(int64_t rows, int64_t nblocks, int& blocks_per_wg) {
+    const int64_t tiles = cdiv(cdiv(rows, 32), kProjWaves);
     int dev = 0, cus = 0;
     (void)hipGetDevice(&dev);
     (void)hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev);
     const int64_t shares = std::max<int64_t>(1, std::min<int64_t>(cus / tiles, nblocks / 2));
-    d.blocks_per_wg = (int)cdiv(nblocks, shares);
-    const dim3 blocks((unsigned)tiles, (unsigned)cdiv(nblocks, d.blocks_per_wg));
+    blocks_per_wg = (int)cdiv(nblocks, shares);
+    return dim3((unsigned)tiles, (unsigned)cdiv(nblocks, blocks_per_wg));
+}
+
+template <typename T, bool LIN>
+int launch_project(ProjDev d, hipStream_t s) {
+    const dim3 blocks = share_blocks(d.rows, cdiv(d.q_out + d.kv_out + 2 * d.heads, 32), d.blocks_per_wg);
     switch (d.dim) {
 #define CASE(DIM)                                                                     \
     case DIM:                                                                         \
@@ -896,12 +902,13 @@ int launch_project(ProjDev d, hipStream_t s) {
 template <typename T, typename R>
 int launch_out_residual(const void* y, const void* wo, const void* x, void* out, int64_t rows, int k, int dim,
                         hipStream_t s) {
-    const unsigned blocks = (unsigned)cdiv(cdiv(rows, 32), kProjWaves);
+    int per = 0;
+    const dim3 blocks = share_blocks(rows, dim / 32, per);
     switch (k) {
 #define CASE(KK)                                                                                                  \
     case KK:                                                                                                      \
         k_out_residual<T, KK / 16, R><<<blocks, 64 * kProjWaves, 0, s>>>((const T*)y, (const T*)wo, (const R*)x, \
-                                                                         (R*)out, rows, dim);                     \
+                                                                         (R*)out, rows, dim, per);                \
         break;
         CASE(64) CASE(96) CASE(128) CASE(192) CASE(256) CASE(384) CASE(512)
 #undef CASE
