@@ -179,6 +179,11 @@ def fused_out_residual(layer, x, y):
     return out
 
 
+def _any_global_hook():
+    """Whether hooks are registered for every module (taken as so where torch does not say)."""
+    return getattr(nn.modules.module, "_has_any_global_hook", lambda: True)()
+
+
 class PACK3DAttention(nn.Module):
     """Local residual plus gated compressed attention and an outer residual (attention.py:10-21)."""
 
@@ -318,7 +323,7 @@ class PACK3DAttention(nn.Module):
             return False
         return (any(p.requires_grad for p in (x, *params)) and fp32_training(x, params)
                 and not any(m.bias is not None for m in (self.to_q, self.to_kv, self.to_out))
-                and not nn.modules.module._has_any_global_hook()
+                and not _any_global_hook()
                 and all(type(m) is nn.Linear and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
                                                       or m._backward_pre_hooks) for m in mods))
 

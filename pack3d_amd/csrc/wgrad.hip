@@ -20,10 +20,9 @@
 // shared x fragments: D = dy^T x, 32 rows by I columns per wave.
 //
 // In fp32 the operands (two tokens of one column per 64 lanes) are plain reads of
-// two tile rows.  It is bound by
-// the fp32 MFMA: 18,711 tokens of to_q, to_kv and the gate at width 192 take
-// 91 us and to_out 50 us, where the library's four products, on a few dozen
-// workgroups, took 403 us.
+// two tile rows, and the pass is bound by the MFMA: 18,711 tokens of to_q, to_kv
+// and the gate at width 192 take 89 us and to_out 51 us, where the library's four
+// products, on a few dozen workgroups, took 403 us.
 #include "attn_common.hpp"
 
 namespace p3d {
