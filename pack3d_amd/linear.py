@@ -79,6 +79,13 @@ def weight_grad_supported(out_features, in_features):
 INPUT_GRAD_DIMS = (64, 96, 128, 192, 256, 384, 512)
 
 
+def _rows_dense(t):
+    """Whether t [rows, cols] lies as the kernels read it: unit column stride,
+    16-byte aligned rows at a stride that covers them.  An expanded gradient
+    (of y.sum(1), say) has a row stride of 0, a single row any."""
+    return t.stride(1) == 1 and t.stride(0) >= t.shape[1] and t.stride(0) % 8 == 0 and t.data_ptr() % 16 == 0
+
+
 def input_grad(dys, ws):
     """dq Wq + dkv Wkv + dgl Wg for the three 16-bit gradients dys [rows, *]
     and the weights ws [*, dim] of the same type, as one contraction summed in
@@ -89,8 +96,7 @@ def input_grad(dys, ws):
     dt, rows, dim = ws[0].dtype, dys[0].shape[0], ws[0].shape[1]
     outs = [w.shape[0] for w in ws]
     if (dt not in (torch.float16, torch.bfloat16) or dim not in INPUT_GRAD_DIMS or any(o % 8 for o in outs)
-            or any(dy.dtype != dt or dy.shape != (rows, o) or dy.stride(1) != 1 or dy.stride(0) % 8
-                   or dy.data_ptr() % 16 for dy, o in zip(dys, outs))):
+            or any(dy.dtype != dt or dy.shape != (rows, o) or not _rows_dense(dy) for dy, o in zip(dys, outs))):
         return None
     k = sum(outs)
     k_pad = -(-k // 64) * 64
@@ -149,10 +155,8 @@ def weight_grad(dy, x):
     if (not weight_grad_supported(out_f, in_f) or dy.dtype != x.dtype or dy.dtype not in _lib.DTYPES
             or _differentiated(dy, x)):
         return torch.mm(dy.t().float(), x.float())
-    dy = dy if dy.stride(1) == 1 and dy.stride(0) % 8 == 0 else dy.contiguous()
-    x = x if x.stride(1) == 1 and x.stride(0) % 8 == 0 else x.contiguous()
-    if dy.data_ptr() % 16 or x.data_ptr() % 16:
-        dy, x = dy.clone(), x.clone()
+    # A copy, not .contiguous(), which returns a single row as it lies.
+    dy, x = (t if _rows_dense(t) else t.clone(memory_format=torch.contiguous_format) for t in (dy, x))
     splits = splits_for(rows, out_f, in_f, dy.dtype)
     dw = torch.empty(out_f, in_f, dtype=torch.float32, device=dy.device)
     work = torch.empty(splits, out_f, in_f, dtype=torch.float32, device=dy.device)
@@ -171,9 +175,7 @@ def weight_grads3(dys, x, out_dtype=torch.float32):
     outs = [dy.shape[1] for dy in dys]
     dt = x.dtype
     if (dt not in _lib.DTYPES or not all(weight_grad_supported(o, in_f) for o in outs) or _differentiated(x, *dys)
-            or x.stride(1) != 1 or x.stride(0) % 8 or x.data_ptr() % 16
-            or any(dy.dtype != dt or dy.shape[0] != rows or dy.stride(1) != 1 or dy.stride(0) % 8
-                   or dy.data_ptr() % 16 for dy in dys)):
+            or not _rows_dense(x) or any(dy.dtype != dt or dy.shape[0] != rows or not _rows_dense(dy) for dy in dys)):
         return None
     total = sum(outs)
     splits = splits_for(rows, total, in_f, dt)
