@@ -6,6 +6,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "index.hpp"
 
 namespace p3d {
 namespace {
@@ -72,7 +73,7 @@ struct LayoutDims {
 __global__ void k_layout_map(LayoutDims d, int64_t* order, int64_t* coords, int32_t* map) {
     int64_t t = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
     if (t >= d.n) return;
-    // N < 2^31: 32-bit arithmetic throughout.
+    // N < 2^31: 32-bit arithmetic for rows (not for entries of the coordinate table).
     const int32_t Y = (int32_t)d.g[1], X = (int32_t)d.g[2], t32 = (int32_t)t;
     const int32_t x = t32 % X, zy = t32 / X, y = zy % Y, z = zy / Y;
     int32_t packed = t32;
@@ -85,9 +86,10 @@ __global__ void k_layout_map(LayoutDims d, int64_t* order, int64_t* coords, int3
     }
     if (map) map[t] = packed;
     order[packed] = t;
-    coords[3 * packed + 0] = z;
-    coords[3 * packed + 1] = y;
-    coords[3 * packed + 2] = x;
+    const int64_t at = coord_start(packed);
+    coords[at + 0] = z;
+    coords[at + 1] = y;
+    coords[at + 2] = x;
 }
 
 // Lanes per row of the row-wise table kernels: two rows share a wave up to 32
