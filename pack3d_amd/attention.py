@@ -184,6 +184,14 @@ def _any_global_hook():
     return getattr(nn.modules.module, "_has_any_global_hook", lambda: True)()
 
 
+def _plain_linear(m):
+    """Whether a call of m is nn.Linear's product and nothing else: no subclass or
+    parametrisation, no hook, no forward replaced on the object (as offloading
+    and casting wrappers do)."""
+    return (type(m) is nn.Linear and "forward" not in vars(m)
+            and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks or m._backward_pre_hooks))
+
+
 class PACK3DAttention(nn.Module):
     """Local residual plus gated compressed attention and an outer residual (attention.py:10-21)."""
 
@@ -318,14 +326,11 @@ class PACK3DAttention(nn.Module):
         OutputResidual: plain fp32 modules on which nothing is registered that
         the functions would skip."""
         mods = (self.to_q, self.to_kv, self.gate, self.to_out)
-        params = [m.weight for m in mods] + [self.gate.bias]
-        if not torch.is_grad_enabled() or any(p is None for p in params):
+        if not torch.is_grad_enabled() or _any_global_hook() or not all(_plain_linear(m) for m in mods):
             return False
-        return (any(p.requires_grad for p in (x, *params)) and fp32_training(x, params)
-                and not any(m.bias is not None for m in (self.to_q, self.to_kv, self.to_out))
-                and not _any_global_hook()
-                and all(type(m) is nn.Linear and not (m._forward_hooks or m._forward_pre_hooks or m._backward_hooks
-                                                      or m._backward_pre_hooks) for m in mods))
+        params = [m.weight for m in mods] + [self.gate.bias]
+        return (self.gate.bias is not None and not any(m.bias is not None for m in (self.to_q, self.to_kv, self.to_out))
+                and any(p.requires_grad for p in (x, *params)) and fp32_training(x, params))
 
     def _hip_linear(self, x):
         """Whether the linear maps run as InputProjections / OutputResidual
