@@ -126,35 +126,39 @@ __global__ __launch_bounds__(256) void k_gate_fwd(const T* logits, void* gate, i
 // (any strides, tokens contiguous in use); a thread takes one token, so that
 // its reads run along the tokens and its writes are one row of logits.  Each
 // block also writes the column sums of its unrounded dlogits, the gradient of
-// the bias that the logits hold, to part[block][2 H].
+// the bias that the logits hold, to part[block][2 H].  Grid y takes kGateHeads
+// heads each, whose sums fit in LDS.
+constexpr int kGateHeads = 2048;
 template <typename T>
 __global__ __launch_bounds__(256) void k_gate_bwd(const T* logits, p3d_view dgate, int dgate_dtype, T* dlogits,
                                                   float* part, int H, int64_t N, int64_t tokens) {
-    extern __shared__ float red[];  // [4 waves][H]
+    extern __shared__ float red[];  // [4 waves][HB]
+    const int h0 = blockIdx.y * kGateHeads, HB = min(kGateHeads, H - h0);
     const int64_t t = (int64_t)blockIdx.x * 256 + threadIdx.x;
     const bool ok = t < tokens;
     const int64_t b = ok ? t / N : 0, n = ok ? t - b * N : 0;
     typedef __attribute__((ext_vector_type(2))) T T2;
-    const T2* l = reinterpret_cast<const T2*>(logits) + (ok ? t : 0) * H;
-    T2* d = reinterpret_cast<T2*>(dlogits) + (ok ? t : 0) * H;
-    for (int h = 0; h < H; ++h) {
+    const T2* l = reinterpret_cast<const T2*>(logits) + (ok ? t : 0) * H + h0;
+    T2* d = reinterpret_cast<T2*>(dlogits) + (ok ? t : 0) * H + h0;
+    for (int h = 0; h < HB; ++h) {
         const T2 x = l[h];
         float y0, y1;
         pair_softmax(to_f32(x[0]), to_f32(x[1]), y0, y1);
-        const float g = load_any(dgate.data, b * dgate.sb + h * dgate.sh + n * dgate.sn, dgate_dtype);
+        const float g = load_any(dgate.data, b * dgate.sb + (int64_t)(h0 + h) * dgate.sh + n * dgate.sn, dgate_dtype);
         const float v = ok ? y0 * y1 * g : 0.f;
         T2 o;
         o[0] = from_f32<T>(-v);
         o[1] = from_f32<T>(v);
         if (ok) d[h] = o;
         const float sum = wave_sum(v);
-        if ((threadIdx.x & 63) == 0) red[(threadIdx.x >> 6) * H + h] = sum;
+        if ((threadIdx.x & 63) == 0) red[(threadIdx.x >> 6) * HB + h] = sum;
     }
     __syncthreads();
-    for (int h = threadIdx.x; h < H; h += 256) {
-        const float s = (red[h] + red[H + h]) + (red[2 * H + h] + red[3 * H + h]);
-        part[(int64_t)blockIdx.x * 2 * H + 2 * h] = -s;
-        part[(int64_t)blockIdx.x * 2 * H + 2 * h + 1] = s;
+    float* mine = part + ((int64_t)blockIdx.x * H + h0) * 2;
+    for (int h = threadIdx.x; h < HB; h += 256) {
+        const float s = (red[h] + red[HB + h]) + (red[2 * HB + h] + red[3 * HB + h]);
+        mine[2 * h] = -s;
+        mine[2 * h + 1] = s;
     }
 }
 
@@ -275,14 +279,15 @@ extern "C" int p3d_gate_fwd(const void* logits, int32_t dtype, void* gate, int32
 
 extern "C" int p3d_gate_bwd(const void* logits, int32_t dtype, p3d_view dgate, int32_t dgate_dtype, void* dlogits,
                             float* part, int32_t batch, int32_t heads, int64_t tokens, void* stream) {
-    P3D_REQUIRE(logits && dgate.data && dlogits && part && heads <= 2048 && batch >= 1 && heads >= 1 && tokens >= 1 && known(dgate_dtype),
+    P3D_REQUIRE(logits && dgate.data && dlogits && part && batch >= 1 && heads >= 1 && heads <= (1 << 24) && tokens >= 1 &&
+                    known(dgate_dtype),
                 "bad gate arguments");
     P3D_REQUIRE(dtype == P3D_F16 || dtype == P3D_BF16, "dtype must be fp16 or bf16");
     const int64_t all = batch * tokens;
     P3D_REQUIRE(cdiv(all, 256) < (1LL << 31), "launch grid too large");
     hipStream_t s = as_stream(stream);
-    const unsigned blocks = (unsigned)cdiv(all, 256);
-    const size_t lds = (size_t)4 * heads * sizeof(float);
+    const dim3 blocks((unsigned)cdiv(all, 256), (unsigned)cdiv(heads, kGateHeads));
+    const size_t lds = (size_t)4 * std::min(heads, kGateHeads) * sizeof(float);
     if (dtype == P3D_F16)
         k_gate_bwd<_Float16><<<blocks, 256, lds, s>>>((const _Float16*)logits, dgate, dgate_dtype, (_Float16*)dlogits,
                                                       part, heads, tokens, all);
