@@ -442,8 +442,8 @@ class OutputResidualWide(torch.autograd.Function):
         y16, wo16 = ctx.saved_tensors
         y_dt, wo_dt = ctx.meta
         d16 = dout.to(y16.dtype)
-        dy = torch.mm(d16, wo16).to(y_dt)
-        return dout, dy, weight_grad(d16, y16).to(wo_dt), None
+        dy = torch.mm(d16, wo16).to(y_dt) if ctx.needs_input_grad[1] else None
+        return dout, dy, weight_grad(d16, y16).to(wo_dt) if ctx.needs_input_grad[2] else None, None
 
 
 class OutputResidual(torch.autograd.Function):
