@@ -273,23 +273,33 @@ def _mix_parts(rows):
 MIN_STAGES = 4
 
 
-def _splits(n, m, bg, rep):
+def _splits(n, m, bg, rep, resident=512):
     """Query splits of the summary dK/dV pass over n queries of rep heads per
-    kv head, m summaries and bg = batch * kv heads.
+    kv head, m summaries and bg = batch * kv heads; resident: workgroups that the
+    GPU runs at a time.
 
     Large problems take at least 1,024 queries a split, which gives every CU
     several workgroups.  Few summaries or few tokens leave most CUs idle there
     (64 workgroups at 16,384 queries and 256 summaries of 2 kv heads, 8 at
     4,096 queries and 128 summaries): shorter splits, down to MIN_STAGES stages
-    a workgroup, up to one round of resident workgroups (two per CU, none with a
-    third: 21 splits of 24 blocks in fp32, 253 us, where 22 took 266).  dK/dV
+    a workgroup, up to one round of resident workgroups (none with a second: 21
+    splits of 24 blocks in fp32, 253 us, where 22 took 266).  dK/dV
     323 -> 117 us (head_dim 128, 256 summaries; 86 us since its stages leave
     room for a second workgroup), 88 -> 36 us (head_dim 64, 64 summaries), 37 ->
     11 us (4,096 queries, head_dim 16), with 3 to 8 us for the sum of the
-    partials."""
+    partials.  Where the LDS holds one workgroup per CU (fp32 from head_dim 64 on)
+    a round is 256: 16,384 queries of 4 heads of 128, 227 us with 512 workgroups,
+    194 with 256 (head_dim 64 alike, 193 and 192, with half the partials).
+
+    A split is a whole number of stages of each head's n queries: counts that
+    leave the last ones without a query (more splits than stages from 5 heads per
+    kv head on, 170 splits of 256 stages of which 128 hold any) come down to the
+    ranges that hold one."""
     blocks = -(-m // 128) * bg
     splits = max(1, min(64, -(-2048 // blocks), -(-n // 1024)))
-    return max(splits, min(512 // blocks, -(-n * rep // (64 * MIN_STAGES))))
+    splits = max(splits, min(resident // blocks, -(-n * rep // (64 * MIN_STAGES))))
+    stages = -(-n // 64)
+    return -(-stages // -(-stages // splits))
 
 
 def backward(dy, q, kl, vl, kg, vg, weight, bias, gate, sl, sg, sk, svt, sk_norm_max, o_local, o_global,
@@ -318,7 +328,7 @@ def backward(dy, q, kl, vl, kg, vg, weight, bias, gate, sl, sg, sk, svt, sk_norm
     gate_k = gate if gate.dtype in _lib.DTYPES else gate.float()
     sl32, sg32 = param_f32(sl), param_f32(sg)
     parts = _mix_parts(b * h * n)
-    splits = _splits(n, m, b * g, h // g)
+    splits = _splits(n, m, b * g, h // g, 256 if q.dtype == torch.float32 and d >= 64 else 512)
 
     def empty(*shape, dtype=q.dtype):
         return torch.empty(*shape, dtype=dtype, device=dev)
