@@ -17,6 +17,7 @@
 // for 64 packed rows per wave, with the local branch read from y (written by
 // the indexed local kernel) or from an fp32 buffer.
 #include "attn_common.hpp"
+#include "strips.hpp"
 
 namespace p3d {
 namespace {
@@ -56,8 +57,10 @@ struct AttnDev {
 // kernel is rows 8 z .. 8 z + 7 of the grid (Z = ceil(Y / 8) strips, rz = 0, one
 // brick in y), each with its own halo plane, whose y halo reaches into the
 // neighbouring strips.  A brick then holds 256 queries instead of 64, so a
-// quarter of the workgroups do the summary sweep and the set-up: 128 x 128
-// slices with 8 heads of 64, 150 us with 4 x 8 x 8 bricks, 133 us in strips.
+// quarter of the workgroups do the summary sweep and the set-up (strips_forward
+// has the measurements).  The strip instances look up each query's rotation with
+// the query fragments live and spill where the bricks do not (30 registers at bf16
+// head_dim 48, 58 at 64, 141 at 128, 591 at fp32 128).
 // (STRIPS is a template argument: as a run-time flag it cost the bricks registers.)
 template <bool STRIPS>
 __device__ __forceinline__ int real_y(int gz, int gy) { return STRIPS ? 8 * gz + gy : gy; }
@@ -1204,11 +1207,10 @@ extern "C" int p3d_attn_fwd_grid(const p3d_attn_args* args, void* stream) {
     d.Z = args->grid[0], d.Y = args->grid[1], d.X = args->grid[2];
     d.rz = args->radius[0], d.ry = args->radius[1], d.rx = args->radius[2];
     d.bricks_y = (int)cdiv(d.Y, 8), d.bricks_x = (int)cdiv(d.X, 8);
-    // Strips once the bricks of a one-plane grid are more than the GPU holds at a
-    // time (two workgroups on each of 256 CUs); fewer run side by side, and
-    // four strips in turn would only make each of them longer.  Unrotated
-    // keys take the rotation window, which strips do not build.
-    const bool strips = d.Z == 1 && d.kl_rotated && (int64_t)d.bricks_y * d.bricks_x * d.B * d.H > 512;
+    // Unrotated keys take the rotation window, which strips do not build.
+    const bool strips = d.Z == 1 && d.kl_rotated &&
+                        strips_forward(args->head_dim, args->dtype == P3D_BF16, d.bricks_y, d.bricks_x,
+                                       (int64_t)d.B * d.H);
     if (strips) {
         d.Z = d.bricks_y, d.bricks_y = 1, d.rz = 0;
     }

@@ -18,6 +18,7 @@
 // same masks with the roles of queries and keys exchanged.  Inputs q and kl
 // are already rotated.
 #include "attn_common.hpp"
+#include "strips.hpp"
 
 namespace p3d {
 namespace {
@@ -43,8 +44,7 @@ struct LbDev {
 
 // A grid of one z plane in strips of 8 rows, as in the forward kernel: plane z
 // of a brick is rows 8 z .. 8 z + 7 of the grid with a halo plane of its own
-// (Z counts strips, rz = 0, one brick in y).  128 x 128 slices with 8 / 2 heads of
-// 64: dQ 102 -> 61 us, dK/dV 88 -> 69 us.
+// (Z counts strips, rz = 0, one brick in y); strips_backward has the measurements.
 template <bool STRIPS>
 __device__ __forceinline__ int real_y(int gz, int gy) { return STRIPS ? 8 * gz + gy : gy; }
 
@@ -896,8 +896,8 @@ extern "C" int p3d_local_bwd_grid(const p3d_bwd_args* args, const int32_t grid[3
     d.Z = grid[0], d.Y = grid[1], d.X = grid[2];
     d.rz = radius[0], d.ry = radius[1], d.rx = radius[2];
     d.bricks_y = (int)cdiv(d.Y, 8), d.bricks_x = (int)cdiv(d.X, 8);
-    // Strips on a one-plane grid with more bricks than CUs (one workgroup each).
-    const bool strips = d.Z == 1 && (int64_t)d.bricks_y * d.bricks_x * d.B * d.G > 256;
+    const bool strips = d.Z == 1 && strips_backward(x.head_dim, x.dtype == P3D_F32, d.bricks_y, d.bricks_x,
+                                                    (int64_t)d.B * d.G);
     if (strips) {
         d.Z = d.bricks_y, d.bricks_y = 1, d.rz = 0;
     }
