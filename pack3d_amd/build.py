@@ -21,15 +21,18 @@ PROBE_LIB = os.path.join(HERE, "libpack3d_probe.so")
 ARCH = "gfx950"
 
 # Packed fp32 VALU ops are disabled for device code: the compiler forms them
-# from ordinary float code, and this pool has seen wrong results from some
-# forms.  The kernels never produce or consume NaN (masked scores are -inf),
-# so fmax needs no NaN-quieting of its operands (-fno-honor-nans).  The
-# kernels keep the default IEEE mode: a kernel compiled with
+# from ordinary float code, and some forms have given wrong results on this
+# hardware.  The attention kernels make no NaN of finite inputs (masked scores
+# are -inf), so fmax needs no NaN-quieting of its operands (-fno-honor-nans);
+# the passes that stand in for torch's softmax and sums keep NaN (HONOR_NANS).
+# The kernels keep the default IEEE mode: a kernel compiled with
 # -mno-amdgpu-ieee cannot inline the device library (threadIdx, blockIdx and
 # __mul24 become out-of-line calls), which costs far more than it saves.
 FLAGS = ["-x", "hip", "-O3", "-std=c++17", "-fPIC", f"--offload-arch={ARCH}", "-Wall", "-Wno-unused-function",
          "-Xclang", "-target-feature", "-Xclang", "-packed-fp32-ops",
          "-fno-honor-nans", "-Wno-nan-infinity-disabled"]
+# Sources whose outputs a loss scaler looks at for what overflowed.
+HONOR_NANS = ("params.hip",)
 
 
 def _hipcc():
@@ -42,7 +45,8 @@ def _hipcc():
 
 def _compile(src, hipcc, verbose):
     obj = os.path.join(BUILD, os.path.basename(src) + ".o")
-    cmd = [hipcc, *FLAGS, "-c", src, "-o", obj]
+    nans = ["-fhonor-nans"] if os.path.basename(src) in HONOR_NANS else []
+    cmd = [hipcc, *FLAGS, *nans, "-c", src, "-o", obj]
     if verbose:
         print(" ".join(cmd), flush=True)
     proc = subprocess.run(cmd, capture_output=True, text=True)

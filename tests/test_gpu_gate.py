@@ -1,4 +1,7 @@
-"""The gate's backward past the heads of one launch row."""
+"""The gate's backward past the heads of one launch row, and both directions of
+the gate on infinite and NaN logits and gradients."""
+import math
+
 import pytest
 import torch
 
@@ -28,3 +31,29 @@ def test_gate_backward_many_heads(gpu, dtype, b, n, h):
     assert bool(((got.double() - exp).abs() <= (16 * EPS[torch.float32] + EPS[dtype]) * exp.abs() + tiny).all())
     bound = (b * n + 16) * EPS[torch.float32] * exp.abs().sum((0, 1))
     assert bool(((dbias.double() - exp.sum((0, 1))).abs() <= bound).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float16, torch.bfloat16])
+@pytest.mark.parametrize("upstream", [1.0, -2.0, 0.0, math.inf, -math.inf, math.nan])
+def test_gate_of_infinite_and_nan_logits(gpu, dtype, upstream):
+    """As an overflowed step leaves them: the gate is NaN where torch's softmax is,
+    a logit gradient is finite where torch's is, and the bias gradient of a head
+    shows what any of its tokens does not hold finite."""
+    print(f"gate specials {dtype} {upstream}", flush=True)
+    inf, nan = math.inf, math.nan
+    values = [nan, inf, -inf, 0.0, 3.0, -200.0, 200.0]
+    pairs = torch.tensor([[a, b] for a in values for b in values])
+    gl = pairs.view(1, 1, -1).to(gpu, dtype).requires_grad_()  # one token, one head per pair
+    heads = len(pairs)
+    bias = torch.zeros(2 * heads, device=gpu, requires_grad=True)
+    gate = linear.GateProbability.apply(gl, bias, heads, torch.float32)
+    dgate = torch.full_like(gate, upstream)
+    got, dbias = torch.autograd.grad(gate, (gl, bias), dgate)
+    ref = gl.detach().float().requires_grad_()
+    exact = ref.view(1, 1, heads, 2).softmax(-1)[..., 1].transpose(1, 2)
+    (exp,) = torch.autograd.grad(exact, ref, dgate)
+    assert torch.equal(gate.isnan(), exact.isnan())
+    assert torch.equal(gate.nan_to_num(), exact.nan_to_num()) or torch.allclose(gate.nan_to_num(), exact.nan_to_num(), rtol=1e-6, atol=0)
+    finite = exp.view(heads, 2).isfinite().all(-1)
+    assert torch.equal(got.view(heads, 2).isfinite().all(-1), finite)
+    assert torch.equal(dbias.view(heads, 2).isfinite().all(-1), finite)
