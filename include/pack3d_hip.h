@@ -26,7 +26,7 @@
 extern "C" {
 #endif
 
-#define P3D_ABI_VERSION 22
+#define P3D_ABI_VERSION 23
 
 enum p3d_status { P3D_OK = 0, P3D_EINVAL = 1, P3D_EHIP = 2, P3D_EUNSUPPORTED = 3 };
 enum p3d_dtype { P3D_F32 = 0, P3D_F16 = 1, P3D_BF16 = 2 };
@@ -525,12 +525,6 @@ typedef struct p3d_sum_job {
 
 /* Up to 8 sums of partial gradients in one launch.  jobs is a host array. */
 int p3d_sum_rows(const p3d_sum_job* jobs, int32_t count, void* stream);
-
-/* part[p][c] = sum of column c of x [rows, cols] (16-bit, row stride ldx a
- * multiple of 8, cols a multiple of 8 up to 256) over the p-th of `parts`
- * equal row ranges, in fp32: the gate bias gradient before p3d_sum_rows. */
-int p3d_column_sums(const void* x, int64_t ldx, int64_t rows, int32_t cols, int32_t dtype, float* part,
-                    int32_t parts, void* stream);
 
 /* Second entry of the softmax over each of `count` pairs of 16-bit logits
  * (attention.py:85), in fp32, written as gate_dtype. */

@@ -25,7 +25,7 @@ class View(ctypes.Structure):
     _fields_ = [("data", c_void_p), ("sb", c_int64), ("sh", c_int64), ("sn", c_int64)]
 
 
-ABI_VERSION = 22  # P3D_ABI_VERSION in include/pack3d_hip.h
+ABI_VERSION = 23  # P3D_ABI_VERSION in include/pack3d_hip.h
 
 
 class Rope(ctypes.Structure):
@@ -137,7 +137,6 @@ SIGNATURES = {
     "p3d_transpose_rows": ([View, _P, c_int32, c_int32, c_int32, c_int32, c_int32, _P], c_int32),
     "p3d_pool_bwd": ([ctypes.POINTER(PoolArgs), _P, _P, c_int32, View, View, _P, _P, c_int32, _P], c_int32),
     "p3d_sum_rows": ([ctypes.POINTER(SumJob), c_int32, _P], c_int32),
-    "p3d_column_sums": ([_P, c_int64, c_int64, c_int32, c_int32, _P, c_int32, _P], c_int32),
     "p3d_gate_fwd": ([_P, c_int32, _P, c_int32, c_int64, _P], c_int32),
     "p3d_gate_bwd": ([_P, c_int32, View, c_int32, _P, _P, c_int32, c_int32, c_int64, _P], c_int32),
     "p3d_cast": ([ctypes.POINTER(CastJob), c_int32, _P], c_int32),

@@ -826,13 +826,13 @@ __global__ __launch_bounds__(64 * kWaves) void k_local_dkv_grid_dma(LbDev a) {
 }
 
 template <typename T, int D>
-size_t lds_dq_grid() {
+constexpr size_t lds_dq_grid() {
     typedef Cfg<T, D> C;
     return ((size_t)2 * kPlaneKeys * C::KSTR + (size_t)32 * C::MB * (kPlaneKeys + Piece<T>::N)) * sizeof(T);
 }
 
 template <typename T, int D>
-size_t lds_dkv_grid() {
+constexpr size_t lds_dkv_grid() {
     typedef Cfg<T, D> C;
     return ((size_t)2 * kPlaneKeys * C::KSTR + (size_t)2 * 32 * C::MB * (kPlaneKeys + Piece<T>::N)) * sizeof(T) +
            (size_t)2 * kPlaneKeys * sizeof(float) + (size_t)(D / 2) * sizeof(int4);
@@ -849,9 +849,10 @@ int launch_t(const LbDev& d, hipStream_t s) {
         static_assert(l1 <= 160 * 1024 && l2 <= 160 * 1024, "plane buffers within LDS");
         k_local_dq_grid_dma<T, D, STRIPS><<<dim3(bricks, d.B * d.H), 64 * kWaves, l1, s>>>(d);
         k_local_dkv_grid_dma<T, D, STRIPS><<<dim3(bricks, d.B * d.G), 64 * kWaves, l2, s>>>(d);
+    } else if constexpr (lds_dq_grid<T, D>() > 160 * 1024 || lds_dkv_grid<T, D>() > 160 * 1024) {  // fp32 head_dim 128
+        return fail(P3D_EUNSUPPORTED, "p3d_local_bwd_grid: planes exceed LDS");
     } else {
-        const size_t l1 = lds_dq_grid<T, D>(), l2 = lds_dkv_grid<T, D>();
-        if (l1 > 160 * 1024 || l2 > 160 * 1024) return fail(P3D_EUNSUPPORTED, "p3d_local_bwd_grid: planes exceed LDS");
+        constexpr size_t l1 = lds_dq_grid<T, D>(), l2 = lds_dkv_grid<T, D>();
         k_local_dq_grid<T, D, STRIPS><<<dim3(bricks, d.B * d.H), 64 * kWaves, l1, s>>>(d);
         k_local_dkv_grid<T, D, STRIPS><<<dim3(bricks, d.B * d.G, kSplitDkv<C> ? 2 : 1), 64 * kWaves, l2, s>>>(d);
     }

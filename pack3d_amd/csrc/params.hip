@@ -1,13 +1,13 @@
 // Small passes around the 16-bit training step that carry little data each and
 // were one torch launch (or several) apiece: sums of partial parameter
-// gradients with their cast, column sums of the gate gradient, the gate's pair
-// softmax and its backward, weight casts, and the transposed concatenation of
-// the input projections' weights.  Each is bound by its launch and one or two
-// memory round trips, so what counts is how many there are and that every
-// load of a thread is in flight at once.  A 16-bit training step went from 52
-// launches to 34; in one of 32,768 tokens at dim 512 the parameter sums and
-// casts fell from 150 to 25 us, the gate's backward (a fill, a strided copy, a
-// product and a softmax backward) to 9 us, the gate and bias casts to 4.
+// gradients with their cast, the gate's pair softmax and its backward, weight
+// casts, and the transposed concatenation of the input projections' weights.
+// Each is bound by its launch and one or two memory round trips, so what counts
+// is how many there are and that every load of a thread is in flight at once.  A
+// 16-bit training step went from 52 launches to 32; in one of 32,768 tokens at
+// dim 512 the parameter sums and casts fell from 150 to 25 us, the gate's backward
+// (a fill, a strided copy, a product and a softmax backward) to 9 us, the gate and
+// bias casts to 4.
 #include <algorithm>
 
 #include "common.hpp"
@@ -66,39 +66,6 @@ __global__ __launch_bounds__(kSumThreads) void k_sum_rows(SumJobs a) {
         __syncthreads();
     }
     if (grp == 0 && c < job.cols) store_any(job.dst, c, job.dtype, part[lc]);
-}
-
-// ---------------------------------------------------------- column sums
-// part[b][c] = sum of column c of x over block b's rows (16-bit x, cols a
-// multiple of 8 up to 256): 16-byte pieces, consecutive threads on consecutive
-// pieces of a row.
-template <typename T>
-__global__ __launch_bounds__(256) void k_column_sums(const T* x, int64_t ldx, int64_t rows, int cols, int64_t per,
-                                                     float* part) {
-    __shared__ float red[256][9];  // one more than the piece: no two rows of threads share a bank
-    const int pieces = cols / 8, lanes = 256 / pieces;
-    const int p = threadIdx.x % pieces, g = threadIdx.x / pieces;
-    const int64_t first = (int64_t)blockIdx.x * per, last = min(rows, first + per);
-    float sum[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-    if (g < lanes)
-        for (int64_t r = first + g; r < last; r += 4 * lanes) {
-            float v[4][8];
-#pragma unroll
-            for (int i = 0; i < 4; ++i) load_piece<T>(x + min(r + (int64_t)i * lanes, last - 1) * ldx + 8 * p, v[i]);
-#pragma unroll
-            for (int i = 0; i < 4; ++i)
-                if (r + (int64_t)i * lanes < last)
-#pragma unroll
-                    for (int e = 0; e < 8; ++e) sum[e] += v[i][e];
-        }
-#pragma unroll
-    for (int e = 0; e < 8; ++e) red[threadIdx.x][e] = sum[e];
-    __syncthreads();
-    for (int c = threadIdx.x; c < cols; c += 256) {
-        float t = 0.f;
-        for (int k = 0; k < lanes; ++k) t += red[k * pieces + c / 8][c % 8];
-        part[(int64_t)blockIdx.x * cols + c] = t;
-    }
 }
 
 // ----------------------------------------------------------------- gate
@@ -246,21 +213,6 @@ extern "C" int p3d_sum_rows(const p3d_sum_job* jobs, int32_t count, void* stream
     a.first_block[count] = (int)blocks;
     k_sum_rows<<<(unsigned)blocks, kSumThreads, 0, as_stream(stream)>>>(a);
     return check_launch("p3d_sum_rows");
-}
-
-extern "C" int p3d_column_sums(const void* x, int64_t ldx, int64_t rows, int32_t cols, int32_t dtype, float* part,
-                               int32_t parts, void* stream) {
-    P3D_REQUIRE(x && part && rows >= 1 && parts >= 1 && parts < 65536, "bad column sum");
-    P3D_REQUIRE(dtype == P3D_F16 || dtype == P3D_BF16, "dtype must be fp16 or bf16");
-    P3D_REQUIRE(cols >= 8 && cols % 8 == 0 && cols <= 256, "cols must be a multiple of 8 up to 256");
-    P3D_REQUIRE(ldx >= cols && ldx % 8 == 0 && aligned16(x), "rows must be 16-byte aligned");
-    const int64_t per = cdiv(rows, parts);
-    hipStream_t s = as_stream(stream);
-    if (dtype == P3D_F16)
-        k_column_sums<_Float16><<<parts, 256, 0, s>>>((const _Float16*)x, ldx, rows, cols, per, part);
-    else
-        k_column_sums<__bf16><<<parts, 256, 0, s>>>((const __bf16*)x, ldx, rows, cols, per, part);
-    return check_launch("p3d_column_sums");
 }
 
 extern "C" int p3d_gate_fwd(const void* logits, int32_t dtype, void* gate, int32_t gate_dtype, int64_t count,

@@ -188,20 +188,8 @@ def weight_grads3(dys, x, out_dtype=torch.float32):
 
 
 def column_sums(x, dtype):
-    """Sum over the rows of a 16-bit x [rows, cols] in fp32, rounded to dtype
-    (``p3d_column_sums`` and one ``p3d_sum_rows``; torch where they do not
-    take the shape)."""
-    rows, cols = x.shape
-    if (x.dtype not in (torch.float16, torch.bfloat16) or dtype not in _lib.DTYPES or not 8 <= cols <= 256 or cols % 8
-            or x.stride(1) != 1 or x.stride(0) % 8 or x.stride(0) < cols or x.data_ptr() % 16):
-        return x.float().sum(0).to(dtype)
-    parts = max(1, min(512, rows // 128))
-    part = torch.empty(parts, cols, dtype=torch.float32, device=x.device)
-    out = torch.empty(cols, dtype=dtype, device=x.device)
-    _lib.call("p3d_column_sums", x.data_ptr(), x.stride(0), rows, cols, _lib.DTYPES[x.dtype], part.data_ptr(), parts,
-              _lib.stream_of(x.device))
-    _lib.sum_rows([(part, out)], x.device)
-    return out
+    """Sum over the rows of x [rows, cols] in fp32, rounded to dtype."""
+    return x.float().sum(0).to(dtype)
 
 
 def cast_all(tensors, dt):
@@ -230,8 +218,8 @@ class GateProbability(torch.autograd.Function):
     view), in out_dtype.  Computed in fp32 from the logits in both directions,
     one kernel each (``p3d_gate_fwd`` / ``p3d_gate_bwd``).  bias: the bias that
     gl already holds, whose gradient is summed from the unrounded logit
-    gradients in the same pass (the product that made gl then takes the bias
-    detached); None where the product's own backward gives it."""
+    gradients in the same pass (the product that made gl takes the bias
+    detached)."""
 
     @staticmethod
     def forward(ctx, gl, bias, heads, out_dtype):
@@ -241,7 +229,7 @@ class GateProbability(torch.autograd.Function):
         _lib.call("p3d_gate_fwd", gl.data_ptr(), _lib.DTYPES[gl.dtype], gate.data_ptr(), _lib.DTYPES[out_dtype],
                   gate.numel(), _lib.stream_of(gl.device))
         ctx.save_for_backward(gl)
-        ctx.meta = (heads, None if bias is None else bias.dtype)
+        ctx.meta = (heads, bias.dtype)
         return gate.transpose(1, 2)
 
     @staticmethod
@@ -255,7 +243,7 @@ class GateProbability(torch.autograd.Function):
         _lib.call("p3d_gate_bwd", gl.data_ptr(), _lib.DTYPES[gl.dtype], _lib.view3(dgate), _lib.DTYPES[dgate.dtype],
                   dgl.data_ptr(), part.data_ptr(), b, heads, n, _lib.stream_of(gl.device))
         dbias = None
-        if bias_dtype is not None and ctx.needs_input_grad[1]:
+        if ctx.needs_input_grad[1]:
             dbias = torch.empty(2 * heads, dtype=bias_dtype if bias_dtype in _lib.DTYPES else torch.float32,
                                 device=gl.device)
             _lib.sum_rows([(part, dbias)], gl.device)
