@@ -401,7 +401,7 @@ __global__ __launch_bounds__(64 * kWaves, (D >= 128 ? 1 : 2)) void k_global_dq(B
                 // Wide types load sk^T once the scores are done (a scheduling
                 // barrier keeps the loads there): all three sets together spill.
                 // 16-bit head_dim 128, 16,384 queries of 4 heads: 124 us with
-                // 284 registers spilled, 37 us.
+                // 284 registers spilled, 47 us with 21.
                 constexpr bool LATE = D >= 128 || sizeof(T) == 4;
                 if constexpr (!LATE) load_vfrags<C, true>(cur + 2 * SK * C::KSTR, S::TGS, 32 * tt, lane, tf);
 #pragma unroll

@@ -869,8 +869,9 @@ constexpr size_t grid_lds_bytes() {
 
 // Workgroups per CU that the register budget is for (one wave per SIMD each).
 // Where the LDS holds only one workgroup (head_dim 128, and fp32 from head_dim
-// 64) a cap for two bought nothing and spilled 88 to 5,764 registers: head_dim
-// 128 in bf16, 16,384 tokens of 4 heads, 181 us with 350 spilled, 115 us with 14.
+// 64) a cap for two bought nothing and spilled 87 (fp32 64) to 686 registers (fp32
+// 128, which spills 215 without it): head_dim 128 in bf16, 16,384 tokens of 4
+// heads, 181 us with 350 spilled, 115 us with 14.
 // fp32 head_dim 48 keeps two (one spilled register): 297 us against 368 with one
 // workgroup of unspilled waves (18,711 tokens of 4 heads).
 template <typename C, int PW>

@@ -234,8 +234,9 @@ __device__ __forceinline__ void dq_chunk(const typename C::Frag* kf, const typen
 // Which of dK and dV a workgroup of the dK/dV kernel computes.  At 16-bit
 // head_dim 128 the two accumulators (128 registers) beside the key and value
 // fragments (64) spill, so there each goes to workgroups of its own: the scores
-// are computed twice (20 against 16 MFMA groups per chunk), nothing spills, and
-// twice as many workgroups run.  16,384 tokens of 2 kv heads: 353 -> 115 us.
+// are computed twice (20 against 16 MFMA groups per chunk), 15 to 29 registers
+// spill instead of 220, and twice as many workgroups run.  16,384 tokens of 2 kv
+// heads: 353 -> 115 us.
 constexpr int kDK = 1, kDV = 2;
 
 // Types whose resident key fragments and accumulators leave no room for a

@@ -928,7 +928,7 @@ __global__ __launch_bounds__(256) void k_pool_bwd(PoolDev a, PoolBwdDev bd) {
 // takes 16 float4 columns of one tensor and 16 groups of splits, so that
 // every load of a thread is in flight at once, and adds the groups in order.
 // The pooling backward walks few items with few waves, and summed there the
-// splits of the small-grid launches (up to 256) cost one memory round trip per 8;
+// splits of the small-grid launches (up to 512) cost one memory round trip per 8;
 // here 6.5 us for 128 splits of 2 x 16,384 floats (17 MB).
 constexpr int kSumCols = 16, kSumGroups = 16;
 __global__ __launch_bounds__(kSumCols * kSumGroups) void k_sum_splits(float* dsk, float* dsv, int splits,

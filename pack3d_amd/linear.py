@@ -10,8 +10,10 @@ input gradient as one contraction (``p3d_input_grad``); the output
 projection's products stay torch GEMMs.  These functions replace the to_q, to_kv,
 gate (attention.py:64-67,85 of amilworks/Pack3D) and to_out + residual
 (attention.py:89) steps of ``PACK3DAttention.forward`` when it runs in a
-16-bit compute type with autograd active; weight gradients are accumulated
-in fp32 (torch's autocast path rounds them to the compute type first).
+16-bit compute type with autograd active, and those of an fp32 model in
+training (``fp32_training``; its products stay torch's, its LayerNorm and
+gate torch modules); weight gradients are accumulated in fp32 (torch's
+autocast path rounds them to the compute type first).
 """
 from __future__ import annotations
 
