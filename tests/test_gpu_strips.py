@@ -1,7 +1,8 @@
-"""One-plane grids with more bricks than the GPU holds at a time: the brick
-kernels take them in strips of 8 rows.  Forward and every gradient against the
-oracle, with the rotation fused (axial and by packed row), on ragged rows and
-columns, every head_dim and type, and both plane widths of head_dim 64."""
+"""One-plane grids of 670 to 1,200 bricks, on either side of the line where the
+brick kernels take them in strips of 8 rows (test_gpu_strips_large.py is well past
+it).  Forward and every gradient against the oracle, with the rotation fused
+(axial and by packed row), on ragged rows and columns, every head_dim and type,
+and both plane widths of head_dim 64."""
 import math
 
 import pytest

@@ -43,6 +43,7 @@ def test_rule(tmp_path):
         (False, False, 64, "bf16", 1, 4, 1, 1),
     ]
     kinds = {torch.float32: "fp32", torch.float16: "fp16", torch.bfloat16: "bf16"}
+    points += [(True, True, 16, "fp32", 15, 8, 16, 8)]  # the packed rotation's layer
     points += [(True, True, d, kinds[t], *_bricks(shape), b * h, b * g) for shape, _, _, _, b, h, g, d, t in CASES]
     body = "".join(
         f'printf("%d %d\\n", p3d::strips_forward({d}, {int(kind == "bf16")}, {by}, {bx}, {h}), '
@@ -72,3 +73,25 @@ def test_strips_match_oracle(gpu, shape, block, radius, kind, b, heads, kv_heads
         err = rel_l2(a.float(), x.float())
         print(f"  {name}: rel_l2={err:.3g}", flush=True)
         assert torch.isfinite(a).all() and err < TOL[dtype], (name, err)
+
+
+@pytest.mark.gpu
+def test_strips_packed_rotation_layer(gpu):
+    """The rotation by packed row (the layer's "packed" positions) in strips, with
+    every gradient of the layer."""
+    print("strips packed rotation layer", flush=True)
+    torch.manual_seed(0)
+    shape, b = (1, 120, 64), 2
+    kw = dict(heads=8, kv_heads=4, head_dim=16, block_volume=64, position_encoding="packed")
+    oracle, layer = ref.PACK3DAttention(64, **kw), p3d.PACK3DAttention(64, **kw)
+    layer.load_state_dict(oracle.state_dict())
+    layer = layer.to(gpu)
+    kw = dict(radius=(0, 1, 1), pool_size=4, layout="native_block_morton")
+    x, dy = torch.randn(2, b, math.prod(shape), 64)
+    out = []
+    for m, lay, dev in ((layer, p3d.build_layout(shape, (1, 8, 8), **kw), gpu), (oracle, ref.build_layout(shape, (1, 8, 8), **kw), "cpu")):
+        xs = x.to(dev).requires_grad_()
+        y = m(xs, lay)
+        out.append([y, *torch.autograd.grad(y, [xs, *m.parameters()], dy.to(dev))])
+    for a, e in zip(*out):
+        assert rel_l2(a, e) < TOL[torch.float32]
